@@ -20,6 +20,7 @@
 #include "pp_batch_core.h"
 #include "pp_launch.h"
 #include "pp_line_bs.h"
+#include "pp_line_mm.h"
 #include "pp_resx.h"
 
 #define PPB_CHECK(x)                                  \
@@ -57,18 +58,19 @@ int put(T *dst, const std::vector<T> &v, hipStream_t s)
 TableCache::~TableCache()
 {
     for (auto &kv : t_)
-        for (double *p : {kv.second.tw, kv.second.A, kv.second.B, kv.second.C, kv.second.D})
+        for (double *p : {kv.second.tw, kv.second.A, kv.second.B, kv.second.C, kv.second.D, kv.second.mm})
             if (p) (void)hipFree(p);
 }
 
-int TableCache::get(int N, AxisDev &out)
+int TableCache::get(int N, int kind, int axis, AxisDev &out)
 {
-    auto it = t_.find(N);
+    const bool dense = kind >= 0 && mm_serves(N, kind, axis);
+    const std::pair<int, int> key = {N, dense ? mm_family(kind) : -1};
+    auto it = t_.find(key);
     if (it != t_.end()) {
         out = it->second;
         return PP_SUCCESS;
     }
-    const AxisTables &t = axis_tables_cached(N);
     AxisDev d;
     auto up = [](double **dst, const std::vector<double> &v) -> int {
         if (hipMalloc((void **)dst, v.size() * sizeof(double)) != hipSuccess) return PP_ALLOCATION_FAIL;
@@ -77,10 +79,27 @@ int TableCache::get(int N, AxisDev &out)
         return PP_SUCCESS;
     };
     int rc;
+    if (dense) {
+        std::vector<double> oct(mm_octant_size(N));
+        fill_mm_octant(N, oct.data());
+        if ((rc = up(&d.A, oct))) return rc;
+        if (hipMalloc((void **)&d.mm, mm_tables_size(N, kind) * sizeof(double)) != hipSuccess) {
+            (void)hipFree(d.A);
+            return PP_ALLOCATION_FAIL;
+        }
+        d.mmi = d.mm + mm_inverse_offset(N, kind);
+        t_[key] = d;
+        // finished before the first batch that reads them, on whichever stream that runs
+        PPB_CHECK(launch_mm_tables(d.mm, d.A, N, kind, nullptr));
+        PPB_CHECK(hipStreamSynchronize(nullptr));
+        out = d;
+        return PP_SUCCESS;
+    }
+    const AxisTables &t = axis_tables_cached(N);
     if ((rc = up(&d.tw, t.tw)) || (rc = up(&d.A, t.A)) || (rc = up(&d.B, t.B)) || (rc = up(&d.C, t.C)) ||
         (rc = up(&d.D, t.D)))
         return rc;
-    t_[N] = d;
+    t_[key] = d;
     out = d;
     return PP_SUCCESS;
 }
@@ -105,12 +124,12 @@ int BatchCore::add(int nx, int ny, int nz, const char *bc, const double *X, int 
     if (16.0 * nx * ny * sizeof(double) >= 4294967296.0) return PP_UNSUPPORTED_SIZE;
     // FP64 members hand the z solve 16-column tiles, which y blocks of 16 columns fill alone
     // and narrower y blocks (a divisor of 16) fill together; periodic z stays in place
-    if (precision == 0 && !zper) {
-        const int ly = line_lines_any<double>(ny, 1);
-        if (ly <= 0 || zsolve_cpb<double>() % ly != 0) return PP_UNSUPPORTED_SIZE;
-    }
     const int rc = setup_boundary(m.g, bc);
     if (rc) return rc;
+    if (precision == 0 && !zper) {
+        const int ly = line_lines_any<double>(ny, m.g.kind[1], 1);
+        if (ly <= 0 || zsolve_cpb<double>() % ly != 0) return PP_UNSUPPORTED_SIZE;
+    }
     for (int i = 0; i < 6; i++) m.g.X[i] = X[i];
     setup_coords(m.g);
     *id = (int)mem.size();
@@ -130,10 +149,22 @@ template <typename R>
 int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
 {
     std::map<std::pair<int, int>, std::vector<LineItem>> cls;
+    // dense-product classes: launch shape from the class's units of 16 lines / columns
+    std::map<std::pair<int, int>, long> units;
+    for (const BatchMember &m : mem) {
+        const int N = axis == 0 ? m.g.nx : m.g.ny;
+        if (mm_serves(N, m.g.kind[axis], axis))
+            units[{N, m.g.kind[axis]}] += axis == 0 ? ((long)m.g.ny * m.g.nz + 15) / 16 : (long)((m.g.nx + 15) / 16) * m.g.nz;
+    }
+    std::map<std::pair<int, int>, MmPlan> plans;
+    for (const auto &kv : units) plans[kv.first] = mm_plan(kv.first.first, kv.first.second, axis, kv.second);
     for (int m = 0; m < (int)mem.size(); m++) {
         const SolveSetup &g = mem[m].g;
         const int N = axis == 0 ? g.nx : g.ny;
-        const int lines = line_lines_any<R>(N, axis);
+        const auto pl = plans.find({N, g.kind[axis]});
+        const int group = pl == plans.end() ? 1 : pl->second.units;
+        const int lines = line_lines_any<R>(N, g.kind[axis], axis) * (axis == 0 ? group : 1);
+        const int planes = axis == 1 ? group : 1;  // y: consecutive planes per block
         if (lines <= 0) return PP_UNSUPPORTED_SIZE;
         auto &items = cls[{N, g.kind[axis]}];
         if (axis == 0) {
@@ -141,7 +172,7 @@ int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
             for (long bx = 0; bx < (nl + lines - 1) / lines; bx++) items.push_back({m, (int)bx, 0});
         } else {
             const int nbx = (g.nx + lines - 1) / lines;
-            for (int z = 0; z < g.nz; z++)
+            for (int z = 0; z < (g.nz + planes - 1) / planes; z++)
                 for (int bx = 0; bx < nbx; bx++) items.push_back({m, bx, z});
         }
     }
@@ -150,8 +181,11 @@ int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
         HostClass c;
         c.key = kv.first.first;
         c.kind = kv.first.second;
+        c.axis = axis;
         c.nitems = (int)kv.second.size();
         c.li = std::move(kv.second);
+        const auto pl = plans.find(kv.first);
+        if (pl != plans.end()) c.mm = pl->second;
         if (sizeof(R) == 8 && axis == 0 && line_has_variant(c.key)) {
             // x blocks of the alternative shape hold a different number of lines
             const int la = line_block_lines_alt(c.key, 0);
@@ -402,6 +436,8 @@ int BatchCore::plan()
                 HostClass h;
                 h.key = c.key;
                 h.kind = c.kind;
+                h.axis = c.axis;
+                h.mm = c.mm;
                 h.fused = f != 0;
                 for (const LineItem &it : c.li)
                     if ((mfused_[it.solve] != 0) == h.fused) h.li.push_back(it);
@@ -484,20 +520,20 @@ int BatchCore::bind(char *base, TableCache *tc)
     for (auto *v : {&lx_, &ly_})
         for (HostClass &h : *v) {
             AxisDev t;
-            if ((rc = tc->get(h.key, t))) return rc;
-            tabs_[h.key] = t;
+            if ((rc = tc->get(h.key, h.kind, h.axis, t))) return rc;
+            tabs_[{h.key, h.kind, h.axis}] = t;
         }
     // periodic z: the complex FFT of length nz uses the twiddles of real lines of 2 nz; other
     // lengths take the real line tables of length nz
     for (HostClass &h : lzp_) {
         AxisDev t;
-        if ((rc = tc->get(2 * h.key, t))) return rc;
-        tabs_[2 * h.key] = t;
+        if ((rc = tc->get(2 * h.key, -1, 1, t))) return rc;
+        tabs_[{2 * h.key, -1, 1}] = t;
     }
     for (int m : zpl_) {
         AxisDev t;
-        if ((rc = tc->get(mem[m].g.nz, t))) return rc;
-        tabs_[mem[m].g.nz] = t;
+        if ((rc = tc->get(mem[m].g.nz, KIND_PP, 1, t))) return rc;
+        tabs_[{mem[m].g.nz, KIND_PP, 1}] = t;
     }
     if (precision == 1) {
         d_sums_ = (double *)(base + o_sums_);
@@ -618,9 +654,14 @@ int BatchCore::launch_class(hipStream_t s, const HostClass &c, int form, int axi
     {
         const int v = (form == FORM_F64 && line_has_variant(c.key)) ? (force_var >= 0 ? force_var : c.var[fwd ? 0 : 1]) : 0;
         const bool alt_items = v && axis == 0;
-        const AxisDev &t = tabs_.at(c.key);
+        const AxisDev &t = tabs_.at({c.key, c.kind, c.axis});
         LineArgs a{};
         a.variant = v;
+        a.mm = t.mm;
+        a.mmi = t.mmi;
+        a.mm_pw = c.mm.pw;
+        a.mm_units = c.mm.units;
+        a.mm_waves = c.mm.waves;
         a.in = in;
         a.out = out;
         a.tw = t.tw;
@@ -759,7 +800,7 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
         ZPerArgs zp{};
         zp.data = pdata;
         zp.nz = c.key;
-        zp.tw = tabs_.at(2 * c.key).tw;
+        zp.tw = tabs_.at({2 * c.key, -1, 1}).tw;
         zp.c2 = d_zc2_ + zc2_off_.at(c.key);
         zp.pinned_zero = f32 ? 1 : 0;
         zp.items = (const ZItem *)c.d_items;
@@ -768,7 +809,7 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
     }
     for (int m : zpl_) {
         const SolveSetup &g = mem[m].g;
-        const AxisDev &t = tabs_.at(g.nz);
+        const AxisDev &t = tabs_.at({g.nz, KIND_PP, 1});
         const long off = mem[m].offset;
         void *data = f32 ? (void *)(d_w + off) : (void *)(d_sol + off);
         ZPerArgs zp{};
@@ -791,6 +832,8 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
         a.B = t.B;
         a.C = t.C;
         a.D = t.D;
+        a.mm = t.mm;
+        a.mmi = t.mmi;
         a.in_scale = 1.0;
         a.out_scale = 1.0;
         a.nlines = (long)g.nx * g.ny;
@@ -876,7 +919,7 @@ int BatchCore::run_mixed(hipStream_t s, Marks *mk)
         // the corrections' x forward: fused members compute their residual inside it
         for (const HostClass &c : lxc_) {
             if (c.fused) {
-                const AxisDev &t = tabs_.at(c.key);
+                const AxisDev &t = tabs_.at({c.key, c.kind, c.axis});
                 LineArgs a{};
                 a.in = d_w;
                 a.out = d_w;

@@ -8,11 +8,13 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <map>
 #include <vector>
 
 #include "pp_launch.h"
 #include "pp_line.h"
+#include "pp_line_mm.h"
 #include "pp_mixed.h"
 #include "pp_setup.h"
 #include "pp_zsolve.h"
@@ -21,16 +23,20 @@ namespace pp {
 
 struct AxisDev {
     double *tw = nullptr, *A = nullptr, *B = nullptr, *C = nullptr, *D = nullptr;
+    double *mm = nullptr, *mmi = nullptr;  // dense-product matrices (one allocation, at mm)
 };
 
-// FP64 twiddle tables per line length, resident on the device until destruction
+// FP64 tables per line length (and, dense products, symmetry family), resident on the device
+// until destruction
 class TableCache {
   public:
     ~TableCache();
-    int get(int N, AxisDev &out);
+    // tables of lines of length N along x (axis 0) or across it; kind -1: the complex twiddles
+    // of a compiled plan only
+    int get(int N, int kind, int axis, AxisDev &out);
 
   private:
-    std::map<int, AxisDev> t_;
+    std::map<std::pair<int, int>, AxisDev> t_;  // {length, family (dense products) or -1}
 };
 
 // events recorded between the launches of one run (null ev: no timing)
@@ -91,7 +97,8 @@ class BatchCore {
 
   private:
     struct HostClass {
-        int key = 0, kind = 0, nitems = 0;
+        int key = 0, kind = 0, axis = 0, nitems = 0;
+        MmPlan mm{};  // dense-product line classes: the launch shape
         std::vector<LineItem> li;
         std::vector<ZItem> zi;
         size_t off = 0;
@@ -157,7 +164,7 @@ class BatchCore {
     // region layout (byte offsets)
     size_t o_zth_ = 0, o_zth_tab_ = 0, o_u0_ = 0, o_cacc_ = 0, o_zc2_ = 0, o_smt_ = 0, o_rhs_ = 0, o_sol_ = 0, o_tiles_ = 0, o_w_ = 0, o_lam_ = 0, o_dtab_ = 0, o_ls_ = 0, o_zs_ = 0, o_sums_ = 0, o_plane_ = 0,
            o_upart_ = 0, o_fix_ = 0, o_m00_ = 0, o_res_ = 0, o_ritems_ = 0, o_rpitems_ = 0;
-    std::map<int, AxisDev> tabs_;
+    std::map<std::array<int, 3>, AxisDev> tabs_;  // {length, kind, axis}; kind -1: complex z plans
     // device pointers of the tables
     double *d_lam_ = nullptr, *d_dtab_ = nullptr, *d_sums_ = nullptr, *d_plane_ = nullptr, *d_upart_ = nullptr;
     LineSolve *d_ls_ = nullptr;

@@ -14,6 +14,7 @@ namespace pp {
 // device table pointers of one axis (twiddles and transform tables, pp_setup.h)
 struct DevTables {
     void *tw = nullptr, *A = nullptr, *B = nullptr, *C = nullptr, *D = nullptr;
+    double *mm = nullptr, *mmi = nullptr;  // dense-product matrices (one allocation, at mm)
 };
 
 }  // namespace pp

@@ -92,9 +92,13 @@ struct LineArgs {
     int tile_w;  // tile width W (0: LINES, the block's column count); a multiple of LINES
     // host side, FP64 form: 1 = the alternative launch shape (line_threads_alt), 0 = default
     int variant;
-    // line length; read by the arbitrary-length kernels (pp_line_bs.h), whose length is not a
-    // template parameter
+    // line length; read by the arbitrary-length kernels (pp_line_bs.h, pp_line_mm.h), whose
+    // length is not a template parameter
     int n;
+    // forward and inverse matrices of the dense-product kernels (pp_line_mm.h); null: the
+    // Stockham plans or the chirp convolution.  Batched launches bring their shape (mm_plan)
+    const double *mm, *mmi;
+    int mm_pw, mm_units, mm_waves;
 };
 enum : int { ZT_OUT = 1, ZT_IN = 2 };
 

@@ -337,11 +337,4 @@ inline int bs_block_lines(int N, int AX)
 // every line length 2..1024: the compiled plans of pp_line.h, the rest through this file
 inline bool line_size_supported(int n) { return line_compiled(n) || (n >= 2 && n <= kBsMaxN); }
 
-// lines (x) or columns (y) per block of whichever launch serves length N
-template <typename R>
-inline int line_lines_any(int N, int AX)
-{
-    return line_compiled(N) ? line_block_lines<R>(N, AX) : bs_block_lines<R>(N, AX);
-}
-
 }  // namespace pp

@@ -40,6 +40,8 @@ struct Resident {
     size_t tab[2][5] = {};  // offsets (doubles) of tw, A, B, C, D per axis
     size_t ztab[5] = {};    // periodic z without a compiled complex plan: real z-line tables
     size_t lamx = 0, lamy = 0, dtab = 0, ztw = 0, zc2 = 0;
+    // dense-product lines (x, y, periodic z): where their matrices are written (0: none)
+    size_t mm[3] = {};
     int zsing_x = -1, zsing_y = -1;
     double zsing_eig = -2.0;
     size_t used = 0;  // doubles of scratch in use
@@ -56,10 +58,13 @@ bool same_key(const Resident &r, int nx, int ny, int nz, const char *bc, const d
            std::memcmp(r.bc, bc, 6) == 0 && std::memcmp(r.X, X, sizeof(r.X)) == 0;
 }
 
-// lay the tables of `g` out in g_host (offsets into r); false if they exceed kScratchDoubles
-bool build_host_tables(const SolveSetup &g, Resident &r)
+// lay the tables of `g` out in g_host (offsets into r); false if they exceed kScratchDoubles.
+// dense: lines without a compiled plan take the dense products (their octant table here, room
+// for their matrices behind the copied part), else the chirp convolution
+bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
 {
     size_t o = 0;
+    r = Resident{};
     auto take = [&](size_t n) {
         const size_t at = o;
         o += (n + 31) / 32 * 32;  // 256-byte aligned sub-arrays
@@ -67,6 +72,10 @@ bool build_host_tables(const SolveSetup &g, Resident &r)
     };
     const int n[2] = {g.nx, g.ny};
     for (int a = 0; a < 2; a++) {
+        if (dense && mm_serves(n[a], g.kind[a], a)) {
+            r.tab[a][1] = take(mm_octant_size(n[a]));
+            continue;
+        }
         const AxisTableSizes z = axis_table_sizes(n[a]);
         for (int i = 0; i < 5; i++) r.tab[a][i] = take(z.n[i]);
     }
@@ -79,16 +88,28 @@ bool build_host_tables(const SolveSetup &g, Resident &r)
         zs = axis_table_sizes(zc ? 2 * g.nz : g.nz);
         if (zc) {
             r.ztw = take(zs.n[0]);
+        } else if (dense && mm_serves(g.nz, KIND_PP, 1)) {
+            r.ztab[1] = take(mm_octant_size(g.nz));
         } else {
             for (int i = 0; i < 5; i++) r.ztab[i] = take(zs.n[i]);
         }
         r.zc2 = take((size_t)g.nz);
     }
+    r.used = o;
+    // the matrices are written on the device, behind the part that is copied
+    if (dense) {
+        for (int a = 0; a < 2; a++)
+            if (mm_serves(n[a], g.kind[a], a)) r.mm[a] = take(mm_tables_size(n[a], g.kind[a]));
+        if (g.zper && !zc && mm_serves(g.nz, KIND_PP, 1)) r.mm[2] = take(mm_tables_size(g.nz, KIND_PP));
+    }
     if (o > kScratchDoubles) return false;
-    std::memset(g_host, 0, o * sizeof(double));
-    for (int a = 0; a < 2; a++)
-        fill_axis_tables(n[a], g_host + r.tab[a][0], g_host + r.tab[a][1], g_host + r.tab[a][2], g_host + r.tab[a][3],
-                         g_host + r.tab[a][4]);
+    std::memset(g_host, 0, r.used * sizeof(double));
+    for (int a = 0; a < 2; a++) {
+        if (r.mm[a]) fill_mm_octant(n[a], g_host + r.tab[a][1]);
+        else
+            fill_axis_tables(n[a], g_host + r.tab[a][0], g_host + r.tab[a][1], g_host + r.tab[a][2],
+                             g_host + r.tab[a][3], g_host + r.tab[a][4]);
+    }
     fill_eig_factors(g, 0, g_host + r.lamx);
     fill_eig_factors(g, 1, g_host + r.lamy);
     fill_dirichlet_table(g, g_host + r.dtab);
@@ -98,6 +119,8 @@ bool build_host_tables(const SolveSetup &g, Resident &r)
             // complex FFT of length nz: only its twiddles are read
             static double unused[4][2 * 1024 + 2];
             fill_axis_tables(2 * g.nz, g_host + r.ztw, unused[0], unused[1], unused[2], unused[3]);
+        } else if (r.mm[2]) {
+            fill_mm_octant(g.nz, g_host + r.ztab[1]);
         } else {
             fill_axis_tables(g.nz, g_host + r.ztab[0], g_host + r.ztab[1], g_host + r.ztab[2], g_host + r.ztab[3],
                              g_host + r.ztab[4]);
@@ -121,7 +144,6 @@ bool build_host_tables(const SolveSetup &g, Resident &r)
                 }
             }
     }
-    r.used = o;
     return true;
 }
 
@@ -173,10 +195,17 @@ extern "C" int pp_solve_device_oop_noalloc(int nx, int ny, int nz, const char *b
             if (cs != hipStreamCaptureStatusNone) return PP_CALL_ORDER;
             g_res[dev].valid = false;
             Resident nr;
-            if (!build_host_tables(g, nr)) return PP_UNSUPPORTED_SIZE;
-            if (hipMemcpyAsync(base, g_host, nr.used * sizeof(double), hipMemcpyHostToDevice, s) != hipSuccess ||
-                hipStreamSynchronize(s) != hipSuccess)
+            // matrices that do not fit the array: the chirp convolution, whose tables do
+            if (!build_host_tables(g, nr, true) && !build_host_tables(g, nr, false)) return PP_UNSUPPORTED_SIZE;
+            if (hipMemcpyAsync(base, g_host, nr.used * sizeof(double), hipMemcpyHostToDevice, s) != hipSuccess)
                 return PP_HIP_ERROR;
+            const int len[3] = {nx, ny, nz}, kind[3] = {g.kind[0], g.kind[1], KIND_PP};
+            for (int a = 0; a < 3; a++) {
+                const double *oct = base + (a < 2 ? nr.tab[a][1] : nr.ztab[1]);
+                if (nr.mm[a] && launch_mm_tables(base + nr.mm[a], oct, len[a], kind[a], s) != hipSuccess)
+                    return PP_HIP_ERROR;
+            }
+            if (hipStreamSynchronize(s) != hipSuccess) return PP_HIP_ERROR;
             nr.nx = nx;
             nr.ny = ny;
             nr.nz = nz;
@@ -201,6 +230,10 @@ extern "C" int pp_solve_device_oop_noalloc(int nx, int ny, int nz, const char *b
     for (int a = 0; a < 2; a++) {
         void **t[5] = {&h.tab64[a].tw, &h.tab64[a].A, &h.tab64[a].B, &h.tab64[a].C, &h.tab64[a].D};
         for (int i = 0; i < 5; i++) *t[i] = base + r.tab[a][i];
+        if (r.mm[a]) {
+            h.tab64[a].mm = base + r.mm[a];
+            h.tab64[a].mmi = h.tab64[a].mm + mm_inverse_offset(a == 0 ? nx : ny, g.kind[a]);
+        }
     }
     h.d_lamx = base + r.lamx;
     h.d_lamy = base + r.lamy;
@@ -211,6 +244,10 @@ extern "C" int pp_solve_device_oop_noalloc(int nx, int ny, int nz, const char *b
         } else {
             void **t[5] = {&h.tabz.tw, &h.tabz.A, &h.tabz.B, &h.tabz.C, &h.tabz.D};
             for (int i = 0; i < 5; i++) *t[i] = base + r.ztab[i];
+            if (r.mm[2]) {
+                h.tabz.mm = base + r.mm[2];
+                h.tabz.mmi = h.tabz.mm + mm_inverse_offset(nz, KIND_PP);
+            }
         }
         h.d_zc2 = base + r.zc2;
         h.zsing_x = r.zsing_x;

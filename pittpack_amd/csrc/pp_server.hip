@@ -444,7 +444,7 @@ int pp_server_create(long long hbm_bytes, long long staging_bytes, int streams, 
     for (int n = 16; n <= 1024; n += 2)
         if (line_compiled(n)) {
             AxisDev t;
-            const int rc = s->tables.get(n, t);
+            const int rc = s->tables.get(n, -1, 0, t);
             if (rc) return fail(rc);
         }
     s->worker = std::thread(worker_loop, s);

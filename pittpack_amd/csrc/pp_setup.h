@@ -15,6 +15,7 @@
 #include "pittpack_hip.h"
 #include "pp_line.h"
 #include "pp_line_bs.h"
+#include "pp_line_mm.h"
 
 namespace pp {
 
@@ -221,6 +222,17 @@ inline const AxisTables &axis_tables_cached(int N)
         make_axis_tables(N, *p);
     }
     return *p;
+}
+
+// octant table of the dense-product transforms (pp_line_mm.h): {cos, sin}(2 pi q / (8 N)),
+// q = 0 .. N
+inline void fill_mm_octant(int N, double *oct)
+{
+    const long double step = 3.141592653589793238462643383279502884L / (4 * (long double)N);
+    for (int q = 0; q <= N; q++) {
+        oct[2 * q] = (double)std::cos(q * step);
+        oct[2 * q + 1] = (double)std::sin(q * step);
+    }
 }
 
 // everything one solve's kernels need from (sizes, bc, box)

@@ -16,6 +16,7 @@
 #include "pittpack_hip.h"
 #include "pp_line.h"
 #include "pp_line_bs.h"
+#include "pp_line_mm.h"
 #include "pp_launch.h"
 #include "pp_mixed.h"
 #include "pp_resx.h"
@@ -60,10 +61,29 @@ extern template hipError_t launch_line_bs_kind<KIND_PP>(int, int, int, const Lin
 extern template hipError_t launch_line_bs_kind<KIND_ND>(int, int, int, const LineArgs &, hipStream_t);
 extern template hipError_t launch_line_bs_kind<KIND_DN>(int, int, int, const LineArgs &, hipStream_t);
 
-// line transforms: one translation unit per kind (pp_line_<kind>.hip for the compiled
-// lengths, pp_line_bs_<kind>.hip for the others)
+extern template hipError_t launch_line_mm_kind<KIND_DD>(int, int, int, const LineArgs &, hipStream_t);
+extern template hipError_t launch_line_mm_kind<KIND_NN>(int, int, int, const LineArgs &, hipStream_t);
+extern template hipError_t launch_line_mm_kind<KIND_PP>(int, int, int, const LineArgs &, hipStream_t);
+extern template hipError_t launch_line_mm_kind<KIND_ND>(int, int, int, const LineArgs &, hipStream_t);
+extern template hipError_t launch_line_mm_kind<KIND_DN>(int, int, int, const LineArgs &, hipStream_t);
+
+// line transforms: one translation unit per kind (pp_line_<kind>.hip for the compiled lengths,
+// pp_line_mm_<kind>.hip for the dense products where the caller brings their matrices,
+// pp_line_bs_<kind>.hip for the rest)
 hipError_t launch_line(int form, int kind, int N, int AX, int FWD, const LineArgs &a0, hipStream_t s)
 {
+    if (a0.mm) {
+        LineArgs a = a0;
+        a.n = N;
+        switch (kind) {
+        case KIND_DD: return launch_line_mm_kind<KIND_DD>(form, AX, FWD, a, s);
+        case KIND_NN: return launch_line_mm_kind<KIND_NN>(form, AX, FWD, a, s);
+        case KIND_PP: return launch_line_mm_kind<KIND_PP>(form, AX, FWD, a, s);
+        case KIND_ND: return launch_line_mm_kind<KIND_ND>(form, AX, FWD, a, s);
+        case KIND_DN: return launch_line_mm_kind<KIND_DN>(form, AX, FWD, a, s);
+        default: return hipErrorInvalidValue;
+        }
+    }
     if (!line_compiled(N)) {
         LineArgs a = a0;
         a.n = N;
@@ -231,6 +251,8 @@ void free_tables(pp_solver *h)
             if (*p) (void)hipFree(*p);
             *p = nullptr;
         }
+        if (t->mm) (void)hipFree(t->mm);
+        t->mm = t->mmi = nullptr;
     }
     for (double **p : {&h->d_lamx, &h->d_lamy, &h->d_dtab, &h->d_ztw, &h->d_zc2}) {
         if (*p) (void)hipFree(*p);
@@ -246,6 +268,30 @@ int upload(void **dst, const std::vector<double> &v)
     return PP_SUCCESS;
 }
 
+// The tables of lines of length n and kind `kind` along x (axis 0) or across it: the dense products' matrices (their octant
+// table stays in A), or the Stockham / chirp convolution tables
+int upload_axis(pp_solver *h, int n, int kind, int axis, DevTables &d)
+{
+    int rc;
+    if (mm_serves(n, kind, axis)) {
+        std::vector<double> oct(mm_octant_size(n));
+        fill_mm_octant(n, oct.data());
+        if ((rc = upload(&d.A, oct))) return rc;
+        if (hipMalloc((void **)&d.mm, mm_tables_size(n, kind) * sizeof(double)) != hipSuccess) {
+            d.mm = nullptr;
+            return PP_ALLOCATION_FAIL;
+        }
+        d.mmi = d.mm + mm_inverse_offset(n, kind);
+        PP_HIP_CHECK(launch_mm_tables(d.mm, (const double *)d.A, n, kind, h->stream));
+        return PP_SUCCESS;
+    }
+    const AxisTables &t = axis_tables_cached(n);
+    if ((rc = upload(&d.tw, t.tw)) || (rc = upload(&d.A, t.A)) || (rc = upload(&d.B, t.B)) ||
+        (rc = upload(&d.C, t.C)) || (rc = upload(&d.D, t.D)))
+        return rc;
+    return PP_SUCCESS;
+}
+
 // Build everything that depends on (sizes, bc, box): eigenvalue factors, twiddles and the
 // Dirichlet boundary term tables.  Mirrors assignBoundary/setEigenVal/setScale/setCoords.
 int build_tables(pp_solver *h)
@@ -253,15 +299,8 @@ int build_tables(pp_solver *h)
     free_tables(h);
     const int n[2] = {h->g.nx, h->g.ny};
     int rc;
-    for (int a = 0; a < 2; a++) {
-        const AxisTables &t = axis_tables_cached(n[a]);
-        DevTables &d = h->tab64[a];
-        if ((rc = upload(&d.tw, t.tw))) return rc;
-        if ((rc = upload(&d.A, t.A))) return rc;
-        if ((rc = upload(&d.B, t.B))) return rc;
-        if ((rc = upload(&d.C, t.C))) return rc;
-        if ((rc = upload(&d.D, t.D))) return rc;
-    }
+    for (int a = 0; a < 2; a++)
+        if ((rc = upload_axis(h, n[a], h->g.kind[a], a, h->tab64[a]))) return rc;
     const std::vector<double> lx = eig_factors(h->g, 0), ly = eig_factors(h->g, 1);
     if ((rc = upload((void **)&h->d_lamx, lx))) return rc;
     if ((rc = upload((void **)&h->d_lamy, ly))) return rc;
@@ -276,11 +315,7 @@ int build_tables(pp_solver *h)
             if ((rc = upload((void **)&h->d_ztw, zt.tw))) return rc;
         } else {
             // real z-line transforms of length nz (R2HC / HC2R)
-            make_axis_tables(h->g.nz, zt);
-            DevTables &d = h->tabz;
-            if ((rc = upload(&d.tw, zt.tw)) || (rc = upload(&d.A, zt.A)) || (rc = upload(&d.B, zt.B)) ||
-                (rc = upload(&d.C, zt.C)) || (rc = upload(&d.D, zt.D)))
-                return rc;
+            if ((rc = upload_axis(h, h->g.nz, KIND_PP, 1, h->tabz))) return rc;
         }
         if ((rc = upload((void **)&h->d_zc2, zper_cos2(h->g.nz)))) return rc;
         const double Cx = (h->g.dxyz[2] / h->g.dxyz[0]) * (h->g.dxyz[2] / h->g.dxyz[0]);
@@ -338,6 +373,8 @@ LineArgs line_args(pp_solver *h, int axis, double *field)
     a.B = (const double *)t.B;
     a.C = (const double *)t.C;
     a.D = (const double *)t.D;
+    a.mm = t.mm;
+    a.mmi = t.mmi;
     a.in_scale = 1.0;
     a.out_scale = 1.0;
     a.dtab = h->d_dtab;
@@ -367,7 +404,7 @@ bool use_ztiles(pp_solver *h)
     // in-place layout)
     if (!h->ztiles || h->zsolver != 0 || h->g.zper) return false;
     if (!zsolve_supported_f64(h->g.nz) && !zsolve_long_supported_f64(h->g.nz)) return false;
-    const int ly = line_lines_any<double>(h->g.ny, 1);
+    const int ly = line_lines_any<double>(h->g.ny, h->g.kind[1], 1);
     return ly > 0 && zsolve_cpb<double>() % ly == 0;
 }
 
@@ -420,6 +457,8 @@ int run_zperiodic(pp_solver *h, void *data, bool f32)
     a.B = (const double *)t.B;
     a.C = (const double *)t.C;
     a.D = (const double *)t.D;
+    a.mm = t.mm;
+    a.mmi = t.mmi;
     a.in_scale = 1.0;
     a.out_scale = 1.0;
     a.nlines = (long)h->g.nx * h->g.ny;
