@@ -20,6 +20,7 @@
 
 #include "pp_line.h"
 #include "pp_mixed.h"
+#include "pp_zsing.h"
 #include "pp_zsolve.h"
 
 namespace pp {
@@ -114,8 +115,9 @@ __global__ void __launch_bounds__(256) k_zfix64(ZArgs a0, const int4 *cols)
     for (int i = threadIdx.x; i < n; i += blockDim.x) data[off + (long)i * zs] = (R)(rd[i] / rb[i]);
 }
 
-// One block, FP64, for the pinned (0,0) column.  R(z) = sum_y line_sums[y + ny z] is the
-// column's right-hand side (plane sums of the forward-x input).
+// The pinned (0,0) column in FP64.  R(z) = sum_y line_sums[y + ny z] is the column's right-hand
+// side (plane sums of the forward-x input); k_plane_sums leaves it in plane_add[0 .. nz), whose
+// previous contents the last inverse-x store has read.
 //  initial (correct == 0): solve P u = R with P the pinned operator (row 0: u0 = r0,
 //      interior 1 -2 1, last row bn); plane_add[z] = u(z)/(NxNy);
 //      plane_add[nz] = (b0 u0 + u1 - S0)/(NxNy), the row-0 defect of the unpinned operator,
@@ -125,22 +127,39 @@ __global__ void __launch_bounds__(256) k_zfix64(ZArgs a0, const int4 *cols)
 //      kernel's per-block partial sums upart[0..nparts).  plane_add[z] = du(z)/(NxNy).
 // Periodic z (zper): the column is the reference's singular cyclic one
 // (shermanMorrisonThomasV1, src/triDiag.cpp:2112-2255), i.e. the cyclic operator with row 0
-// replaced by u0 + u_{N-1} = (r0 + r_{N-1})/2, solved by the same Sherman-Morrison sweeps as
-// k_smt_v1; plane_add[nz] = (u_{N-1} - 2 u0 + u1 - S0)/(NxNy) and plane_add[nz+1] = the
-// row-0 target (S0 + S_{N-1})/2; in a correction, row 0 is that target minus the sum of the
-// current u over planes 0 and N-1 (the residual kernel's partial sums take both planes).
-__device__ void mode00_body(const double *line_sums, int ny, int nz, double b0, double bn, double inv_scale,
-                            double *plane_add, const double *upart, int nparts, int correct, int zper)
+// replaced by u0 + u_{N-1} = (r0 + r_{N-1})/2; plane_add[nz] = (u_{N-1} - 2 u0 + u1 - S0)/(NxNy) and
+// plane_add[nz+1] = the row-0 target (S0 + S_{N-1})/2; in a correction, row 0 is that target minus
+// the sum of the current u over planes 0 and N-1 (the residual kernel's partial sums take both
+// planes).
+// One wave per plane: 512^2 line sums are 2 MB, which a single block read in 20 us
+__device__ void plane_sum(const double *line_sums, int ny, int nz, double *plane_add)
+{
+    const int z = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (z >= nz) return;
+    double acc = 0.0;
+    for (int y = lane; y < ny; y += 64) acc += line_sums[(long)z * ny + y];
+    for (int s = 32; s > 0; s >>= 1) acc += __shfl_xor(acc, s, 64);
+    if (lane == 0) plane_add[z] = acc;
+}
+
+__global__ void __launch_bounds__(256) k_plane_sums(const double *line_sums, int ny, int nz, double *plane_add)
+{
+    plane_sum(line_sums, ny, nz, plane_add);
+}
+
+__global__ void __launch_bounds__(256) k_plane_sums_batch(const Mode00Item *items)
+{
+    const Mode00Item it = items[blockIdx.y];
+    plane_sum(it.line_sums, it.ny, it.nz, it.plane_add);
+}
+
+__device__ void mode00_body(int nz, double b0, double bn, double inv_scale, double *plane_add, const double *upart,
+                            int nparts, int correct, int zper)
 {
     extern __shared__ double m0[];
     double *r = m0;
-    double *cp = m0 + nz;
-    __shared__ double red[1024];
-    for (int z = threadIdx.x; z < nz; z += blockDim.x) {
-        double acc = 0.0;
-        for (int y = 0; y < ny; y++) acc += line_sums[(long)z * ny + y];
-        r[z] = acc;
-    }
+    __shared__ double red[256];
+    for (int z = threadIdx.x; z < nz; z += blockDim.x) r[z] = plane_add[z];
     double part = 0.0;
     if (correct)
         for (int i = threadIdx.x; i < nparts; i += blockDim.x) part += upart[i];
@@ -150,75 +169,34 @@ __device__ void mode00_body(const double *line_sums, int ny, int nz, double b0, 
         if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0 && zper) {
-        const double s0 = r[0];
-        const double target = correct ? plane_add[nz + 1] : (r[0] + r[nz - 1]) * 0.5;
-        r[0] = correct ? target - red[0] : target;
-        // thomasLowMemNoBCV1 sweeps of shermanMorrisonThomasV1 (b = {1, -2, -2}, gamma = -1,
-        // alpha = beta = 1): row 0 decoupled with diagonal 2, interior 1 -2 1, last row -1
-        const double bb[3] = {2.0, -2.0, -1.0};
-        auto sweep = [&](double *x) {
-            double bet = bb[0];
-            x[0] = x[0] / bet;
-            cp[1] = 0.0;
-            bet = bb[1];
-            x[1] = (x[1] - x[0]) / bet;
-            for (int j = 2; j < nz - 1; j++) {
-                cp[j] = 1.0 / bet;
-                bet = bb[1] - cp[j];
-                x[j] = (x[j] - x[j - 1]) / bet;
-            }
-            cp[nz - 1] = 1.0 / bet;
-            bet = bb[2] - cp[nz - 1];
-            x[nz - 1] = (x[nz - 1] - x[nz - 2]) / bet;
-            for (int j = nz - 2; j >= 0; j--) x[j] -= cp[j + 1] * x[j + 1];
-        };
-        double *q = red;  // the Sherman-Morrison vector (the reduction is done with red)
-        sweep(r);
-        for (int i = 0; i < nz; i++) q[i] = 0.0;
-        q[0] = -1.0;
-        q[nz - 1] = 1.0;
-        sweep(q);
-        const double fact = (r[0] - r[nz - 1]) / (1. + q[0] - q[nz - 1]);
-        for (int i = 0; i < nz; i++) r[i] -= fact * q[i];
-        if (!correct) {
-            plane_add[nz] = (r[nz - 1] - 2.0 * r[0] + r[1] - s0) * inv_scale;
-            plane_add[nz + 1] = target;
-        }
-    } else if (threadIdx.x == 0) {
-        const double s0 = correct ? plane_add[nz + 1] : r[0];
-        if (correct) r[0] = s0 - red[0];
-        cp[0] = 0.0;
-        for (int i = 1; i < nz; i++) {
-            const double b = (i == nz - 1) ? bn : -2.0;
-            const double c = (i == nz - 1) ? 0.0 : 1.0;
-            const double inv = 1.0 / (b - cp[i - 1]);
-            cp[i] = c * inv;
-            r[i] = (r[i] - r[i - 1]) * inv;
-        }
-        for (int i = nz - 2; i >= 0; i--) r[i] = r[i] - cp[i] * r[i + 1];
-        if (!correct) {
-            plane_add[nz] = (b0 * r[0] + r[1] - s0) * inv_scale;
-            plane_add[nz + 1] = s0;
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x;
+        const double s0 = r[0], t0 = correct ? plane_add[nz + 1] : (zper ? (r[0] + r[nz - 1]) * 0.5 : r[0]);
+        const double row0 = correct ? t0 - red[0] : t0;
+        __builtin_amdgcn_wave_barrier();
+        if (zper) singular_periodic_column(r, nz, row0, lane);
+        else singular_column(r, nz, row0, bn, lane);
+        __builtin_amdgcn_wave_barrier();
+        if (lane == 0 && !correct) {
+            plane_add[nz] = ((zper ? r[nz - 1] - 2.0 * r[0] : b0 * r[0]) + r[1] - s0) * inv_scale;
+            plane_add[nz + 1] = t0;
         }
     }
     __syncthreads();
     for (int z = threadIdx.x; z < nz; z += blockDim.x) plane_add[z] = r[z] * inv_scale;
 }
 
-__global__ void __launch_bounds__(1024) k_mode00(const double *line_sums, int ny, int nz, double b0, double bn,
-                                                 double inv_scale, double *plane_add, const double *upart, int nparts,
-                                                 int correct, int zper)
+__global__ void __launch_bounds__(256) k_mode00(int nz, double b0, double bn, double inv_scale, double *plane_add,
+                                                const double *upart, int nparts, int correct, int zper)
 {
-    mode00_body(line_sums, ny, nz, b0, bn, inv_scale, plane_add, upart, nparts, correct, zper);
+    mode00_body(nz, b0, bn, inv_scale, plane_add, upart, nparts, correct, zper);
 }
 
 // batched: block b handles pinned member items[b]
-__global__ void __launch_bounds__(1024) k_mode00_batch(const Mode00Item *items, int correct)
+__global__ void __launch_bounds__(256) k_mode00_batch(const Mode00Item *items, int correct)
 {
     const Mode00Item it = items[blockIdx.x];
-    mode00_body(it.line_sums, it.ny, it.nz, it.b0, it.bn, it.inv_scale, it.plane_add, it.upart, it.nparts, correct,
-                it.zper);
+    mode00_body(it.nz, it.b0, it.bn, it.inv_scale, it.plane_add, it.upart, it.nparts, correct, it.zper);
 }
 
 constexpr int RES_ZC = 30;  // planes marched per thread (a multiple of the 3-plane unroll)
@@ -656,10 +634,10 @@ hipError_t launch_zfix64_f32(const ZArgs &a, const int4 *cols, int ncols, int nz
 hipError_t launch_mode00(const double *line_sums, int ny, int nz, double b0, double bn, double inv_scale,
                          double *plane_add, const double *upart, int nparts, int correct, int zper, hipStream_t s)
 {
-    if (nz > 1024 || (zper && nz < 3)) return hipErrorInvalidValue;  // red[] holds the periodic column's vector
-    const size_t lds = 2 * (size_t)nz * sizeof(double);
-    hipLaunchKernelGGL(k_mode00, dim3(1), dim3(1024), lds, s, line_sums, ny, nz, b0, bn, inv_scale, plane_add, upart,
-                       nparts, correct, zper);
+    if (nz > 1024 || nz < 3) return hipErrorInvalidValue;  // singular_column: 16 rows a lane, three at least
+    hipLaunchKernelGGL(k_plane_sums, dim3((unsigned)((nz + 3) / 4)), dim3(256), 0, s, line_sums, ny, nz, plane_add);
+    hipLaunchKernelGGL(k_mode00, dim3(1), dim3(256), (size_t)nz * sizeof(double), s, nz, b0, bn, inv_scale, plane_add,
+                       upart, nparts, correct, zper);
     return hipGetLastError();
 }
 
@@ -667,8 +645,8 @@ hipError_t launch_mode00_batch(const Mode00Item *items, int nitems, int nz_max, 
 {
     if (nitems == 0) return hipSuccess;
     if (nz_max > 1024) return hipErrorInvalidValue;
-    const size_t lds = 2 * (size_t)nz_max * sizeof(double);
-    hipLaunchKernelGGL(k_mode00_batch, dim3(nitems), dim3(1024), lds, s, items, correct);
+    hipLaunchKernelGGL(k_plane_sums_batch, dim3((unsigned)((nz_max + 3) / 4), (unsigned)nitems), dim3(256), 0, s, items);
+    hipLaunchKernelGGL(k_mode00_batch, dim3(nitems), dim3(256), (size_t)nz_max * sizeof(double), s, items, correct);
     return hipGetLastError();
 }
 

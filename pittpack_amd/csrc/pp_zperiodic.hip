@@ -10,7 +10,7 @@
 // The singular column (|eig + 2| < 1e-10: x and y in {P, N}, mode (0, 0)) follows the
 // reference's own branch (shermanMorrisonThomasV1, src/triDiag.cpp:2112-2255: first row
 // replaced by the average of the first and last right-hand sides, pinned Thomas sweeps and
-// the Sherman-Morrison correction), restated serially in FP64 by k_smt_v1.  The mixed form
+// the Sherman-Morrison correction), in FP64 by k_smt_v1.  The mixed form
 // solves that column from FP64 plane sums instead (k_mode00, pp_mixed.hip) and has it
 // written as zeros here.
 //
@@ -25,6 +25,7 @@
 #include "pp_fft.h"
 #include "pp_launch.h"
 #include "pp_line.h"
+#include "pp_zsing.h"
 #include "pp_zsolve.h"
 
 namespace pp {
@@ -91,7 +92,9 @@ __global__ void __launch_bounds__(T *LINES) k_zper(ZPerArgs a)
     }
 }
 
-// the reference's singular periodic branch on one column (sx, sy), FP64, serial
+// the reference's singular periodic branch on one column (sx, sy), FP64: by scans where the
+// diagonal is exactly -2 (mode (0, 0) of periodic and Neumann axes); a diagonal only within 1e-10 of
+// it (cells 1e5 times thinner in z) takes the reference's sweeps, whose factors carry it
 __device__ void smt_v1_body(double *data, int SX, int SY, int nz, int sx, int sy, double diag)
 {
     extern __shared__ double sv[];
@@ -99,7 +102,9 @@ __device__ void smt_v1_body(double *data, int SX, int SY, int nz, int sx, int sy
     const long stride = (long)SX * SY, base = (long)sy * SX + sx;
     for (int i = threadIdx.x; i < nz; i += blockDim.x) rh[i] = data[base + i * stride];
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (diag == -2.0 && nz >= 3) {
+        if (threadIdx.x < 64) singular_periodic_column(rh, nz, (rh[0] + rh[nz - 1]) * 0.5, threadIdx.x);
+    } else if (threadIdx.x == 0) {
         const int N = nz;
         const double alpha = 1.0, beta = 1.0;
         // shermanMorrisonThomasV1 with b = {1, diag, diag}
