@@ -241,7 +241,7 @@ void BatchCore::plan_z()
                     for (int sx = 0; sx < g.nx && !found; sx++) {
                         const double eig = column_eig(lx, ly, sx, sy, Cx, Cy);
                         if (std::fabs(eig + 2.) < 1.e-10) {
-                            smt_.push_back({mem[m].offset, g.nx, g.ny, g.nz, sx, sy, eig});
+                            smt_.push_back({mem[m].offset + (long)sy * g.nx + sx, (long)g.nx * g.ny, g.nz, eig});
                             smt_nz_max_ = std::max(smt_nz_max_, g.nz);
                             found = true;
                         }
@@ -523,12 +523,11 @@ int BatchCore::bind(char *base, TableCache *tc)
             if ((rc = tc->get(h.key, h.kind, h.axis, t))) return rc;
             tabs_[{h.key, h.kind, h.axis}] = t;
         }
-    // periodic z: the complex FFT of length nz uses the twiddles of real lines of 2 nz; other
-    // lengths take the real line tables of length nz
+    // periodic z: line tables of length nz
     for (HostClass &h : lzp_) {
         AxisDev t;
-        if ((rc = tc->get(2 * h.key, -1, 1, t))) return rc;
-        tabs_[{2 * h.key, -1, 1}] = t;
+        if ((rc = tc->get(h.key, -1, 1, t))) return rc;
+        tabs_[{h.key, -1, 1}] = t;
     }
     for (int m : zpl_) {
         AxisDev t;
@@ -800,7 +799,8 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
         ZPerArgs zp{};
         zp.data = pdata;
         zp.nz = c.key;
-        zp.tw = tabs_.at({2 * c.key, -1, 1}).tw;
+        zp.tw = tabs_.at({c.key, -1, 1}).tw;
+        zp.A = tabs_.at({c.key, -1, 1}).A;
         zp.c2 = d_zc2_ + zc2_off_.at(c.key);
         zp.pinned_zero = f32 ? 1 : 0;
         zp.items = (const ZItem *)c.d_items;

@@ -29,8 +29,10 @@ struct pp_solver {
     bool own_stream = false;
     double *d_field = nullptr;
     double *d_lamx = nullptr, *d_lamy = nullptr, *d_dtab = nullptr;
-    double *d_ztw = nullptr, *d_zc2 = nullptr;  // periodic z: twiddles and 2 cos(2 pi k / nz)
+    double *d_ztw = nullptr, *d_zA = nullptr;   // periodic z: line tables tw and A of length nz
+    double *d_zc2 = nullptr;                    //   and 2 cos(2 pi k / nz)
     double *d_zt = nullptr;                     // z tiles of the FP64 form
+    bool no_zt = false;                         // periodic z: no room for them, in place instead
     int ztiles = 1;                             // PP_OPT_ZLAYOUT
     // autotuner (PP_OPT_AUTOTUNE): launch shape per FP64 line stage (x fwd, y fwd, y inv,
     // x inv; 1 = line_threads_alt) and the z configuration, chosen by timing
@@ -59,7 +61,7 @@ struct pp_solver {
     double zsing_eig = -2.0;
     std::vector<double> lamx_h, lamy_h;  // host copies of the eigenvalue factors
     pp::DevTables tab64[2];
-    pp::DevTables tabz;  // periodic z without a compiled complex plan: real z-line tables
+    pp::DevTables tabz;  // periodic z without a compiled plan: real z-line tables
     // kernel-timing ring: slot s holds up to kMaxMarks events recorded between the kernel
     // launches of one solve
     static constexpr int kMaxMarks = 64;

@@ -61,11 +61,15 @@ inline void zthomas_factors(double eig, double b0, double bn, int n, double *out
 // periodic z (pp_zperiodic.hip): circulant columns by z FFT, FP64 arithmetic on FP64 or FP32
 // storage; the singular column by the reference's own branch
 struct ZPerArgs {
-    void *data;  // [nz][SY][SX], in place; double (f64 launchers) or float (f32 launchers)
+    // [nz][SY][SX], in place, or (tile_rows > 0) 16-column z tiles: element (x, y, z) at
+    // ((x/16 * SY + y) * tile_rows + z) * 16 + x%16, every tile whole; double (f64 launchers) or
+    // float (f32 launchers)
+    void *data;
     int SX, SY, nz;
+    int tile_rows;
     const double *lamx, *lamy;
     double Cx, Cy;
-    const double *tw;
+    const double *tw, *A;  // line tables of length nz (pp_setup.h)
     const double *c2;
     // mixed form: the singular column is written as zeros (its contribution is solved from
     // plane sums in FP64 elsewhere); otherwise it is left for the reference's branch
@@ -76,7 +80,7 @@ struct ZPerArgs {
     const ZItem *items;
     const ZSolve *solves;
 };
-// one-pass kernel: nz with a compiled complex plan (zperiodic_supported); other nz: real
+// one-pass kernel: nz with a compiled line plan (zperiodic_supported); other nz: real
 // z-line transforms around launch_zper_divide
 bool zperiodic_supported(int nz);
 int zper_lines(int nz);  // columns per block of the one-pass kernel
@@ -87,13 +91,14 @@ hipError_t launch_zperiodic_f64_batch(const ZPerArgs &a, int nitems, hipStream_t
 hipError_t launch_zperiodic_f32_batch(const ZPerArgs &a, int nitems, hipStream_t s);
 hipError_t launch_zper_divide(const ZPerArgs &a, hipStream_t s);
 hipError_t launch_zper_divide_f32(const ZPerArgs &a, hipStream_t s);
-hipError_t launch_smt_v1(double *data, int SX, int SY, int nz, int sx, int sy, double diag, hipStream_t s);
-// the singular column of several solves (batched form): one block per item
+// the singular column: element z at data[offset + z * stride]
 struct SmtItem {
-    long offset;  // element offset of the solve's field in the data arena
-    int SX, SY, nz, sx, sy;
+    long offset, stride;
+    int nz;
     double diag;
 };
+hipError_t launch_smt_v1(double *data, const SmtItem &it, hipStream_t s);
+// the singular columns of several solves (batched form): one block per item
 hipError_t launch_smt_v1_batch(double *data, const SmtItem *items, int nitems, int nz_max, hipStream_t s);
 
 // counter-generator right-hand side (pp_solver.hip): out[i] = 2 u - 1,

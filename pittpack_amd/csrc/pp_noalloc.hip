@@ -38,8 +38,8 @@ struct Resident {
     char bc[6] = {};
     double X[6] = {};
     size_t tab[2][5] = {};  // offsets (doubles) of tw, A, B, C, D per axis
-    size_t ztab[5] = {};    // periodic z without a compiled complex plan: real z-line tables
-    size_t lamx = 0, lamy = 0, dtab = 0, ztw = 0, zc2 = 0;
+    size_t ztab[5] = {};    // periodic z without a compiled plan: real z-line tables
+    size_t lamx = 0, lamy = 0, dtab = 0, ztw = 0, zA = 0, zc2 = 0;
     // dense-product lines (x, y, periodic z): where their matrices are written (0: none)
     size_t mm[3] = {};
     int zsing_x = -1, zsing_y = -1;
@@ -85,9 +85,10 @@ bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
     const bool zc = g.zper && zperiodic_supported(g.nz);
     AxisTableSizes zs{};
     if (g.zper) {
-        zs = axis_table_sizes(zc ? 2 * g.nz : g.nz);
+        zs = axis_table_sizes(g.nz);
         if (zc) {
             r.ztw = take(zs.n[0]);
+            r.zA = take(zs.n[1]);
         } else if (dense && mm_serves(g.nz, KIND_PP, 1)) {
             r.ztab[1] = take(mm_octant_size(g.nz));
         } else {
@@ -116,9 +117,9 @@ bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
     r.zsing_x = r.zsing_y = -1;
     if (g.zper) {
         if (zc) {
-            // complex FFT of length nz: only its twiddles are read
-            static double unused[4][2 * 1024 + 2];
-            fill_axis_tables(2 * g.nz, g_host + r.ztw, unused[0], unused[1], unused[2], unused[3]);
+            // only tw and A of the line tables are read
+            static double unused[3][1024 + 2];
+            fill_axis_tables(g.nz, g_host + r.ztw, g_host + r.zA, unused[0], unused[1], unused[2]);
         } else if (r.mm[2]) {
             fill_mm_octant(g.nz, g_host + r.ztab[1]);
         } else {
@@ -241,6 +242,7 @@ extern "C" int pp_solve_device_oop_noalloc(int nx, int ny, int nz, const char *b
     if (g.zper) {
         if (zperiodic_supported(nz)) {
             h.d_ztw = base + r.ztw;
+            h.d_zA = base + r.zA;
         } else {
             void **t[5] = {&h.tabz.tw, &h.tabz.A, &h.tabz.B, &h.tabz.C, &h.tabz.D};
             for (int i = 0; i < 5; i++) *t[i] = base + r.ztab[i];

@@ -254,7 +254,7 @@ void free_tables(pp_solver *h)
         if (t->mm) (void)hipFree(t->mm);
         t->mm = t->mmi = nullptr;
     }
-    for (double **p : {&h->d_lamx, &h->d_lamy, &h->d_dtab, &h->d_ztw, &h->d_zc2}) {
+    for (double **p : {&h->d_lamx, &h->d_lamy, &h->d_dtab, &h->d_ztw, &h->d_zA, &h->d_zc2}) {
         if (*p) (void)hipFree(*p);
         *p = nullptr;
     }
@@ -309,10 +309,9 @@ int build_tables(pp_solver *h)
     if ((rc = upload((void **)&h->d_dtab, dirichlet_table(h->g)))) return rc;
     h->zsing_x = h->zsing_y = -1;
     if (h->g.zper) {
-        AxisTables zt;
         if (zperiodic_supported(h->g.nz)) {
-            make_axis_tables(2 * h->g.nz, zt);  // complex FFT of length nz
-            if ((rc = upload((void **)&h->d_ztw, zt.tw))) return rc;
+            const AxisTables &zt = axis_tables_cached(h->g.nz);
+            if ((rc = upload((void **)&h->d_ztw, zt.tw)) || (rc = upload((void **)&h->d_zA, zt.A))) return rc;
         } else {
             // real z-line transforms of length nz (R2HC / HC2R)
             if ((rc = upload_axis(h, h->g.nz, KIND_PP, 1, h->tabz))) return rc;
@@ -397,13 +396,21 @@ LineArgs line_args(pp_solver *h, int axis, double *field)
 // (x/16, y) tile of nz rows x 16 columns (one 128-byte line per row) contiguously, so the z
 // solve reads and writes whole tiles instead of one row per z plane.  y blocks of 16 columns
 // fill a tile, y blocks of 8 (1280- to 2048-byte y lines' LDS slices) half of one; z blocks
-// take a whole tile (up to 512 rows) or half (longer columns).  z not periodic.
+// take a whole tile (up to 512 rows) or half (longer columns).  Periodic z: where the one-pass
+// kernel takes the column (others go through z-line transforms of the whole field), from 512 rows,
+// whose planes lie far apart in memory: 512^3 0.72 -> 0.57 ms, 256^2 x 1024 0.45 -> 0.35 ms; shorter
+// columns measured the same either way (256^3 72 / 68 us, 384 x 256 x 320 175 / 178 us) and are
+// spared the second field.
 bool use_ztiles(pp_solver *h)
 {
     // (the partitioned solver rounds its rows per lane up to a coarser set, so it keeps the
     // in-place layout)
-    if (!h->ztiles || h->zsolver != 0 || h->g.zper) return false;
-    if (!zsolve_supported_f64(h->g.nz) && !zsolve_long_supported_f64(h->g.nz)) return false;
+    if (!h->ztiles) return false;
+    if (h->g.zper) {
+        if (h->no_zt || h->g.nz < 512 || !zperiodic_supported(h->g.nz)) return false;
+    } else if (h->zsolver != 0 || (!zsolve_supported_f64(h->g.nz) && !zsolve_long_supported_f64(h->g.nz))) {
+        return false;
+    }
     const int ly = line_lines_any<double>(h->g.ny, h->g.kind[1], 1);
     return ly > 0 && zsolve_cpb<double>() % ly == 0;
 }
@@ -427,9 +434,10 @@ int ensure_ztiles(pp_solver *h)
 }
 
 // Periodic z solve of the field in place: the one-pass kernel for lengths with a compiled
-// complex plan, else real z-line transforms (the columns of a [nz][ny*nx] array: R2HC,
+// plan, else real z-line transforms (the columns of a [nz][ny*nx] array: R2HC,
 // divide, HC2R).  f32: the mixed form's FP32 work field, singular column written as zeros.
-int run_zperiodic(pp_solver *h, void *data, bool f32)
+// tile_rows: data holds z tiles of that many rows (0: in place).
+int run_zperiodic(pp_solver *h, void *data, bool f32, int tile_rows)
 {
     hipStream_t s = h->stream;
     ZPerArgs zp{};
@@ -437,11 +445,13 @@ int run_zperiodic(pp_solver *h, void *data, bool f32)
     zp.SX = h->g.nx;
     zp.SY = h->g.ny;
     zp.nz = h->g.nz;
+    zp.tile_rows = tile_rows;
     zp.lamx = h->d_lamx;
     zp.lamy = h->d_lamy;
     zp.Cx = (h->g.dxyz[2] / h->g.dxyz[0]) * (h->g.dxyz[2] / h->g.dxyz[0]);
     zp.Cy = (h->g.dxyz[2] / h->g.dxyz[1]) * (h->g.dxyz[2] / h->g.dxyz[1]);
     zp.tw = h->d_ztw;
+    zp.A = h->d_zA;
     zp.c2 = h->d_zc2;
     zp.pinned_zero = f32 ? 1 : 0;
     if (zperiodic_supported(h->g.nz)) {
@@ -525,9 +535,15 @@ int ensure_zthomas(pp_solver *h)
 int run_fp64_stages(pp_solver *h, const double *rhs, double *field)
 {
     hipStream_t s = h->stream;
-    const bool zt = use_ztiles(h);
+    bool zt = use_ztiles(h);
     int rc;
-    if (zt && (rc = ensure_ztiles(h))) return rc;
+    if (zt && (rc = ensure_ztiles(h))) {
+        if (!h->g.zper || rc != PP_ALLOCATION_FAIL) return rc;
+        // periodic z needs no second field: in place where there is no room for one
+        (void)hipGetLastError();
+        h->no_zt = true;
+        zt = false;
+    }
     const bool zth = zthomas_on(h);
     if (zth && (rc = ensure_zthomas(h))) return rc;
     double *zdata = zt ? h->d_zt : field;
@@ -571,9 +587,15 @@ int run_fp64_stages(pp_solver *h, const double *rhs, double *field)
         z.zhi_dirichlet = h->g.zhi_d;
         z.zero_mode = h->zero_mode;
         if (h->g.zper) {
-            if ((rc = run_zperiodic(h, field, false))) return rc;
-            if (h->zsing_x >= 0)
-                PP_HIP_CHECK(launch_smt_v1(field, h->g.nx, h->g.ny, h->g.nz, h->zsing_x, h->zsing_y, h->zsing_eig, s));
+            if ((rc = run_zperiodic(h, zdata, false, zt ? ztile_rows(h->g.nz) : 0))) return rc;
+            if (h->zsing_x >= 0) {
+                SmtItem it = {(long)h->zsing_y * h->g.nx + h->zsing_x, (long)h->g.nx * h->g.ny, h->g.nz, h->zsing_eig};
+                if (zt) {
+                    it.offset = ((long)(h->zsing_x / 16) * h->g.ny + h->zsing_y) * ztile_rows(h->g.nz) * 16 + h->zsing_x % 16;
+                    it.stride = 16;
+                }
+                PP_HIP_CHECK(launch_smt_v1(zdata, it, s));
+            }
         } else {
             // nearly singular columns left to the reference's serial Thomas (PP_OPT_ZTHOMAS_TAU)
             if (zth) z.tau = h->zthomas_tau;
@@ -906,7 +928,7 @@ int mixed_inner(pp_solver *h)
     if ((rc = mark(h))) return rc;
     if (h->g.zper) {
         // periodic z: FP64 arithmetic on the FP32 field, singular column zeroed
-        if ((rc = run_zperiodic(h, h->d_w, true))) return rc;
+        if ((rc = run_zperiodic(h, h->d_w, true, 0))) return rc;
         if ((rc = mark(h))) return rc;
     } else {
         ZArgs z = z_args(h, zdata);

@@ -3,7 +3,7 @@
 // The reference solves each (kx, ky) column's cyclic tridiagonal system (diagonal eig, unit
 // off-diagonals, wrap-around corners) by Sherman-Morrison on top of two Thomas sweeps
 // (shermanMorrisonThomas, src/triDiag.cpp:1961-2108).  That system is circulant, so here a
-// block diagonalises it exactly instead: complex FFT of the column along z, division of mode
+// block diagonalises it exactly instead: real FFT of the column along z, division of mode
 // k by eig + 2 cos(2 pi k / nz), inverse FFT -- one read and one write of the column, with the
 // Stockham passes of the line transforms (pp_fft.h) running on z-columns.
 //
@@ -14,7 +14,7 @@
 // solves that column from FP64 plane sums instead (k_mode00, pp_mixed.hip) and has it
 // written as zeros here.
 //
-// Lengths without a compiled complex plan take three passes instead of one: real z-line
+// Lengths without a compiled plan take three passes instead of one: real z-line
 // transforms of any length (the line kernels) around a division kernel (k_zper_divide).
 //
 // Storage is FP64 (FP64 form) or FP32 (the mixed form's work field); the arithmetic of the
@@ -30,12 +30,24 @@
 
 namespace pp {
 
-// ZPerArgs (pp_launch.h): data [nz][SY][SX] in place; tw = exp(-2 pi i e / nz), e < nz,
-// interleaved; c2 = 2 cos(2 pi k / nz), k < nz.  S is the storage type: the FP64 form and the
-// mixed form's FP32 work field both compute in FP64 (the transform and the division by the
-// mode's eigenvalue), so near-singular columns need no separate treatment in either form.
+// ZPerArgs (pp_launch.h): data [nz][SY][SX] in place, nz = 2 M; tw = exp(-2 pi i e / M), e < M, and
+// A = exp(-2 pi i k / nz), k <= M, interleaved; c2 = 2 cos(2 pi k / nz), k < nz.  S is the storage
+// type: the FP64 form and the mixed form's FP32 work field both compute in FP64 (the transform and
+// the division by the mode's eigenvalue), so near-singular columns need no separate treatment in
+// either form.
+//
+// A real column is one complex line of half its length, z_m = x_2m + i x_2m+1, whose rows arrive and
+// leave in the FFT's own register layout (no LDS scatter).  With Z its FFT, Zc = conj Z_{M-k},
+// P = (Z_k + Zc) / 2, R = (Z_k - Zc) / 2, w = exp(-2 pi i k / nz) and s_k = 1 / (nz (eig + c2_k)),
+// splitting Z into the column's spectrum, dividing and packing it again collapses to
+//     Z'_k = (s_k + s_{M-k}) Z_k + i (s_k - s_{M-k}) (conj(w) P - w R),
+// one mirrored LDS read between the two FFTs (256^3: 86 us with full-length complex lines -> 56 us).
+// At least four waves per SIMD (128 registers) where a thread holds 8 elements
+template <int M, int T, int LINES>
+constexpr int zper_min_waves() { return M / T == 8 ? 4 : 2; }
+
 template <typename S, int M, int T, int LINES>
-__global__ void __launch_bounds__(T *LINES) k_zper(ZPerArgs a)
+__global__ void __launch_bounds__(T *LINES, (zper_min_waves<M, T, LINES>())) k_zper(ZPerArgs a)
 {
     using R = double;
     constexpr int E = M / T;
@@ -64,43 +76,71 @@ __global__ void __launch_bounds__(T *LINES) k_zper(ZPerArgs a)
     const int sx0 = bx * LINES + l;
     const bool valid = sx0 < a.SX;
     const int sx = valid ? sx0 : a.SX - 1;
-    const long base = (long)sy * a.SX + sx;
-    const long stride = (long)a.SX * a.SY;
+    // row 2 (t + T m) + h of the lane's column: a block-uniform pointer per (m, h) and one 32-bit
+    // byte offset per lane (2 T planes of at most 1024^2 doubles: below 2^31)
+    const bool tiled = a.tile_rows > 0;
+    const long stride = tiled ? 16 : (long)a.SX * a.SY;
+    const int c0 = bx * LINES;
+    S *const col0 = data + (tiled ? ((long)(c0 / 16) * a.SY + sy) * a.tile_rows * 16 + c0 % 16 : (long)sy * a.SX + c0);
+    // (in place, columns past the grid read the last one; a tile's padding columns are its own)
+    const unsigned lane_bytes = (unsigned)((2L * t * stride + (tiled ? l : sx - c0)) * (long)sizeof(S));
+    auto at = [&](int m, int h) {
+        return reinterpret_cast<S *>(reinterpret_cast<char *>(col0 + (2L * T * m + h) * stride) + lane_bytes);
+    };
 
     cpx<R> v[E];
 #pragma unroll
-    for (int m = 0; m < E; m++) v[m] = {valid ? (R)data[base + (long)(t + T * m) * stride] : 0.0, 0.0};
+    for (int m = 0; m < E; m++) v[m] = {(R)*at(m, 0), (R)*at(m, 1)};
     FFTSeeds<R, M, T> fs;
     fs.load(t, a.tw);
+    c64 w = ld64(a.A, t);
+    const c64 wT = ld64(a.A, T);
     // eigenvalue of this (kx, ky) column, src/pencilDcmp.cpp:4393-4417, without contraction
-    const double eig = __dadd_rn(__dadd_rn(-2.0, __dmul_rn(a.lamx[sx], a.Cx)), __dmul_rn(a.lamy[sy], a.Cy));
+    double eig = __dadd_rn(__dadd_rn(-2.0, __dmul_rn(a.lamx[sx], a.Cx)), __dmul_rn(a.lamy[sy], a.Cy));
     const bool singular = fabs(eig + 2.) < 1.e-10;
 
     line_fft<R, M, T, -1>(v, L, t, fs);
 #pragma unroll
+    for (int m = 0; m < E; m++) L[padc(t + T * m)] = v[m];
+    __syncthreads();
+    // (the factors of a mode are formed where they are used: hoisted above the FFT, which the
+    // compiler does for all modes at once unless held back, they cost a wave per SIMD)
+    int kt = t;
+    asm volatile("" : "+v"(eig), "+v"(kt));
+#pragma unroll
     for (int m = 0; m < E; m++) {
-        const int k = t + T * m;
-        const double den = (eig + a.c2[k]) * (double)M;
-        const double s = singular ? 0.0 : 1.0 / den;
-        v[m] = c_scale(v[m], s);
+        const int k = kt + T * m;
+        const cpx<R> Zk = v[m], Zc = c_conj(L[padc(k == 0 ? 0 : M - k)]);
+        const cpx<R> wk = to_c<R>(w);
+        w = m64(w, wT);
+        const double c2 = a.c2[k];  // mode M - k has -c2
+        const double s0 = singular ? 0.0 : rcp_nr((eig + c2) * (double)(2 * M));
+        const double s1 = singular ? 0.0 : rcp_nr((eig - c2) * (double)(2 * M));
+        const cpx<R> P = c_scale(c_add(Zk, Zc), 0.5), Q = c_scale(c_sub(Zk, Zc), 0.5);
+        const cpx<R> q = c_scale(c_sub(c_mulc(P, wk), c_mul(Q, wk)), s0 - s1);
+        v[m] = {(s0 + s1) * Zk.x - q.y, (s0 + s1) * Zk.y + q.x};
+        if (m % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     }
+    __syncthreads();
     line_fft<R, M, T, +1>(v, L, t, fs);
     // the singular column: zeros (pinned_zero, v is zero) or left for k_smt_v1
     if (valid && (!singular || a.pinned_zero)) {
 #pragma unroll
-        for (int m = 0; m < E; m++) data[base + (long)(t + T * m) * stride] = (S)v[m].x;
+        for (int m = 0; m < E; m++) {
+            *at(m, 0) = (S)v[m].x;
+            *at(m, 1) = (S)v[m].y;
+        }
     }
 }
 
-// the reference's singular periodic branch on one column (sx, sy), FP64: by scans where the
+// the reference's singular periodic branch on one column, FP64: by scans where the
 // diagonal is exactly -2 (mode (0, 0) of periodic and Neumann axes); a diagonal only within 1e-10 of
 // it (cells 1e5 times thinner in z) takes the reference's sweeps, whose factors carry it
-__device__ void smt_v1_body(double *data, int SX, int SY, int nz, int sx, int sy, double diag)
+__device__ void smt_v1_body(double *data, long stride, int nz, double diag)
 {
     extern __shared__ double sv[];
     double *rh = sv, *rh1 = sv + nz, *tmp = sv + 2 * nz;
-    const long stride = (long)SX * SY, base = (long)sy * SX + sx;
-    for (int i = threadIdx.x; i < nz; i += blockDim.x) rh[i] = data[base + i * stride];
+    for (int i = threadIdx.x; i < nz; i += blockDim.x) rh[i] = data[i * stride];
     __syncthreads();
     if (diag == -2.0 && nz >= 3) {
         if (threadIdx.x < 64) singular_periodic_column(rh, nz, (rh[0] + rh[nz - 1]) * 0.5, threadIdx.x);
@@ -142,43 +182,38 @@ __device__ void smt_v1_body(double *data, int SX, int SY, int nz, int sx, int sy
         for (int i = 0; i < N; i++) rh[i] -= fact * rh1[i];
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < nz; i += blockDim.x) data[base + i * stride] = rh[i];
+    for (int i = threadIdx.x; i < nz; i += blockDim.x) data[i * stride] = rh[i];
 }
 
-__global__ void k_smt_v1(double *data, int SX, int SY, int nz, int sx, int sy, double diag)
-{
-    smt_v1_body(data, SX, SY, nz, sx, sy, diag);
-}
+__global__ void k_smt_v1(double *data, SmtItem it) { smt_v1_body(data + it.offset, it.stride, it.nz, it.diag); }
 
 // batched: block b solves the singular column of items[b]
 __global__ void k_smt_v1_batch(double *data, const SmtItem *items)
 {
     const SmtItem it = items[blockIdx.x];
-    smt_v1_body(data + it.offset, it.SX, it.SY, it.nz, it.sx, it.sy, it.diag);
+    smt_v1_body(data + it.offset, it.stride, it.nz, it.diag);
 }
 
+// columns per block: 16 (128-byte FP64 rows) while the slices fit 80 KB, 8 for longer lines, as
+// the y transforms on the field in place
 template <int M>
 constexpr int zper_lines_m()
 {
-    // 16 columns (128-byte FP64 rows) while the block's line slices fit in 80 KB, else 8
-    return (16 * line_slots<M>() * 16 <= 80 * 1024) ? 16 : 8;
+    constexpr int L = line_lines<double, M, 1>();
+    return line_threads(M, 1) >= 64 && L > 8 ? 8 : L;
 }
 
 // grid: column blocks x SY (one solve), or nitems blocks (batched, a.items set)
 template <typename S, int M>
 static hipError_t launch_zper_m(const ZPerArgs &a, int nitems, hipStream_t s)
 {
-    constexpr int T = line_threads(M, 0);
+    constexpr int T = line_threads(M, 1);
     constexpr int LINES = zper_lines_m<M>();
     const size_t lds = (size_t)LINES * line_slots<M>() * sizeof(cpx<double>);
     auto kern = k_zper<S, M, T, LINES>;
     if (lds > 64 * 1024) {
-        static bool attr = false;
-        if (!attr) {
-            hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-            attr = true;
-        }
+        hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
     }
     const dim3 grid = a.items ? dim3((unsigned)nitems) : dim3((unsigned)((a.SX + LINES - 1) / LINES), (unsigned)a.SY);
     if (a.items && nitems == 0) return hipSuccess;
@@ -186,11 +221,11 @@ static hipError_t launch_zper_m(const ZPerArgs &a, int nitems, hipStream_t s)
     return hipGetLastError();
 }
 
-bool zperiodic_supported(int nz) { return nz >= 8 && line_threads(nz, 0) > 0; }
+bool zperiodic_supported(int nz) { return nz >= 8 && line_compiled(nz); }
 
 int zper_lines(int nz)
 {
-    switch (nz) {
+    switch (nz / 2) {
 #define PPM(m) \
     case m: return zper_lines_m<m>();
         PP_FFT_LENGTHS(PPM)
@@ -237,7 +272,7 @@ hipError_t launch_zper_divide_f32(const ZPerArgs &a, hipStream_t s) { return lau
 template <typename S>
 static hipError_t launch_zperiodic_s(const ZPerArgs &a, int nitems, hipStream_t s)
 {
-    switch (a.nz) {
+    switch (line_compiled(a.nz) ? a.nz / 2 : 0) {
 #define PPM(m) \
     case m: return launch_zper_m<S, m>(a, nitems, s);
         PP_FFT_LENGTHS(PPM)
@@ -260,10 +295,9 @@ hipError_t launch_zperiodic_f32_batch(const ZPerArgs &a, int nitems, hipStream_t
     return a.items ? launch_zperiodic_s<float>(a, nitems, s) : hipErrorInvalidValue;
 }
 
-hipError_t launch_smt_v1(double *data, int SX, int SY, int nz, int sx, int sy, double diag, hipStream_t s)
+hipError_t launch_smt_v1(double *data, const SmtItem &it, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_smt_v1, dim3(1), dim3(256), 3 * (size_t)nz * sizeof(double), s, data, SX, SY, nz, sx, sy,
-                       diag);
+    hipLaunchKernelGGL(k_smt_v1, dim3(1), dim3(256), 3 * (size_t)it.nz * sizeof(double), s, data, it);
     return hipGetLastError();
 }
 
