@@ -297,7 +297,8 @@ int pp_batch_destroy(pp_batch b);
 int pp_batch_add(pp_batch b, int nx, int ny, int nz, const char *bc, const double *X, int *id);
 int pp_batch_finalize(pp_batch b);
 int pp_batch_count(pp_batch b, int *members, long long *points);
-/* launches per stage: x, y, z (one per shape class) */
+/* shape classes per stage: x, y, z.  A stage runs as one launch per class; FP64 members with
+ * small planes (at most 64 x 64 points) share launches for both x and y, whatever their classes */
 int pp_batch_launch_count(pp_batch b, int *per_stage3);
 /* device pointers of a member's right-hand side and solution (nx*ny*nz doubles each) */
 int pp_batch_field(pp_batch b, int id, double **d_rhs);

@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <cstring>
 #include <new>
+#include <set>
 #include <tuple>
 #include <vector>
 
@@ -58,19 +59,51 @@ int put(T *dst, const std::vector<T> &v, hipStream_t s)
 TableCache::~TableCache()
 {
     for (auto &kv : t_)
-        for (double *p : {kv.second.tw, kv.second.A, kv.second.B, kv.second.C, kv.second.D, kv.second.mm})
+        for (double *p : {kv.second.tw, kv.second.A, kv.second.B, kv.second.C, kv.second.D})
             if (p) (void)hipFree(p);
+    for (auto &kv : m_)
+        if (kv.second.base) (void)hipFree(kv.second.base);
+}
+
+int TableCache::get_mm(int N, int kind, const double *&mm, const double *&mmi)
+{
+    Matrices &e = m_[{N, mm_family(kind)}];
+    if (!e.base) {
+        std::vector<double> oct(mm_octant_size(N));
+        fill_mm_octant(N, oct.data());
+        const size_t o = (oct.size() + 31) / 32 * 32;
+        if (hipMalloc((void **)&e.base, (o + mm_tables_size(N, kind)) * sizeof(double)) != hipSuccess) {
+            e.base = nullptr;
+            return PP_ALLOCATION_FAIL;
+        }
+        // finished before the first batch that reads them, on whichever stream that runs
+        if (hipMemcpy(e.base, oct.data(), oct.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
+            launch_mm_tables(e.base + o, e.base, N, kind, nullptr) != hipSuccess ||
+            hipStreamSynchronize(nullptr) != hipSuccess) {
+            (void)hipFree(e.base);
+            e.base = nullptr;
+            return PP_HIP_ERROR;
+        }
+        e.mm = e.base + o;
+        e.mmi = e.mm + mm_inverse_offset(N, kind);
+    }
+    mm = e.mm;
+    mmi = e.mmi;
+    return PP_SUCCESS;
 }
 
 int TableCache::get(int N, int kind, int axis, AxisDev &out)
 {
-    const bool dense = kind >= 0 && mm_serves(N, kind, axis);
-    const std::pair<int, int> key = {N, dense ? mm_family(kind) : -1};
-    auto it = t_.find(key);
+    if (kind >= 0 && mm_serves(N, kind, axis)) {
+        out = AxisDev{};
+        return get_mm(N, kind, out.mm, out.mmi);
+    }
+    auto it = t_.find(N);
     if (it != t_.end()) {
         out = it->second;
         return PP_SUCCESS;
     }
+    const AxisTables &t = axis_tables_cached(N);
     AxisDev d;
     auto up = [](double **dst, const std::vector<double> &v) -> int {
         if (hipMalloc((void **)dst, v.size() * sizeof(double)) != hipSuccess) return PP_ALLOCATION_FAIL;
@@ -79,27 +112,10 @@ int TableCache::get(int N, int kind, int axis, AxisDev &out)
         return PP_SUCCESS;
     };
     int rc;
-    if (dense) {
-        std::vector<double> oct(mm_octant_size(N));
-        fill_mm_octant(N, oct.data());
-        if ((rc = up(&d.A, oct))) return rc;
-        if (hipMalloc((void **)&d.mm, mm_tables_size(N, kind) * sizeof(double)) != hipSuccess) {
-            (void)hipFree(d.A);
-            return PP_ALLOCATION_FAIL;
-        }
-        d.mmi = d.mm + mm_inverse_offset(N, kind);
-        t_[key] = d;
-        // finished before the first batch that reads them, on whichever stream that runs
-        PPB_CHECK(launch_mm_tables(d.mm, d.A, N, kind, nullptr));
-        PPB_CHECK(hipStreamSynchronize(nullptr));
-        out = d;
-        return PP_SUCCESS;
-    }
-    const AxisTables &t = axis_tables_cached(N);
     if ((rc = up(&d.tw, t.tw)) || (rc = up(&d.A, t.A)) || (rc = up(&d.B, t.B)) || (rc = up(&d.C, t.C)) ||
         (rc = up(&d.D, t.D)))
         return rc;
-    t_[key] = d;
+    t_[N] = d;
     out = d;
     return PP_SUCCESS;
 }
@@ -152,6 +168,7 @@ int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
     // dense-product classes: launch shape from the class's units of 16 lines / columns
     std::map<std::pair<int, int>, long> units;
     for (const BatchMember &m : mem) {
+        if (m.plane) continue;
         const int N = axis == 0 ? m.g.nx : m.g.ny;
         if (mm_serves(N, m.g.kind[axis], axis))
             units[{N, m.g.kind[axis]}] += axis == 0 ? ((long)m.g.ny * m.g.nz + 15) / 16 : (long)((m.g.nx + 15) / 16) * m.g.nz;
@@ -159,6 +176,7 @@ int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
     std::map<std::pair<int, int>, MmPlan> plans;
     for (const auto &kv : units) plans[kv.first] = mm_plan(kv.first.first, kv.first.second, axis, kv.second);
     for (int m = 0; m < (int)mem.size(); m++) {
+        if (mem[m].plane) continue;
         const SolveSetup &g = mem[m].g;
         const int N = axis == 0 ? g.nx : g.ny;
         const auto pl = plans.find({N, g.kind[axis]});
@@ -191,7 +209,7 @@ int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
             const int la = line_block_lines_alt(c.key, 0);
             for (int m = 0; m < (int)mem.size(); m++) {
                 const SolveSetup &g = mem[m].g;
-                if (g.nx != c.key || g.kind[0] != c.kind) continue;
+                if (mem[m].plane || g.nx != c.key || g.kind[0] != c.kind) continue;
                 const long nl = (long)g.ny * g.nz;
                 for (long bx = 0; bx < (nl + la - 1) / la; bx++) c.li_alt.push_back({m, (int)bx, 0});
             }
@@ -446,11 +464,37 @@ int BatchCore::plan()
             }
         if ((rc = plan_mixed())) return rc;
     } else {
+        // small planes: both axes in one launch over the planes of every such member whose block
+        // has as many waves (the line kernels where their shape is forced, as in the handle)
+        lp_.clear();
+        HostClass by_waves[4];
+        for (int i = 0; i < (int)mem.size(); i++) {
+            const SolveSetup &g = mem[i].g;
+            mem[i].plane = force_var < 0 && mm_plane(g.nx, g.ny, g.kind[0], g.kind[1]);
+            if (!mem[i].plane) continue;
+            const int jobs = plane_jobs(g.nx, g.ny, g.kind[0], g.kind[1]);
+            const int q = jobs > 4 ? 3 : jobs > 2 ? 2 : jobs > 1 ? 1 : 0;
+            HostClass &c = by_waves[q];
+            c.key = 1 << q;
+            for (int z = 0; z < g.nz; z++) c.li.push_back({i, z, 0});
+            c.lds = std::max(c.lds, plane_lds(g.nx, g.ny, g.kind[0], g.kind[1]));
+        }
+        for (HostClass &c : by_waves) {
+            c.nitems = (int)c.li.size();
+            if (c.nitems) lp_.push_back(std::move(c));
+        }
+        ps_.assign(!lp_.empty() ? mem.size() : 0, PlaneSolve{});
         if ((rc = plan_lines<double>(0, lx_)) || (rc = plan_lines<double>(1, ly_))) return rc;
     }
     plan_z();
-    launches[0] = (int)lx_.size();
-    launches[1] = (int)ly_.size();
+    // shape classes per stage: the plane members' count too, though they share one launch
+    for (int a = 0; a < 2; a++) {
+        std::set<std::pair<int, int>> cls;
+        for (const HostClass &c : a == 0 ? lx_ : ly_) cls.insert({c.key, c.kind});
+        for (const BatchMember &m : mem)
+            if (m.plane) cls.insert({a == 0 ? m.g.nx : m.g.ny, m.g.kind[a]});
+        launches[a] = (int)cls.size();
+    }
     launches[2] = (int)(lz_.size() + lzp_.size() + 3 * zpl_.size() + zlong_.size() + (smt_.empty() ? 0 : 1));
     ls_.assign(mem.size(), LineSolve{});
     zs_.assign(mem.size(), ZSolve{});
@@ -472,6 +516,8 @@ int BatchCore::plan()
             h.off = take(c, h.li.size() * sizeof(LineItem));
             if (!h.li_alt.empty()) h.off_alt = take(c, h.li_alt.size() * sizeof(LineItem));
         }
+    for (HostClass &h : lp_) h.off = take(c, h.li.size() * sizeof(LineItem));
+    if (!lp_.empty()) o_ps_ = take(c, ps_.size() * sizeof(PlaneSolve));
     for (HostClass &h : lz_) h.off = take(c, h.zi.size() * sizeof(ZItem));
     for (HostClass &h : lzp_) h.off = take(c, h.zi.size() * sizeof(ZItem));
     o_zc2_ = take(c, zc2_.size() * sizeof(double));
@@ -512,6 +558,8 @@ int BatchCore::bind(char *base, TableCache *tc)
             h.d_items = base + h.off;
             h.d_items_alt = h.li_alt.empty() ? nullptr : base + h.off_alt;
         }
+    for (HostClass &h : lp_) h.d_items = base + h.off;
+    d_ps_ = !lp_.empty() ? (PlaneSolve *)(base + o_ps_) : nullptr;
     d_zc2_ = (double *)(base + o_zc2_);
     d_zth_ = (ZThomasItem *)(base + o_zth_);
     d_zth_tab_ = (double *)(base + o_zth_tab_);
@@ -561,6 +609,11 @@ int BatchCore::bind(char *base, TableCache *tc)
         l.plane_off = m.plane_off;
         l.toffset = m.toff;
         l.tnz = (precision == 0 && m.toff < 0) ? 0 : (g.nz + 15) / 16 * 16;
+        for (int a = 0; a < 2 && m.plane; a++) {
+            PlaneSolve &p = ps_[i];
+            p.kind[a] = g.kind[a];
+            if ((rc = tc->get_mm(a == 0 ? g.nx : g.ny, g.kind[a], p.mm[a], p.mmi[a]))) return rc;
+        }
         ZSolve &z = zs_[i];
         z.offset = (precision == 0 && m.toff >= 0) ? m.toff : m.offset;  // FP64 solves the z tiles
         z.SX = g.nx;
@@ -608,6 +661,9 @@ int BatchCore::upload(hipStream_t s)
     int rc;
     // tile padding (rows from nz, columns from nx) is never written by the transforms
     if (precision == 0 && ntiles_) PPB_CHECK(hipMemsetAsync(d_tiles, 0, (size_t)ntiles_ * sizeof(double), s));
+    for (HostClass &h : lp_)
+        if ((rc = put((LineItem *)h.d_items, h.li, s))) return rc;
+    if (!lp_.empty() && (rc = put(d_ps_, ps_, s))) return rc;
     if ((rc = put(d_lam_, lam_, s)) || (rc = put(d_dtab_, dtab_, s)) || (rc = put(d_ls_, ls_, s)) ||
         (rc = put(d_zs_, zs_, s)))
         return rc;
@@ -848,9 +904,31 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
     return PP_SUCCESS;
 }
 
+// the plane launches of the members whose planes are small: forward (right-hand sides to z tiles) or
+// inverse (z tiles to solutions)
+int BatchCore::run_planes(hipStream_t s, int fwd)
+{
+    LineArgs x{}, y{};
+    x.solves = y.solves = d_ls_;
+    x.in = fwd ? d_rhs : d_sol;
+    x.out = d_sol;
+    x.bflags = fwd ? BF_RHS : BF_SCALE;
+    y.in = fwd ? d_sol : d_tiles;
+    y.out = fwd ? d_tiles : d_sol;
+    y.ztiled = fwd ? ZT_OUT : ZT_IN;
+    y.tile_w = zsolve_cpb<double>();
+    for (const HostClass &c : lp_) {
+        x.items = y.items = (const LineItem *)c.d_items;
+        x.nlines = c.nitems;
+        PPB_CHECK(launch_plane_mm(fwd, 0, 0, x, y, c.lds, s, d_ps_, c.key));
+    }
+    return PP_SUCCESS;
+}
+
 int BatchCore::run_fp64(hipStream_t s, Marks *mk)
 {
     int rc;
+    if ((rc = run_planes(s, 1))) return rc;
     if ((rc = run_line_stage(s, lx_, FORM_F64, 0, 1, d_rhs, d_sol, BF_RHS, nullptr, nullptr, 0))) return rc;
     if ((rc = mark(s, mk))) return rc;
     if ((rc = run_line_stage(s, ly_, FORM_F64, 1, 1, d_sol, d_tiles, 0, nullptr, nullptr, 0, ZT_OUT))) return rc;
@@ -860,6 +938,7 @@ int BatchCore::run_fp64(hipStream_t s, Marks *mk)
     if ((rc = run_line_stage(s, ly_, FORM_F64, 1, 0, d_tiles, d_sol, 0, nullptr, nullptr, 0, ZT_IN))) return rc;
     if ((rc = mark(s, mk))) return rc;
     if ((rc = run_line_stage(s, lx_, FORM_F64, 0, 0, d_sol, d_sol, BF_SCALE, nullptr, nullptr, 0))) return rc;
+    if ((rc = run_planes(s, 0))) return rc;
     return mark(s, mk);
 }
 

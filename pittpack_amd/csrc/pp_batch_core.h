@@ -16,6 +16,7 @@
 #include "pp_line.h"
 #include "pp_line_mm.h"
 #include "pp_mixed.h"
+#include "pp_plane_mm.h"
 #include "pp_setup.h"
 #include "pp_zsolve.h"
 
@@ -23,7 +24,7 @@ namespace pp {
 
 struct AxisDev {
     double *tw = nullptr, *A = nullptr, *B = nullptr, *C = nullptr, *D = nullptr;
-    double *mm = nullptr, *mmi = nullptr;  // dense-product matrices (one allocation, at mm)
+    const double *mm = nullptr, *mmi = nullptr;  // dense-product matrices
 };
 
 // FP64 tables per line length (and, dense products, symmetry family), resident on the device
@@ -33,9 +34,16 @@ class TableCache {
     ~TableCache();
     // tables of lines of length N along x (axis 0) or across it; kind -1: a compiled plan's
     int get(int N, int kind, int axis, AxisDev &out);
+    // dense-product matrices of (N, kind)
+    int get_mm(int N, int kind, const double *&mm, const double *&mmi);
 
   private:
-    std::map<std::pair<int, int>, AxisDev> t_;  // {length, family (dense products) or -1}
+    struct Matrices {
+        double *base = nullptr;  // octant table, then the matrices
+        const double *mm = nullptr, *mmi = nullptr;
+    };
+    std::map<int, AxisDev> t_;
+    std::map<std::pair<int, int>, Matrices> m_;  // {length, symmetry family}
 };
 
 // events recorded between the launches of one run (null ev: no timing)
@@ -51,6 +59,7 @@ struct BatchMember {
     long dtab_off = 0;
     bool pinned = false;  // mixed form: pinned (0,0) column solved in FP64 from plane sums
     long sums_off = 0, plane_off = 0, upart_off = 0;
+    bool plane = false;  // FP64: both transforms of a plane in one launch (pp_plane_mm.h)
     long toff = 0;  // FP64: offset of the member's z tiles in the tile arena (-1: none)
 };
 
@@ -108,6 +117,7 @@ class BatchCore {
         std::vector<LineItem> li_alt;
         size_t off_alt = 0;
         void *d_items_alt = nullptr;
+        size_t lds = 0;      // plane classes: of their largest plane
         bool fused = false;  // correction x classes: members whose residual runs in k_resx
     };
     int launch_class(hipStream_t s, const HostClass &c, int form, int axis, int fwd, const void *in, void *out,
@@ -121,6 +131,7 @@ class BatchCore {
                        void *out, int bflags, double *sums, const double *plane, int accumulate, int ztiled = 0,
                        const float *acc0 = nullptr, const float *acc1 = nullptr);
     int run_z_stage(hipStream_t s, bool f32);
+    int run_planes(hipStream_t s, int fwd);
     int run_fp64(hipStream_t s, Marks *mk);
     int mixed_inner(hipStream_t s, Marks *mk);
     int run_mixed(hipStream_t s, Marks *mk);
@@ -130,6 +141,10 @@ class BatchCore {
     std::vector<LineSolve> ls_;
     std::vector<ZSolve> zs_;
     std::vector<HostClass> lx_, ly_, lz_;
+    std::vector<HostClass> lp_;  // FP64: plane launches, items {member, z}, by waves a block
+    std::vector<PlaneSolve> ps_;
+    PlaneSolve *d_ps_ = nullptr;
+    size_t o_ps_ = 0;
     // mixed form: the corrections' x forward, each x class split into the members whose
     // residual is computed inside it (k_resx: ny a multiple of its lines per block, as the
     // single-solve handle decides) and the rest (residual kernel, then the FP32 transform)

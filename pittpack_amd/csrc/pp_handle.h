@@ -13,8 +13,9 @@ namespace pp {
 
 // device table pointers of one axis (twiddles and transform tables, pp_setup.h)
 struct DevTables {
+    double *base = nullptr;  // the allocation they sit in (null: tables of another owner)
     void *tw = nullptr, *A = nullptr, *B = nullptr, *C = nullptr, *D = nullptr;
-    double *mm = nullptr, *mmi = nullptr;  // dense-product matrices (one allocation, at mm)
+    double *mm = nullptr, *mmi = nullptr;  // dense-product matrices, forward and inverse
 };
 
 }  // namespace pp

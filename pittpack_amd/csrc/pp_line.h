@@ -171,7 +171,47 @@ __device__ __forceinline__ R &lr(cpx<R> *L, int p)
 
 // Block coordinates of a line launch.  y blocks narrower than a cache line keep the tiles of
 // one plane on one XCD; a batched launch (a0.items) takes its block's item and the item's
-// solve: per-solve fields, sizes and scalings are resolved into `a`.
+// solve: per-solve fields, sizes and scalings are resolved into `a` (line_item).
+template <typename TIn, typename TOut, int AX>
+__device__ __forceinline__ void line_item(const LineArgs &a0, LineArgs &a, int item, int &bx, int &by)
+{
+    const LineItem it = a0.items[item];
+    const LineSolve sv = a0.solves[it.solve];
+    if (a0.ztiled && sv.tnz == 0) {
+        // a solve without z tiles (periodic z) keeps its field in place: the y transform
+        // reads and writes the launch's other arena (tiled launches are FP64 -> FP64)
+        TOut *f = (a0.ztiled & ZT_OUT) ? reinterpret_cast<TOut *>(const_cast<void *>(a0.in))
+                                       : reinterpret_cast<TOut *>(a0.out);
+        a.in = f + sv.offset;
+        a.out = f + sv.offset;
+        a.ztiled = 0;
+    } else {
+        a.in = reinterpret_cast<const TIn *>(a0.in) + ((a0.ztiled & ZT_IN) ? sv.toffset : sv.offset);
+        a.out = reinterpret_cast<TOut *>(a0.out) + ((a0.ztiled & ZT_OUT) ? sv.toffset : sv.offset);
+    }
+    a.tnz = sv.tnz;
+    a.nx = sv.nx;
+    a.ny = sv.ny;
+    a.nz = sv.nz;
+    if constexpr (AX == 0) {
+        a.nlines = (long)sv.ny * sv.nz;
+    } else {
+        a.nlines = sv.nx;
+        a.ncols = sv.nx;
+        a.nplanes = sv.nz;
+    }
+    a.in_scale = (a0.bflags & BF_RHS) ? sv.dz : 1.0;
+    a.dmask = (a0.bflags & BF_RHS) ? sv.dmask : 0;
+    a.dtab = sv.dtab;
+    a.out_scale = (a0.bflags & BF_SCALE) ? sv.inv_scale : 1.0;
+    if (a0.line_sums) a.line_sums = a0.line_sums + sv.sums_off;
+    if (a0.plane_add) a.plane_add = a0.plane_add + sv.plane_off;
+    if (a0.acc0) a.acc0 = a0.acc0 + sv.offset;
+    if (a0.acc1) a.acc1 = a0.acc1 + sv.offset;
+    bx = it.bx;
+    by = it.by;
+}
+
 template <typename TIn, typename TOut, typename R, int LINES, int AX>
 __device__ __forceinline__ void line_block(const LineArgs &a0, LineArgs &a, int &bx, int &by)
 {
@@ -184,43 +224,7 @@ __device__ __forceinline__ void line_block(const LineArgs &a0, LineArgs &a, int 
             by = lin / gridDim.x;
         }
     }
-    if (a0.items) {
-        const LineItem it = a0.items[blockIdx.x];
-        const LineSolve sv = a0.solves[it.solve];
-        if (a0.ztiled && sv.tnz == 0) {
-            // a solve without z tiles (periodic z) keeps its field in place: the y transform
-            // reads and writes the launch's other arena (tiled launches are FP64 -> FP64)
-            TOut *f = (a0.ztiled & ZT_OUT) ? reinterpret_cast<TOut *>(const_cast<void *>(a0.in))
-                                           : reinterpret_cast<TOut *>(a0.out);
-            a.in = f + sv.offset;
-            a.out = f + sv.offset;
-            a.ztiled = 0;
-        } else {
-            a.in = reinterpret_cast<const TIn *>(a0.in) + ((a0.ztiled & ZT_IN) ? sv.toffset : sv.offset);
-            a.out = reinterpret_cast<TOut *>(a0.out) + ((a0.ztiled & ZT_OUT) ? sv.toffset : sv.offset);
-        }
-        a.tnz = sv.tnz;
-        a.nx = sv.nx;
-        a.ny = sv.ny;
-        a.nz = sv.nz;
-        if constexpr (AX == 0) {
-            a.nlines = (long)sv.ny * sv.nz;
-        } else {
-            a.nlines = sv.nx;
-            a.ncols = sv.nx;
-            a.nplanes = sv.nz;
-        }
-        a.in_scale = (a0.bflags & BF_RHS) ? sv.dz : 1.0;
-        a.dmask = (a0.bflags & BF_RHS) ? sv.dmask : 0;
-        a.dtab = sv.dtab;
-        a.out_scale = (a0.bflags & BF_SCALE) ? sv.inv_scale : 1.0;
-        if (a0.line_sums) a.line_sums = a0.line_sums + sv.sums_off;
-        if (a0.plane_add) a.plane_add = a0.plane_add + sv.plane_off;
-        if (a0.acc0) a.acc0 = a0.acc0 + sv.offset;
-        if (a0.acc1) a.acc1 = a0.acc1 + sv.offset;
-        bx = it.bx;
-        by = it.by;
-    }
+    if (a0.items) line_item<TIn, TOut, AX>(a0, a, blockIdx.x, bx, by);
 }
 
 // Where line l of block (bx, by) lives: element n at base + n * stride (tbase + n * tstride

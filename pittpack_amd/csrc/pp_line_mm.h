@@ -44,7 +44,7 @@
 namespace pp {
 
 // symmetry family of a kind: 0 DCT/DST-II/III (NN, DD), 1 DCT/DST-IV (ND, DN), 2 real DFT (PP)
-constexpr int mm_family(int kind) { return kind == KIND_PP ? 2 : (kind == KIND_NN || kind == KIND_DD) ? 0 : 1; }
+__host__ __device__ constexpr int mm_family(int kind) { return kind == KIND_PP ? 2 : (kind == KIND_NN || kind == KIND_DD) ? 0 : 1; }
 // length of one half's sum (rows of staged data) and its number of outputs
 __host__ __device__ constexpr int mm_depth(int N, int fam) { return fam == 2 ? N / 2 + 1 : fam == 0 ? (N + 1) / 2 : N; }
 __host__ __device__ constexpr int mm_rows(int N, int fam) { return fam == 2 ? N / 2 + 1 : (N + 1) / 2; }
@@ -142,22 +142,22 @@ __device__ __forceinline__ MmIn mm_in(int N, int m)
 }
 
 // Matrix products of one wave: PW units (`unit` doubles apart in LDS), row tile i of `mm`
-// ([e, o] x [D8][R16]).  The loop is software-pipelined by hand: matrix elements are loaded (as
+// ([e, o] x [D8][R16]); `stride` is a line's in LDS for x, a depth row's for y.  The loop is software-pipelined by hand: matrix elements are loaded (as
 // buffer loads: a scalar offset walks the matrix, no address arithmetic per load) two pairs of
 // steps ahead, staged values one pair ahead, so that the wait for L2 (some 500 cycles) and LDS lies
 // under the 64-cycle products of the pairs between.
 template <int AX, int FAM, int PW>
 __device__ __forceinline__ void mm_products(const double *mm, int D8, int R16, int i, const double *lds, int unit,
-                                            int xstride, int lane, mm_d4 (&e)[PW], mm_d4 (&o)[PW])
+                                            int stride, int lane, mm_d4 (&e)[PW], mm_d4 (&o)[PW])
 {
     typedef unsigned int u2 __attribute__((ext_vector_type(2)));
     const int r = lane >> 4, c = lane & 15;
     const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(mm), 0, 2 * D8 * R16 * 8, 0x00027000);
     const int vo = (r * R16 + 16 * i + c) * 8, half = D8 * R16 * 8, cs = 4 * R16 * 8;
     auto coef = [&](int so) { return __builtin_bit_cast(double, (u2)__builtin_amdgcn_raw_buffer_load_b64(rs, vo, so, 0)); };
-    const double *ld = lds + (AX == 0 ? c * xstride + r : r * 16 + c);
-    constexpr int DS = AX == 0 ? 4 : 64;                       // one step of depth 4
-    const int po = FAM == 1 ? 0 : (AX == 0 ? D8 : D8 * 16);    // the second part
+    const double *ld = lds + (AX == 0 ? c * stride + r : r * stride + c);
+    const int DS = AX == 0 ? 4 : 4 * stride;                       // one step of depth 4
+    const int po = FAM == 1 ? 0 : (AX == 0 ? D8 : D8 * stride);    // the second part
     mm_d4 acc[2][2][PW];
 #pragma unroll
     for (int q = 0; q < 2; q++)
@@ -417,7 +417,7 @@ __global__ void __launch_bounds__(1024) k_line_mm(LineArgs a0, int units)
         const int g = job / KT, i = job - g * KT;
         mm_d4 e[PW], o[PW];
         const int p0 = g * PW;
-        mm_products<AX, FAM, PW>(mm, D8, R16, i, lds + p0 * unit, unit, xs, lane, e, o);
+        mm_products<AX, FAM, PW>(mm, D8, R16, i, lds + p0 * unit, unit, AX == 0 ? xs : 16, lane, e, o);
 #pragma unroll
         for (int p = 0; p < PW; p++) {
             if constexpr (AX == 0) {

@@ -20,6 +20,7 @@
 #include "pittpack_hip.h"
 #include "pp_handle.h"
 #include "pp_launch.h"
+#include "pp_plane_mm.h"
 #include "pp_setup.h"
 
 namespace {
@@ -40,8 +41,9 @@ struct Resident {
     size_t tab[2][5] = {};  // offsets (doubles) of tw, A, B, C, D per axis
     size_t ztab[5] = {};    // periodic z without a compiled plan: real z-line tables
     size_t lamx = 0, lamy = 0, dtab = 0, ztw = 0, zA = 0, zc2 = 0;
-    // dense-product lines (x, y, periodic z): where their matrices are written (0: none)
-    size_t mm[3] = {};
+    // dense-product lines (x, y, periodic z): where their matrices are written (0: none) and
+    // their octant tables
+    size_t mm[3] = {}, oct[3] = {};
     int zsing_x = -1, zsing_y = -1;
     double zsing_eig = -2.0;
     size_t used = 0;  // doubles of scratch in use
@@ -58,6 +60,12 @@ bool same_key(const Resident &r, int nx, int ny, int nz, const char *bc, const d
            std::memcmp(r.bc, bc, 6) == 0 && std::memcmp(r.X, X, sizeof(r.X)) == 0;
 }
 
+// lines of axis a (0 x, 1 y) whose matrices the handle would have
+bool mm_lines(const SolveSetup &g, int a)
+{
+    return mm_serves(a == 0 ? g.nx : g.ny, g.kind[a], a) || mm_plane(g.nx, g.ny, g.kind[0], g.kind[1]);
+}
+
 // lay the tables of `g` out in g_host (offsets into r); false if they exceed kScratchDoubles.
 // dense: lines without a compiled plan take the dense products (their octant table here, room
 // for their matrices behind the copied part), else the chirp convolution
@@ -72,9 +80,9 @@ bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
     };
     const int n[2] = {g.nx, g.ny};
     for (int a = 0; a < 2; a++) {
-        if (dense && mm_serves(n[a], g.kind[a], a)) {
-            r.tab[a][1] = take(mm_octant_size(n[a]));
-            continue;
+        if (dense && mm_lines(g, a)) {
+            r.oct[a] = take(mm_octant_size(n[a]));
+            if (mm_serves(n[a], g.kind[a], a)) continue;
         }
         const AxisTableSizes z = axis_table_sizes(n[a]);
         for (int i = 0; i < 5; i++) r.tab[a][i] = take(z.n[i]);
@@ -90,7 +98,7 @@ bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
             r.ztw = take(zs.n[0]);
             r.zA = take(zs.n[1]);
         } else if (dense && mm_serves(g.nz, KIND_PP, 1)) {
-            r.ztab[1] = take(mm_octant_size(g.nz));
+            r.oct[2] = take(mm_octant_size(g.nz));
         } else {
             for (int i = 0; i < 5; i++) r.ztab[i] = take(zs.n[i]);
         }
@@ -100,14 +108,14 @@ bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
     // the matrices are written on the device, behind the part that is copied
     if (dense) {
         for (int a = 0; a < 2; a++)
-            if (mm_serves(n[a], g.kind[a], a)) r.mm[a] = take(mm_tables_size(n[a], g.kind[a]));
+            if (mm_lines(g, a)) r.mm[a] = take(mm_tables_size(n[a], g.kind[a]));
         if (g.zper && !zc && mm_serves(g.nz, KIND_PP, 1)) r.mm[2] = take(mm_tables_size(g.nz, KIND_PP));
     }
     if (o > kScratchDoubles) return false;
     std::memset(g_host, 0, r.used * sizeof(double));
     for (int a = 0; a < 2; a++) {
-        if (r.mm[a]) fill_mm_octant(n[a], g_host + r.tab[a][1]);
-        else
+        if (r.mm[a]) fill_mm_octant(n[a], g_host + r.oct[a]);
+        if (!r.mm[a] || !mm_serves(n[a], g.kind[a], a))
             fill_axis_tables(n[a], g_host + r.tab[a][0], g_host + r.tab[a][1], g_host + r.tab[a][2],
                              g_host + r.tab[a][3], g_host + r.tab[a][4]);
     }
@@ -121,7 +129,7 @@ bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
             static double unused[3][1024 + 2];
             fill_axis_tables(g.nz, g_host + r.ztw, g_host + r.zA, unused[0], unused[1], unused[2]);
         } else if (r.mm[2]) {
-            fill_mm_octant(g.nz, g_host + r.ztab[1]);
+            fill_mm_octant(g.nz, g_host + r.oct[2]);
         } else {
             fill_axis_tables(g.nz, g_host + r.ztab[0], g_host + r.ztab[1], g_host + r.ztab[2], g_host + r.ztab[3],
                              g_host + r.ztab[4]);
@@ -202,8 +210,7 @@ extern "C" int pp_solve_device_oop_noalloc(int nx, int ny, int nz, const char *b
                 return PP_HIP_ERROR;
             const int len[3] = {nx, ny, nz}, kind[3] = {g.kind[0], g.kind[1], KIND_PP};
             for (int a = 0; a < 3; a++) {
-                const double *oct = base + (a < 2 ? nr.tab[a][1] : nr.ztab[1]);
-                if (nr.mm[a] && launch_mm_tables(base + nr.mm[a], oct, len[a], kind[a], s) != hipSuccess)
+                if (nr.mm[a] && launch_mm_tables(base + nr.mm[a], base + nr.oct[a], len[a], kind[a], s) != hipSuccess)
                     return PP_HIP_ERROR;
             }
             if (hipStreamSynchronize(s) != hipSuccess) return PP_HIP_ERROR;

@@ -4,6 +4,7 @@
 
 #include <cmath>
 #include <cstdio>
+#include <algorithm>
 #include <array>
 #include <cstring>
 #include <map>
@@ -17,6 +18,7 @@
 #include "pp_line.h"
 #include "pp_line_bs.h"
 #include "pp_line_mm.h"
+#include "pp_plane_mm.h"
 #include "pp_launch.h"
 #include "pp_mixed.h"
 #include "pp_resx.h"
@@ -72,7 +74,7 @@ extern template hipError_t launch_line_mm_kind<KIND_DN>(int, int, int, const Lin
 // pp_line_bs_<kind>.hip for the rest)
 hipError_t launch_line(int form, int kind, int N, int AX, int FWD, const LineArgs &a0, hipStream_t s)
 {
-    if (a0.mm) {
+    if (a0.mm && mm_serves(N, kind, AX)) {
         LineArgs a = a0;
         a.n = N;
         switch (kind) {
@@ -247,12 +249,8 @@ void free_tables(pp_solver *h)
 {
     free_zthomas(h);
     for (DevTables *t : {&h->tab64[0], &h->tab64[1], &h->tabz}) {
-        for (void **p : {&t->tw, &t->A, &t->B, &t->C, &t->D}) {
-            if (*p) (void)hipFree(*p);
-            *p = nullptr;
-        }
-        if (t->mm) (void)hipFree(t->mm);
-        t->mm = t->mmi = nullptr;
+        if (t->base) (void)hipFree(t->base);
+        *t = DevTables{};
     }
     for (double **p : {&h->d_lamx, &h->d_lamy, &h->d_dtab, &h->d_ztw, &h->d_zA, &h->d_zc2}) {
         if (*p) (void)hipFree(*p);
@@ -268,27 +266,44 @@ int upload(void **dst, const std::vector<double> &v)
     return PP_SUCCESS;
 }
 
-// The tables of lines of length n and kind `kind` along x (axis 0) or across it: the dense products' matrices (their octant
-// table stays in A), or the Stockham / chirp convolution tables
-int upload_axis(pp_solver *h, int n, int kind, int axis, DevTables &d)
+// The tables of lines of length n and kind `kind` along x (axis 0) or across it, in one
+// allocation and one copy: the Stockham or chirp convolution tables, and (dense) the dense products'
+// matrices, written on the device from their octant table
+int upload_axis(pp_solver *h, int n, int kind, bool dense, bool lines, DevTables &d)
 {
-    int rc;
-    if (mm_serves(n, kind, axis)) {
-        std::vector<double> oct(mm_octant_size(n));
-        fill_mm_octant(n, oct.data());
-        if ((rc = upload(&d.A, oct))) return rc;
-        if (hipMalloc((void **)&d.mm, mm_tables_size(n, kind) * sizeof(double)) != hipSuccess) {
-            d.mm = nullptr;
-            return PP_ALLOCATION_FAIL;
+    std::vector<double> host;
+    size_t at[6] = {0, 0, 0, 0, 0, 0};
+    auto add = [&](size_t count, int i) {
+        at[i] = host.size();
+        host.resize(host.size() + (count + 31) / 32 * 32, 0.0);  // 256-byte aligned sections
+    };
+    if (lines) {
+        const AxisTables &t = axis_tables_cached(n);
+        const std::vector<double> *v[5] = {&t.tw, &t.A, &t.B, &t.C, &t.D};
+        for (int i = 0; i < 5; i++) {
+            add(v[i]->size(), i);
+            std::copy(v[i]->begin(), v[i]->end(), host.begin() + at[i]);
         }
-        d.mmi = d.mm + mm_inverse_offset(n, kind);
-        PP_HIP_CHECK(launch_mm_tables(d.mm, (const double *)d.A, n, kind, h->stream));
-        return PP_SUCCESS;
     }
-    const AxisTables &t = axis_tables_cached(n);
-    if ((rc = upload(&d.tw, t.tw)) || (rc = upload(&d.A, t.A)) || (rc = upload(&d.B, t.B)) ||
-        (rc = upload(&d.C, t.C)) || (rc = upload(&d.D, t.D)))
-        return rc;
+    if (dense) {
+        add(mm_octant_size(n), 5);
+        fill_mm_octant(n, host.data() + at[5]);
+    }
+    const size_t mm = dense ? mm_tables_size(n, kind) : 0;
+    if (hipMalloc((void **)&d.base, (host.size() + mm) * sizeof(double)) != hipSuccess) {
+        d.base = nullptr;
+        return PP_ALLOCATION_FAIL;
+    }
+    PP_HIP_CHECK(hipMemcpy(d.base, host.data(), host.size() * sizeof(double), hipMemcpyHostToDevice));
+    if (lines) {
+        void **p[5] = {&d.tw, &d.A, &d.B, &d.C, &d.D};
+        for (int i = 0; i < 5; i++) *p[i] = d.base + at[i];
+    }
+    if (dense) {
+        d.mm = d.base + host.size();
+        d.mmi = d.mm + mm_inverse_offset(n, kind);
+        PP_HIP_CHECK(launch_mm_tables(d.mm, d.base + at[5], n, kind, h->stream));
+    }
     return PP_SUCCESS;
 }
 
@@ -299,8 +314,11 @@ int build_tables(pp_solver *h)
     free_tables(h);
     const int n[2] = {h->g.nx, h->g.ny};
     int rc;
-    for (int a = 0; a < 2; a++)
-        if ((rc = upload_axis(h, n[a], h->g.kind[a], a, h->tab64[a]))) return rc;
+    const bool plane = mm_plane(n[0], n[1], h->g.kind[0], h->g.kind[1]);
+    for (int a = 0; a < 2; a++) {
+        const bool mm = mm_serves(n[a], h->g.kind[a], a);
+        if ((rc = upload_axis(h, n[a], h->g.kind[a], mm || plane, !mm, h->tab64[a]))) return rc;
+    }
     const std::vector<double> lx = eig_factors(h->g, 0), ly = eig_factors(h->g, 1);
     if ((rc = upload((void **)&h->d_lamx, lx))) return rc;
     if ((rc = upload((void **)&h->d_lamy, ly))) return rc;
@@ -314,7 +332,8 @@ int build_tables(pp_solver *h)
             if ((rc = upload((void **)&h->d_ztw, zt.tw)) || (rc = upload((void **)&h->d_zA, zt.A))) return rc;
         } else {
             // real z-line transforms of length nz (R2HC / HC2R)
-            if ((rc = upload_axis(h, h->g.nz, KIND_PP, 1, h->tabz))) return rc;
+            const bool mm = mm_serves(h->g.nz, KIND_PP, 1);
+            if ((rc = upload_axis(h, h->g.nz, KIND_PP, mm, !mm, h->tabz))) return rc;
         }
         if ((rc = upload((void **)&h->d_zc2, zper_cos2(h->g.nz)))) return rc;
         const double Cx = (h->g.dxyz[2] / h->g.dxyz[0]) * (h->g.dxyz[2] / h->g.dxyz[0]);
@@ -531,6 +550,14 @@ int ensure_zthomas(pp_solver *h)
     return PP_SUCCESS;
 }
 
+// both transforms of a plane in one launch (pp_plane_mm.h); the line kernels where their shape is
+// forced
+bool use_plane(const pp_solver *h)
+{
+    return h->force_var < 0 && h->tab64[0].mm && h->tab64[1].mm &&
+           mm_plane(h->g.nx, h->g.ny, h->g.kind[0], h->g.kind[1]);
+}
+
 // the five stages, FP64: rhs -> field (x forward), then on field (and the z tiles)
 int run_fp64_stages(pp_solver *h, const double *rhs, double *field)
 {
@@ -548,26 +575,30 @@ int run_fp64_stages(pp_solver *h, const double *rhs, double *field)
     if (zth && (rc = ensure_zthomas(h))) return rc;
     double *zdata = zt ? h->d_zt : field;
     if ((rc = begin_timing(h))) return rc;
+    LineArgs xf = line_args(h, 0, field), yf = line_args(h, 1, field), yi = yf, xi = xf;
+    xf.in = rhs;
+    xf.in_scale = h->g.dxyz[2];
+    xf.dmask = h->g.dmask;
+    xf.variant = stage_var(h, 0, h->g.nx);
+    yf.out = zdata;
+    yf.variant = stage_var(h, 1, h->g.ny);
+    yi.in = zdata;
+    yi.variant = stage_var(h, 2, h->g.ny);
+    yf.tnz = yi.tnz = ztile_rows(h->g.nz);
+    yf.ztiled = zt ? ZT_OUT : 0;
+    yi.ztiled = zt ? ZT_IN : 0;
+    yf.tile_w = yi.tile_w = zt ? zsolve_cpb<double>() : 0;
+    xi.out_scale = 1. / (h->g.scale);
+    xi.variant = stage_var(h, 3, h->g.nx);
+    // small planes: both axes in one launch, whose time counts as the x stage's
+    const bool plane = use_plane(h);
+    const size_t plds = plane ? plane_lds(h->g.nx, h->g.ny, h->g.kind[0], h->g.kind[1]) : 0;
     // 1. forward x: rhs * dz^2, Dirichlet boundary term, x transform
-    {
-        LineArgs a = line_args(h, 0, field);
-        a.in = rhs;
-        a.in_scale = h->g.dxyz[2];
-        a.dmask = h->g.dmask;
-        a.variant = stage_var(h, 0, h->g.nx);
-        PP_HIP_CHECK(launch_line(FORM_F64, h->g.kind[0], h->g.nx, 0, 1, a, s));
-    }
+    if (plane) PP_HIP_CHECK(launch_plane_mm(1, h->g.kind[0], h->g.kind[1], xf, yf, plds, s));
+    else PP_HIP_CHECK(launch_line(FORM_F64, h->g.kind[0], h->g.nx, 0, 1, xf, s));
     if ((rc = mark(h))) return rc;
     // 2. forward y (into the z tiles)
-    {
-        LineArgs a = line_args(h, 1, field);
-        a.out = zdata;
-        a.ztiled = zt ? ZT_OUT : 0;
-        a.variant = stage_var(h, 1, h->g.ny);
-        a.tnz = ztile_rows(h->g.nz);
-        a.tile_w = zt ? zsolve_cpb<double>() : 0;
-        PP_HIP_CHECK(launch_line(FORM_F64, h->g.kind[1], h->g.ny, 1, 1, a, s));
-    }
+    if (!plane) PP_HIP_CHECK(launch_line(FORM_F64, h->g.kind[1], h->g.ny, 1, 1, yf, s));
     if ((rc = mark(h))) return rc;
     // 3. z solve
     {
@@ -611,23 +642,11 @@ int run_fp64_stages(pp_solver *h, const double *rhs, double *field)
     }
     if ((rc = mark(h))) return rc;
     // 4. inverse y (from the z tiles)
-    {
-        LineArgs a = line_args(h, 1, field);
-        a.in = zdata;
-        a.ztiled = zt ? ZT_IN : 0;
-        a.variant = stage_var(h, 2, h->g.ny);
-        a.tnz = ztile_rows(h->g.nz);
-        a.tile_w = zt ? zsolve_cpb<double>() : 0;
-        PP_HIP_CHECK(launch_line(FORM_F64, h->g.kind[1], h->g.ny, 1, 0, a, s));
-    }
+    if (!plane) PP_HIP_CHECK(launch_line(FORM_F64, h->g.kind[1], h->g.ny, 1, 0, yi, s));
     if ((rc = mark(h))) return rc;
     // 5. inverse x with the 1/(Nx*Ny) rescale fused
-    {
-        LineArgs a = line_args(h, 0, field);
-        a.out_scale = 1. / (h->g.scale);
-        a.variant = stage_var(h, 3, h->g.nx);
-        PP_HIP_CHECK(launch_line(FORM_F64, h->g.kind[0], h->g.nx, 0, 0, a, s));
-    }
+    if (plane) PP_HIP_CHECK(launch_plane_mm(0, h->g.kind[0], h->g.kind[1], xi, yi, plds, s));
+    else PP_HIP_CHECK(launch_line(FORM_F64, h->g.kind[0], h->g.nx, 0, 0, xi, s));
     if ((rc = mark(h))) return rc;
     end_timing(h);
     return PP_SUCCESS;
