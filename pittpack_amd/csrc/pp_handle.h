@@ -5,6 +5,7 @@
 
 #include <vector>
 
+#include "pp_hostcopy.h"
 #include "pp_launch.h"
 #include "pp_setup.h"
 #include "pp_zsolve.h"
@@ -29,6 +30,7 @@ struct pp_solver {
     hipStream_t stream = nullptr;
     bool own_stream = false;
     double *d_field = nullptr;
+    pp::HostRing ring;  // pinned memory behind pp_get_solution
     double *d_lamx = nullptr, *d_lamy = nullptr, *d_dtab = nullptr;
     double *d_ztw = nullptr, *d_zA = nullptr;   // periodic z: line tables tw and A of length nz
     double *d_zc2 = nullptr;                    //   and 2 cos(2 pi k / nz)

@@ -35,6 +35,7 @@
 
 #include "pittpack_hip.h"
 #include "pp_batch_core.h"
+#include "pp_hostcopy.h"
 #include "pp_launch.h"
 
 using namespace pp;
@@ -567,7 +568,8 @@ int pp_server_wait_ex(pp_server s, long long ticket, double *u, double *latency_
         s->reqs.erase(it);
     }
     const int rc = r->rc;
-    if (!rc && r->staged && u) std::memcpy(u, s->stage + r->stage_off, (size_t)r->points() * sizeof(double));
+    if (!rc && r->staged && u)
+        copy_by_threads(u, s->stage + r->stage_off, (size_t)r->points() * sizeof(double));
     if (latency_ms) *latency_ms = r->t_done - r->t_submit;
     if (batch_seq) *batch_seq = r->batch_seq;
     if (r->staged) {

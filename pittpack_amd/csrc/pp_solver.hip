@@ -1300,6 +1300,7 @@ int pp_destroy(pp_handle h)
     if (h->d_zt) (void)hipFree(h->d_zt);
     if (h->d_partials) (void)hipFree(h->d_partials);
     if (h->d_field) (void)hipFree(h->d_field);
+    free_ring(h->ring);
     for (auto &e : h->ev)
         if (e) (void)hipEventDestroy(e);
     h->ev.clear();
@@ -1403,9 +1404,7 @@ int pp_get_solution(pp_handle h, double *u)
 {
     if (!h) return PP_INVALID_HANDLE;
     if (!u) return PP_INPUT_ARGS;
-    const size_t bytes = (size_t)h->g.nx * h->g.ny * h->g.nz * sizeof(double);
-    PP_HIP_CHECK(hipMemcpyAsync(u, h->d_field, bytes, hipMemcpyDeviceToHost, h->stream));
-    PP_HIP_CHECK(hipStreamSynchronize(h->stream));
+    PP_HIP_CHECK(copy_to_host(h->ring, u, h->d_field, (size_t)h->g.nx * h->g.ny * h->g.nz, h->stream));
     return PP_SUCCESS;
 }
 
