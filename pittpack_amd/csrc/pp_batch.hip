@@ -56,6 +56,70 @@ int put(T *dst, const std::vector<T> &v, hipStream_t s)
 
 }  // namespace
 
+int BatchLanes::create()
+{
+    bool ok = hipEventCreateWithFlags(&fork, hipEventDisableTiming) == hipSuccess;
+    for (int k = 0; ok && k < kSide; k++)
+        ok = hipStreamCreateWithFlags(&side[k], hipStreamNonBlocking) == hipSuccess &&
+             hipEventCreateWithFlags(&join[k], hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();
+        destroy();
+    }
+    return ok ? PP_SUCCESS : PP_HIP_ERROR;
+}
+
+void BatchLanes::destroy()
+{
+    for (int k = 0; k < kSide; k++) {
+        if (side[k]) {
+            (void)hipStreamSynchronize(side[k]);
+            (void)hipStreamDestroy(side[k]);
+        }
+        if (join[k]) (void)hipEventDestroy(join[k]);
+        side[k] = nullptr;
+        join[k] = nullptr;
+    }
+    if (fork) (void)hipEventDestroy(fork);
+    fork = nullptr;
+}
+
+hipError_t BatchLanes::split(hipStream_t s)
+{
+    hipError_t e = hipEventRecord(fork, s);
+    for (int k = 0; e == hipSuccess && k < kSide; k++) e = hipStreamWaitEvent(side[k], fork, 0);
+    return e;
+}
+
+hipError_t BatchLanes::merge(hipStream_t s)
+{
+    hipError_t r = hipSuccess;
+    for (int k = 0; k < kSide; k++) {
+        hipError_t e = hipEventRecord(join[k], side[k]);
+        if (e == hipSuccess) e = hipStreamWaitEvent(s, join[k], 0);
+        if (e != hipSuccess) r = e;
+    }
+    return r;
+}
+
+// The classes of one stage over the lanes: largest first (their order within a stage is free), each
+// to the lane with the least work so far
+void BatchCore::plan_lanes(std::initializer_list<std::vector<HostClass> *> stage)
+{
+    std::vector<HostClass *> all;
+    for (std::vector<HostClass> *v : stage) {
+        std::stable_sort(v->begin(), v->end(), [](const HostClass &a, const HostClass &b) {
+            return (double)a.nitems * a.key > (double)b.nitems * b.key;
+        });
+        for (HostClass &c : *v) all.push_back(&c);
+    }
+    double load[BatchLanes::kSide + 1] = {};
+    for (HostClass *c : all) {
+        c->lane = (int)(std::min_element(std::begin(load), std::end(load)) - std::begin(load));
+        load[c->lane] += (double)c->nitems * c->key;
+    }
+}
+
 TableCache::~TableCache()
 {
     for (auto &kv : t_)
@@ -487,6 +551,10 @@ int BatchCore::plan()
         if ((rc = plan_lines<double>(0, lx_)) || (rc = plan_lines<double>(1, ly_))) return rc;
     }
     plan_z();
+    plan_lanes({&lp_, &lx_});
+    plan_lanes({&ly_});
+    plan_lanes({&lz_, &lzp_});
+    plan_lanes({&lxc_});
     // shape classes per stage: the plane members' count too, though they share one launch
     for (int a = 0; a < 2; a++) {
         std::set<std::pair<int, int>> cls;
@@ -697,7 +765,7 @@ int BatchCore::run_line_stage(hipStream_t s, std::vector<HostClass> &cls, int fo
 {
     int rc;
     for (const HostClass &c : cls)
-        if ((rc = launch_class(s, c, form, axis, fwd, in, out, bflags, sums, plane, accumulate, ztiled, acc0, acc1)))
+        if ((rc = launch_class(lane(s, c.lane), c, form, axis, fwd, in, out, bflags, sums, plane, accumulate, ztiled, acc0, acc1)))
             return rc;
     return PP_SUCCESS;
 }
@@ -813,20 +881,11 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
         if (f32) {
             z.tau = tau;
             z.pinned_zero = 1;
-            PPB_CHECK(launch_zsolve_pcr_f32(16 * c.key, z, s));
+            PPB_CHECK(launch_zsolve_pcr_f32(16 * c.key, z, lane(s, c.lane)));
         } else {
             z.tau = zthomas_tau;  // the nearly singular columns are left to the Thomas sweeps
-            PPB_CHECK(launch_zsolve_pcr_f64(16 * c.key, z, s));
+            PPB_CHECK(launch_zsolve_pcr_f64(16 * c.key, z, lane(s, c.lane)));
         }
-    }
-    if (!f32 && !zth_.empty()) {
-        ZArgs z{};
-        z.data = d_tiles;
-        z.tiled = 1;
-        z.tile_w = zsolve_cpb<double>();
-        z.tile_rows = 0;  // ceil16(nz) per member
-        z.solves = d_zs_;
-        PPB_CHECK(launch_zthomas_f64(z, d_zth_, d_zth_tab_, (int)zth_.size(), s));
     }
     // FP64 columns of 513..1024 rows: the long-column kernel on the member's z tiles
     for (int m : zlong_) {
@@ -846,7 +905,7 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
         z.zlo_dirichlet = zs.zlo_dirichlet;
         z.zhi_dirichlet = zs.zhi_dirichlet;
         z.zero_mode = zero_mode;
-        PPB_CHECK(launch_zsolve_long_f64(zs.nz, z, s));
+        PPB_CHECK(launch_zsolve_long_f64(zs.nz, z, lane(s, m % (BatchLanes::kSide + 1))));
     }
     // periodic z, in place on the solution arena (FP64) or the work arena (FP32 storage, FP64
     // arithmetic, singular column zeroed)
@@ -861,7 +920,8 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
         zp.pinned_zero = f32 ? 1 : 0;
         zp.items = (const ZItem *)c.d_items;
         zp.solves = d_zs_;
-        PPB_CHECK(f32 ? launch_zperiodic_f32_batch(zp, c.nitems, s) : launch_zperiodic_f64_batch(zp, c.nitems, s));
+        const hipStream_t q = lane(s, c.lane);
+        PPB_CHECK(f32 ? launch_zperiodic_f32_batch(zp, c.nitems, q) : launch_zperiodic_f64_batch(zp, c.nitems, q));
     }
     for (int m : zpl_) {
         const SolveSetup &g = mem[m].g;
@@ -896,11 +956,27 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
         a.ncols = g.nx * g.ny;
         a.nplanes = 1;
         const int form = f32 ? FORM_F32 : FORM_F64;
-        PPB_CHECK(launch_line(form, KIND_PP, g.nz, 1, 1, a, s));
-        PPB_CHECK(f32 ? launch_zper_divide_f32(zp, s) : launch_zper_divide(zp, s));
-        PPB_CHECK(launch_line(form, KIND_PP, g.nz, 1, 0, a, s));
+        const hipStream_t q = lane(s, m % (BatchLanes::kSide + 1));
+        PPB_CHECK(launch_line(form, KIND_PP, g.nz, 1, 1, a, q));
+        PPB_CHECK(f32 ? launch_zper_divide_f32(zp, q) : launch_zper_divide(zp, q));
+        PPB_CHECK(launch_line(form, KIND_PP, g.nz, 1, 0, a, q));
     }
-    if (!f32) PPB_CHECK(launch_smt_v1_batch(d_sol, d_smt_, (int)smt_.size(), smt_nz_max_, s));
+    return PP_SUCCESS;
+}
+
+// FP64: the columns the z stage's other launches leave out, on tiles and fields they have written
+int BatchCore::run_z_columns(hipStream_t s)
+{
+    if (!zth_.empty()) {
+        ZArgs z{};
+        z.data = d_tiles;
+        z.tiled = 1;
+        z.tile_w = zsolve_cpb<double>();
+        z.tile_rows = 0;  // ceil16(nz) per member
+        z.solves = d_zs_;
+        PPB_CHECK(launch_zthomas_f64(z, d_zth_, d_zth_tab_, (int)zth_.size(), s));
+    }
+    PPB_CHECK(launch_smt_v1_batch(d_sol, d_smt_, (int)smt_.size(), smt_nz_max_, s));
     return PP_SUCCESS;
 }
 
@@ -920,25 +996,54 @@ int BatchCore::run_planes(hipStream_t s, int fwd)
     for (const HostClass &c : lp_) {
         x.items = y.items = (const LineItem *)c.d_items;
         x.nlines = c.nitems;
-        PPB_CHECK(launch_plane_mm(fwd, 0, 0, x, y, c.lds, s, d_ps_, c.key));
+        PPB_CHECK(launch_plane_mm(fwd, 0, 0, x, y, c.lds, lane(s, c.lane), d_ps_, c.key));
     }
     return PP_SUCCESS;
+}
+
+// one stage's launches, over the side streams if there are several to spread
+template <typename F>
+int BatchCore::run_stage(hipStream_t s, size_t classes, const F &launches)
+{
+    forked_ = classes > 1 && lanes;
+    if (forked_ && lanes->split(s) != hipSuccess) {
+        forked_ = false;
+        return PP_HIP_ERROR;
+    }
+    int rc = launches();
+    // (after an error too: no stream is left in a capture or ahead of the batch's own)
+    if (forked_ && lanes->merge(s) != hipSuccess && !rc) rc = PP_HIP_ERROR;
+    forked_ = false;
+    return rc;
 }
 
 int BatchCore::run_fp64(hipStream_t s, Marks *mk)
 {
     int rc;
-    if ((rc = run_planes(s, 1))) return rc;
-    if ((rc = run_line_stage(s, lx_, FORM_F64, 0, 1, d_rhs, d_sol, BF_RHS, nullptr, nullptr, 0))) return rc;
+    const size_t nx = lx_.size() + lp_.size(), ny = ly_.size();
+    if ((rc = run_stage(s, nx, [&] {
+             const int r = run_planes(s, 1);
+             return r ? r : run_line_stage(s, lx_, FORM_F64, 0, 1, d_rhs, d_sol, BF_RHS, nullptr, nullptr, 0);
+         })))
+        return rc;
     if ((rc = mark(s, mk))) return rc;
-    if ((rc = run_line_stage(s, ly_, FORM_F64, 1, 1, d_sol, d_tiles, 0, nullptr, nullptr, 0, ZT_OUT))) return rc;
+    if ((rc = run_stage(s, ny, [&] {
+             return run_line_stage(s, ly_, FORM_F64, 1, 1, d_sol, d_tiles, 0, nullptr, nullptr, 0, ZT_OUT);
+         })))
+        return rc;
     if ((rc = mark(s, mk))) return rc;
-    if ((rc = run_z_stage(s, false))) return rc;
+    if ((rc = run_stage(s, z_classes(), [&] { return run_z_stage(s, false); })) || (rc = run_z_columns(s))) return rc;
     if ((rc = mark(s, mk))) return rc;
-    if ((rc = run_line_stage(s, ly_, FORM_F64, 1, 0, d_tiles, d_sol, 0, nullptr, nullptr, 0, ZT_IN))) return rc;
+    if ((rc = run_stage(s, ny, [&] {
+             return run_line_stage(s, ly_, FORM_F64, 1, 0, d_tiles, d_sol, 0, nullptr, nullptr, 0, ZT_IN);
+         })))
+        return rc;
     if ((rc = mark(s, mk))) return rc;
-    if ((rc = run_line_stage(s, lx_, FORM_F64, 0, 0, d_sol, d_sol, BF_SCALE, nullptr, nullptr, 0))) return rc;
-    if ((rc = run_planes(s, 0))) return rc;
+    if ((rc = run_stage(s, nx, [&] {
+             const int r = run_line_stage(s, lx_, FORM_F64, 0, 0, d_sol, d_sol, BF_SCALE, nullptr, nullptr, 0);
+             return r ? r : run_planes(s, 0);
+         })))
+        return rc;
     return mark(s, mk);
 }
 
@@ -946,9 +1051,14 @@ int BatchCore::run_fp64(hipStream_t s, Marks *mk)
 int BatchCore::mixed_inner(hipStream_t s, Marks *mk)
 {
     int rc;
-    if ((rc = run_line_stage(s, ly_, FORM_F32, 1, 1, d_w, d_w, 0, nullptr, nullptr, 0))) return rc;
+    auto y = [&](int fwd) {
+        return run_stage(s, ly_.size(), [&] {
+            return run_line_stage(s, ly_, FORM_F32, 1, fwd, d_w, d_w, 0, nullptr, nullptr, 0);
+        });
+    };
+    if ((rc = y(1))) return rc;
     if ((rc = mark(s, mk))) return rc;
-    if ((rc = run_z_stage(s, true))) return rc;
+    if ((rc = run_stage(s, z_classes(), [&] { return run_z_stage(s, true); }))) return rc;
     if (!fix_.empty()) {
         ZArgs z{};
         z.data = d_w;
@@ -967,7 +1077,7 @@ int BatchCore::mixed_inner(hipStream_t s, Marks *mk)
         }
     }
     if ((rc = mark(s, mk))) return rc;
-    if ((rc = run_line_stage(s, ly_, FORM_F32, 1, 0, d_w, d_w, 0, nullptr, nullptr, 0))) return rc;
+    if ((rc = y(0))) return rc;
     return mark(s, mk);
 }
 
@@ -979,15 +1089,19 @@ int BatchCore::run_mixed(hipStream_t s, Marks *mk)
     double *sums = nm00 ? d_sums_ : nullptr;
     const double *plane = nm00 ? d_plane_ : nullptr;
     const int R = refine;
-    if ((rc = run_line_stage(s, lx_, FORM_F64_TO_F32, 0, 1, d_rhs, d_w, BF_RHS, sums, nullptr, 0))) return rc;
+    auto x = [&](int form, int fwd, const void *in, void *out, int bflags, double *ls, const double *pl, int acc,
+                 const float *a0 = nullptr, const float *a1 = nullptr) {
+        return run_stage(s, lx_.size(), [&] { return run_line_stage(s, lx_, form, 0, fwd, in, out, bflags, ls, pl, acc, 0, a0, a1); });
+    };
+    if ((rc = x(FORM_F64_TO_F32, 1, d_rhs, d_w, BF_RHS, sums, nullptr, 0))) return rc;
     if ((rc = mark(s, mk))) return rc;
     if ((rc = mixed_inner(s, mk))) return rc;
     if (nm00) PPB_CHECK(launch_mode00_batch(d_m00_, nm00, nz_max_, 0, s));
     // u0 in FP32 while refinement follows, else the FP64 solution
     if (R > 0) {
-        if ((rc = run_line_stage(s, lx_, FORM_F32, 0, 0, d_w, d_u0, BF_SCALE, nullptr, plane, 0))) return rc;
+        if ((rc = x(FORM_F32, 0, d_w, d_u0, BF_SCALE, nullptr, plane, 0))) return rc;
     } else {
-        if ((rc = run_line_stage(s, lx_, FORM_F32_TO_F64, 0, 0, d_w, d_sol, BF_SCALE, nullptr, plane, 0))) return rc;
+        if ((rc = x(FORM_F32_TO_F64, 0, d_w, d_sol, BF_SCALE, nullptr, plane, 0))) return rc;
     }
     if ((rc = mark(s, mk))) return rc;
     for (int it = 0; it < R; it++) {
@@ -996,39 +1110,42 @@ int BatchCore::run_mixed(hipStream_t s, Marks *mk)
         PPB_CHECK(launch_residual_pair_f32_batch(d_res_, d_rpitems_, (int)rpitems_.size(), resp_two_, src, s));
         if ((rc = mark(s, mk))) return rc;
         // the corrections' x forward: fused members compute their residual inside it
-        for (const HostClass &c : lxc_) {
-            if (c.fused) {
-                const AxisDev &t = tabs_.at({c.key, c.kind, c.axis});
-                LineArgs a{};
-                a.in = d_w;
-                a.out = d_w;
-                a.tw = t.tw;
-                a.A = t.A;
-                a.B = t.B;
-                a.C = t.C;
-                a.D = t.D;
-                a.in_scale = 1.0;
-                a.out_scale = 1.0;
-                a.items = (const LineItem *)c.d_items;
-                a.solves = d_ls_;
-                a.nlines = c.nitems;
-                a.line_sums = sums;
-                PPB_CHECK(launch_resx(c.kind, c.key, src, a, ResArgs{}, d_res_, s));
-            } else if ((rc = launch_class(s, c, FORM_F32, 0, 1, d_w, d_w, 0, sums, nullptr, 0, 0))) {
-                return rc;
+        rc = run_stage(s, lxc_.size(), [&]() -> int {
+            for (const HostClass &c : lxc_) {
+                if (c.fused) {
+                    const AxisDev &t = tabs_.at({c.key, c.kind, c.axis});
+                    LineArgs a{};
+                    a.in = d_w;
+                    a.out = d_w;
+                    a.tw = t.tw;
+                    a.A = t.A;
+                    a.B = t.B;
+                    a.C = t.C;
+                    a.D = t.D;
+                    a.in_scale = 1.0;
+                    a.out_scale = 1.0;
+                    a.items = (const LineItem *)c.d_items;
+                    a.solves = d_ls_;
+                    a.nlines = c.nitems;
+                    a.line_sums = sums;
+                    PPB_CHECK(launch_resx(c.kind, c.key, src, a, ResArgs{}, d_res_, lane(s, c.lane)));
+                } else if (int r = launch_class(lane(s, c.lane), c, FORM_F32, 0, 1, d_w, d_w, 0, sums, nullptr, 0, 0)) {
+                    return r;
+                }
             }
-        }
+            return PP_SUCCESS;
+        });
+        if (rc) return rc;
         if ((rc = mark(s, mk))) return rc;
         if ((rc = mixed_inner(s, mk))) return rc;
         if (nm00) PPB_CHECK(launch_mode00_batch(d_m00_, nm00, nz_max_, 1, s));
         if (it == R - 1) {
             // u = u0 + csum + c, in FP64
-            if ((rc = run_line_stage(s, lx_, FORM_F32_TO_F64, 0, 0, d_w, d_sol, BF_SCALE, nullptr, plane, 0, 0, d_u0,
-                                     it > 0 ? d_cacc : nullptr)))
+            if ((rc = x(FORM_F32_TO_F64, 0, d_w, d_sol, BF_SCALE, nullptr, plane, 0, d_u0, it > 0 ? d_cacc : nullptr)))
                 return rc;
         } else {
             // csum = c1, then csum += c
-            if ((rc = run_line_stage(s, lx_, FORM_F32, 0, 0, d_w, d_cacc, BF_SCALE, nullptr, plane, it > 0 ? 1 : 0)))
+            if ((rc = x(FORM_F32, 0, d_w, d_cacc, BF_SCALE, nullptr, plane, it > 0 ? 1 : 0)))
                 return rc;
         }
         if ((rc = mark(s, mk))) return rc;
@@ -1332,9 +1449,13 @@ int pp_batch_solve(pp_batch b)
         // capture this solve's launches (kernels only: no memset or copy is recorded) and
         // replay the graph from now on
         hipGraph_t g = nullptr;
-        PPB_CHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeRelaxed));
-        const int rc = b->core.run(b->stream, nullptr);
-        const hipError_t ec = hipStreamEndCapture(b->stream, &g);
+        BatchLanes lanes;  // become branches of the graph
+        if (b->core.points() >= BatchLanes::kMinPoints && lanes.create() == PP_SUCCESS) b->core.lanes = &lanes;
+        const hipError_t eb = hipStreamBeginCapture(b->stream, hipStreamCaptureModeRelaxed);
+        const int rc = eb == hipSuccess ? b->core.run(b->stream, nullptr) : PP_HIP_ERROR;
+        const hipError_t ec = eb == hipSuccess ? hipStreamEndCapture(b->stream, &g) : eb;
+        b->core.lanes = nullptr;
+        lanes.destroy();
         if (rc || ec != hipSuccess) {
             if (g) (void)hipGraphDestroy(g);
             return rc ? rc : PP_HIP_ERROR;

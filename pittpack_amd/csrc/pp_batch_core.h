@@ -52,6 +52,25 @@ struct Marks {
     int n = 0, max = 0;
 };
 
+// Streams beside a batch's own on which the classes of a stage run at the same time while a solve is
+// captured: branches of its graph.  A class' launch fills the chip only in its middle, and 48 members
+// of 16..96 points a side are some 70 launches of 6 to 65 us: 1.68 ms in series, 1.28 to 1.37 ms over four
+// branches (mixed form 4.25 and 3.61; 200 members 4.1 and 3.6, 1000 members 19.6 and 19.5).  A stage's split
+// and merge cost some 15 us, so batches under kMinPoints stay in series (4.7 million points: 0.21 in
+// series, 0.26 over branches; 12.3 million: 0.51 and 0.43, 13.0 million: 0.41 and 0.40); launched one by one
+// they cost more (4.7 million points: 0.37 ms), so there is no such split outside a graph.
+struct BatchLanes {
+    static constexpr long kMinPoints = 10000000;
+    static constexpr int kSide = 3;  // with the batch's own, the process' four hardware queues
+    hipStream_t side[kSide] = {};
+    hipEvent_t fork = nullptr, join[kSide] = {};
+    int create();  // PP code; nothing is left behind on failure
+    void destroy();
+    // work launched on `s` so far happens before the side streams' / the side streams' before `s`'
+    hipError_t split(hipStream_t s);
+    hipError_t merge(hipStream_t s);
+};
+
 struct BatchMember {
     SolveSetup g;
     long offset = 0;  // element offset of the member's field in the rhs / solution / work arenas
@@ -86,6 +105,7 @@ class BatchCore {
     int upload(hipStream_t s);
     // the solve of every member (right-hand sides kept, solutions in the solution arena)
     int run(hipStream_t s, Marks *mk);
+    BatchLanes *lanes = nullptr;  // a captured run's stages, class by class over these (null: in series)
     // FP64: time each line class in both launch shapes on this batch (bound, uploaded) and
     // keep the faster per class and direction; the right-hand-side arena is overwritten
     int tune_lines(hipStream_t s);
@@ -118,8 +138,11 @@ class BatchCore {
         size_t off_alt = 0;
         void *d_items_alt = nullptr;
         size_t lds = 0;      // plane classes: of their largest plane
+        int lane = 0;        // stream of the class within its stage (0: the batch's own)
         bool fused = false;  // correction x classes: members whose residual runs in k_resx
     };
+    hipStream_t lane(hipStream_t s, int k) const { return forked_ && k > 0 ? lanes->side[k - 1] : s; }
+    void plan_lanes(std::initializer_list<std::vector<HostClass> *> stage);
     int launch_class(hipStream_t s, const HostClass &c, int form, int axis, int fwd, const void *in, void *out,
                      int bflags, double *sums, const double *plane, int accumulate, int ztiled,
                      const float *acc0 = nullptr, const float *acc1 = nullptr);
@@ -131,6 +154,10 @@ class BatchCore {
                        void *out, int bflags, double *sums, const double *plane, int accumulate, int ztiled = 0,
                        const float *acc0 = nullptr, const float *acc1 = nullptr);
     int run_z_stage(hipStream_t s, bool f32);
+    template <typename F>
+    int run_stage(hipStream_t s, size_t classes, const F &launches);
+    size_t z_classes() const { return lz_.size() + lzp_.size() + zlong_.size() + zpl_.size(); }
+    int run_z_columns(hipStream_t s);
     int run_planes(hipStream_t s, int fwd);
     int run_fp64(hipStream_t s, Marks *mk);
     int mixed_inner(hipStream_t s, Marks *mk);
@@ -142,6 +169,7 @@ class BatchCore {
     std::vector<ZSolve> zs_;
     std::vector<HostClass> lx_, ly_, lz_;
     std::vector<HostClass> lp_;  // FP64: plane launches, items {member, z}, by waves a block
+    bool forked_ = false;        // inside run_stage, over the side streams
     std::vector<PlaneSolve> ps_;
     PlaneSolve *d_ps_ = nullptr;
     size_t o_ps_ = 0;
