@@ -112,7 +112,8 @@ enum {
      * src/triDiag.cpp:1693-1822, its factors in the reference's order) instead of the PCR
      * steps, which lose up to ten times more digits on nearly singular columns (long Neumann or
      * periodic axes, cells thinner in z).  Default 1e-3 (the columns where the two differ beyond
-     * 1e-13); 0 = off. */
+     * 1e-13); 0 = off.  Columns of up to 64 rows, and of up to 128 on grids of 8192 columns or
+     * more, are swept from both ends in any case and need no list. */
     PP_OPT_ZTHOMAS_TAU = 15,
     /* mixed form: each refinement step computes the FP64 residual inside its FP32 x-forward
      * transform (one kernel; the residual is never stored), where the x lines have a compiled

@@ -285,7 +285,8 @@ int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
 
 void BatchCore::plan_z()
 {
-    std::map<int, std::vector<ZItem>> cls, pcls;
+    std::map<std::pair<int, int>, std::vector<ZItem>> cls;  // {rows / 16, both ends at once}
+    std::map<int, std::vector<ZItem>> pcls;
     const int cpb = precision == 1 ? zsolve_cpb<float>() : zsolve_cpb<double>();
     zpl_.clear();
     zlong_.clear();
@@ -335,7 +336,8 @@ void BatchCore::plan_z()
             zlong_.push_back(m);
             continue;
         }
-        if (precision == 0 && zthomas_tau > 0.0) {
+        const bool twist = precision == 0 && ztwist_serves(g.nx, g.ny, g.nz);
+        if (precision == 0 && zthomas_tau > 0.0 && !twist) {
             // nearly singular columns, as the single-solve handle lists them
             const std::vector<double> lx = eig_factors(g, 0), ly = eig_factors(g, 1);
             const double Cx = (g.dxyz[2] / g.dxyz[0]) * (g.dxyz[2] / g.dxyz[0]);
@@ -352,19 +354,40 @@ void BatchCore::plan_z()
                                     zth_tab_.data() + zth_tab_.size() - 2 * (size_t)g.nz);
                 }
         }
-        auto &items = cls[(g.nz + 15) / 16];
+        auto &items = cls[{(g.nz + 15) / 16, twist}];
         const int nbx = (g.nx + cpb - 1) / cpb;
+        if (twist) {
+            const int np = (g.ny + 1) / 2;
+            if (ztwist_by_column(g.nx, g.ny, g.nz)) {
+                for (int bx = 0; bx < nbx; bx++)
+                    for (int p = 0; p < np; p++) items.push_back({m, bx, p});
+            } else {
+                for (int p = 0; p < np; p++)
+                    for (int bx = 0; bx < nbx; bx++) items.push_back({m, bx, p});
+            }
+            continue;
+        }
         for (int sy = 0; sy < g.ny; sy++)
             for (int bx = 0; bx < nbx; bx++) items.push_back({m, bx, sy});
     }
     lz_.clear();
     for (auto &kv : cls) {
         HostClass c;
-        c.key = kv.first;
+        c.key = kv.first.first;
+        c.kind = kv.first.second;
         c.nitems = (int)kv.second.size();
         c.zi = std::move(kv.second);
         lz_.push_back(std::move(c));
     }
+    // the Thomas columns in the order of the classes they run beside
+    auto zclass = [&](const ZThomasItem &t) { return (mem[t.solve].g.nz + 15) / 16; };
+    std::stable_sort(zth_.begin(), zth_.end(),
+                     [&](const ZThomasItem &a, const ZThomasItem &b) { return zclass(a) < zclass(b); });
+    for (HostClass &c : lz_)
+        for (int i = 0; i < (int)zth_.size(); i++)
+            if (!c.kind && zclass(zth_[i]) == c.key) {
+                if (c.th_count++ == 0) c.th_first = i;
+            }
     lzp_.clear();
     for (auto &kv : pcls) {
         HostClass c;
@@ -563,7 +586,9 @@ int BatchCore::plan()
             if (m.plane) cls.insert({a == 0 ? m.g.nx : m.g.ny, m.g.kind[a]});
         launches[a] = (int)cls.size();
     }
-    launches[2] = (int)(lz_.size() + lzp_.size() + 3 * zpl_.size() + zlong_.size() + (smt_.empty() ? 0 : 1));
+    std::set<int> zrows;
+    for (const HostClass &c : lz_) zrows.insert(c.key);
+    launches[2] = (int)(zrows.size() + lzp_.size() + 3 * zpl_.size() + zlong_.size() + (smt_.empty() ? 0 : 1));
     ls_.assign(mem.size(), LineSolve{});
     zs_.assign(mem.size(), ZSolve{});
     // region layout
@@ -883,8 +908,13 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
             z.pinned_zero = 1;
             PPB_CHECK(launch_zsolve_pcr_f32(16 * c.key, z, lane(s, c.lane)));
         } else {
-            z.tau = zthomas_tau;  // the nearly singular columns are left to the Thomas sweeps
-            PPB_CHECK(launch_zsolve_pcr_f64(16 * c.key, z, lane(s, c.lane)));
+            z.tau = zthomas_tau;  // the nearly singular columns are the Thomas sweeps'
+            z.tile_w = zsolve_cpb<double>();
+            z.th = d_zth_ + c.th_first;
+            z.th_tab = d_zth_tab_;
+            z.nth = c.th_count;
+            const hipStream_t q = lane(s, c.lane);
+            PPB_CHECK(c.kind ? launch_ztwist(16 * c.key, z, q) : launch_zsolve_pcr_f64(16 * c.key, z, q));
         }
     }
     // FP64 columns of 513..1024 rows: the long-column kernel on the member's z tiles
@@ -964,18 +994,9 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
     return PP_SUCCESS;
 }
 
-// FP64: the columns the z stage's other launches leave out, on tiles and fields they have written
+// FP64: the singular columns of periodic z, on fields the z stage's other launches have written
 int BatchCore::run_z_columns(hipStream_t s)
 {
-    if (!zth_.empty()) {
-        ZArgs z{};
-        z.data = d_tiles;
-        z.tiled = 1;
-        z.tile_w = zsolve_cpb<double>();
-        z.tile_rows = 0;  // ceil16(nz) per member
-        z.solves = d_zs_;
-        PPB_CHECK(launch_zthomas_f64(z, d_zth_, d_zth_tab_, (int)zth_.size(), s));
-    }
     PPB_CHECK(launch_smt_v1_batch(d_sol, d_smt_, (int)smt_.size(), smt_nz_max_, s));
     return PP_SUCCESS;
 }

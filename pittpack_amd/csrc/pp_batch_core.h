@@ -137,6 +137,7 @@ class BatchCore {
         std::vector<LineItem> li_alt;
         size_t off_alt = 0;
         void *d_items_alt = nullptr;
+        int th_first = 0, th_count = 0;  // FP64 z classes: their Thomas columns in zth_
         size_t lds = 0;      // plane classes: of their largest plane
         int lane = 0;        // stream of the class within its stage (0: the batch's own)
         bool fused = false;  // correction x classes: members whose residual runs in k_resx

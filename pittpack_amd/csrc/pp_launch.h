@@ -34,13 +34,19 @@ bool zfix_tiles_supported(int nz);
 hipError_t launch_zfix_tiles_f32(int nz_max, const ZArgs &a, hipStream_t s);
 
 // the reference's Thomas sweeps (thomasLowMem) on listed FP64 columns in place or on z tiles
-// (a's layout), one wave per column, nz <= 1024.  solve >= 0: batched, the member's field and
-// sizes from a.solves; toff: offset of the column's factors {1 / bet_j, tmp_j} in tab
-// (zthomas_factors, 2 nz values)
-struct ZThomasItem {
-    int sx, sy, solve, pad;
-    long toff;
-};
+// (a's layout), one wave per column, nz <= 1024, in a launch of their own (launch_zsolve_pcr_f64 takes
+// them along: a.th)
+// columns of up to 128 rows, in place or on tiles of 16 columns (no Thomas columns: a.tau is not looked at); batched:
+// one item {member, tile column, pair of y lines} per wave.  Which solves take them instead of k_zsolve (a
+// whole solve of nx x ny x nz, us): all up to 64 rows (64x64x64 28.2 : 28.7, 128x128x64 39.4 : 42.9), and up
+// to 128 those of many columns (128x128x96 51.0 : 53.6, but 64x64x96 32.3 : 30.9, 96x64x96 39.2 : 39.1: two
+// lanes a column leave a chip of few columns idle)
+constexpr bool ztwist_serves(int nx, int ny, int nz) { return nz <= 64 || (nz <= 128 && (long)nx * ny >= 8192); }
+// Their blocks go along x first, so that a tile column whose y blocks ran on one XCD is solved there
+// (128x96x64 40.7 to 36.2 us a solve), or, where the field is past half the 256 MB cache, down one tile
+// column after the other, in the order of memory (z stage of 512x512x128: 99.6 to 89.5 us)
+__host__ __device__ inline bool ztwist_by_column(int nx, int ny, int nz) { return (long)nx * ny * nz > (16l << 20); }
+hipError_t launch_ztwist(int nz, const ZArgs &a, hipStream_t s);
 hipError_t launch_zthomas_f64(const ZArgs &a, const ZThomasItem *items, const double *tab, int nitems, hipStream_t s);
 
 // thomasLowMem's factors of one column (src/triDiag.cpp:1693-1822): out[j] = 1 / bet_j,

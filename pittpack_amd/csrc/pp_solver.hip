@@ -504,7 +504,8 @@ int run_zperiodic(pp_solver *h, void *data, bool f32, int tile_rows)
 // most 512 rows, non-periodic z
 bool zthomas_on(const pp_solver *h)
 {
-    return h->zthomas_tau > 0.0 && !h->g.zper && (h->zsolver == 0 || h->zsolver == 1) && zsolve_supported_f64(h->g.nz);
+    return h->zthomas_tau > 0.0 && !h->g.zper && (h->zsolver == 0 || h->zsolver == 1) && zsolve_supported_f64(h->g.nz) &&
+           !(h->zsolver == 0 && ztwist_serves(h->g.nx, h->g.ny, h->g.nz));  // whose sweeps are exact on them
 }
 
 // The columns the serial Thomas takes: |eig+2| < zthomas_tau with the kernels' eigenvalue
@@ -630,14 +631,22 @@ int run_fp64_stages(pp_solver *h, const double *rhs, double *field)
         } else {
             // nearly singular columns left to the reference's serial Thomas (PP_OPT_ZTHOMAS_TAU)
             if (zth) z.tau = h->zthomas_tau;
+            if (zth && h->zsolver == 0) {
+                z.th = h->d_zthomas;
+                z.th_tab = h->d_zthomas_tab;
+                z.nth = h->nzthomas;
+            }
             switch (h->zsolver) {
             case 1: PP_HIP_CHECK(launch_zsolve_scan_f64(h->g.nz, z, s)); break;
             case 2: PP_HIP_CHECK(launch_zsolve_mg_f64(z, h->mg_cycles, h->mg_tol, s)); break;
             case 3: PP_HIP_CHECK(launch_zsolve_pcr_full_f64(z, s)); break;
             case 4: PP_HIP_CHECK(launch_zsolve_cr_f64(z, s)); break;
-            default: PP_HIP_CHECK(launch_zsolve_pcr_f64(h->g.nz, z, s)); break;
+            default:
+                if (ztwist_serves(h->g.nx, h->g.ny, h->g.nz)) PP_HIP_CHECK(launch_ztwist(h->g.nz, z, s));
+                else PP_HIP_CHECK(launch_zsolve_pcr_f64(h->g.nz, z, s));
+                break;
             }
-            if (zth) PP_HIP_CHECK(launch_zthomas_f64(z, h->d_zthomas, h->d_zthomas_tab, h->nzthomas, s));
+            if (zth && h->zsolver != 0) PP_HIP_CHECK(launch_zthomas_f64(z, h->d_zthomas, h->d_zthomas_tab, h->nzthomas, s));
         }
     }
     if ((rc = mark(h))) return rc;

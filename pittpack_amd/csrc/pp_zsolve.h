@@ -20,6 +20,7 @@ namespace pp {
 // ---------------------------------------------------------------------------------------
 struct ZItem;
 struct ZSolve;
+struct ZThomasItem;
 
 struct ZArgs {
     void *data;  // [nz][SY][SX], in place
@@ -42,6 +43,11 @@ struct ZArgs {
     // (rows from nz on are zero padding) of W columns contiguously, element (x, y, z) at
     // ((x/W * SY + y) * 16 J + z) * W + x%W; W = tile_w (0: the block's CPB), a multiple of
     // CPB -- a block then takes CPB columns of a tile
+    // columns by the reference's Thomas sweeps in blocks of the same launch (k_zsolve, FP64 in place):
+    // th[0..nth) with factors th_tab, solved by the launch's last blocks; tau leaves them out of the others
+    const ZThomasItem *th;
+    const double *th_tab;
+    int nth;
     int tiled;
     int tile_w;
     int tile_rows;  // rows per tile (0: 16 J); more than 16 J pads each tile at its end
@@ -57,6 +63,13 @@ struct ZSolve {
 };
 struct ZItem {
     int solve, bx, by;
+};
+// a column of the Thomas sweeps: solve >= 0 batched (offset and
+// sizes from a.solves); toff: offset of the column's factors {1 / bet_j, tmp_j} in tab
+// (zthomas_factors, 2 nz values)
+struct ZThomasItem {
+    int sx, sy, solve, pad;
+    long toff;
 };
 
 // Column element access.  The row stride zs is uniform, so row j of a lane sits at the
@@ -304,6 +317,114 @@ constexpr size_t ztile_bytes_cyclic() { return (size_t)16 * J * (CPB + 1) * size
 template <typename R, int J, int CPB>
 constexpr size_t ztile_bytes_blocked() { return (size_t)16 * blocked_lj<J>() * (CPB + 1) * sizeof(R); }
 
+// The reference's Thomas sweep (thomasLowMem, src/triDiag.cpp:1693-1822, not the pinned
+// branch) on one listed FP64 column per block.  Its factors depend only on the column's
+// eigenvalue and end rows, so the host computes them in the reference's order (bet_0 = b0,
+// tmp_j = 1 / bet_{j-1}, bet_j = eig - tmp_j, the last row bn - tmp) and hands over
+// tab = {1 / bet_j, tmp_j} per column.  The two sweeps are then linear recurrences in the
+// column's values -- forward x_j = (x_j - x_{j-1}) / bet_j, backward x_j -= tmp_{j+1} x_{j+1}
+// -- which one wave runs as a scan: each lane composes the affine maps of its contiguous chunk
+// of rows (C = ceil(nz / 64) <= ZTH_CMAX), a Kogge-Stone scan across the 64 lanes gives each lane the
+// value entering its chunk, and the lane sweeps its rows (about 40 dependent steps per sweep
+// instead of nz).  Against the serial sweep this reassociation moves a column by a few 1e-14
+// of its largest value; the PCR steps it replaces lose ~3e-12 on such columns.  The PCR
+// kernel left these columns untouched (|eig + 2| below its tau).
+template <int ZTH_CMAX>
+__device__ __forceinline__ void zthomas_column(const ZArgs &a0, const ZThomasItem &it, const double *tab)
+{
+    constexpr int W = 64;
+    ZArgs a = a0;
+    if (it.solve >= 0) {
+        // batched: the member's field (its z tiles), sizes
+        const ZSolve sv = a0.solves[it.solve];
+        a.data = reinterpret_cast<double *>(a0.data) + sv.offset;
+        a.SX = sv.SX;
+        a.SY = sv.SY;
+        a.nz = sv.nz;
+    }
+    const int n = a.nz;
+    // element j of the column: in place (stride SX*SY) or in its z tile (stride W)
+    long zs = (long)a.SX * a.SY;
+    long off = (long)it.sy * a.SX + it.sx;
+    if (a.tiled) {
+        const int Wt = a.tile_w;
+        const int rows = a.tile_rows ? a.tile_rows : (n + 15) / 16 * 16;
+        off = (((long)(it.sx / Wt) * a.SY + it.sy) * rows) * Wt + it.sx % Wt;
+        zs = Wt;
+    }
+    double *data = reinterpret_cast<double *>(a.data);
+    const double *ib = tab + it.toff, *tp = ib + n;
+    const int L = threadIdx.x, C = (n + W - 1) / W, j0 = L * C;
+    double x[ZTH_CMAX], g[ZTH_CMAX], q[ZTH_CMAX];
+#pragma unroll
+    for (int k = 0; k < ZTH_CMAX; k++) {
+        const int j = j0 + k;
+        const bool in = k < C && j < n;
+        x[k] = in ? data[off + (long)j * zs] : 0.0;
+        g[k] = in ? ib[j] : 0.0;
+        q[k] = (in && j + 1 < n) ? tp[j + 1] : 0.0;
+    }
+    // forward: x_j = -g_j x_{j-1} + x_j g_j, composed over the chunk, scanned in lane order
+    double A = 1.0, B = 0.0;
+#pragma unroll
+    for (int k = 0; k < ZTH_CMAX; k++) {
+        if (k < C && j0 + k < n) {
+            const double m = -g[k];
+            B = m * B + x[k] * g[k];
+            A = m * A;
+        }
+    }
+    for (int s = 1; s < W; s <<= 1) {
+        const double Au = __shfl_up(A, s, W), Bu = __shfl_up(B, s, W);
+        if (L >= s) {
+            B = A * Bu + B;
+            A = A * Au;
+        }
+    }
+    double v = __shfl_up(B, 1, W);
+    if (L == 0) v = 0.0;
+#pragma unroll
+    for (int k = 0; k < ZTH_CMAX; k++) {
+        if (k < C && j0 + k < n) {
+            v = (x[k] - v) * g[k];
+            x[k] = v;
+        }
+    }
+    // backward: x_j = -tmp_{j+1} x_{j+1} + x_j, composed over the chunk from its last row,
+    // scanned in reverse lane order
+    A = 1.0;
+    B = 0.0;
+#pragma unroll
+    for (int k = ZTH_CMAX - 1; k >= 0; k--) {
+        if (k < C && j0 + k < n) {
+            const double m = -q[k];
+            B = m * B + x[k];
+            A = m * A;
+        }
+    }
+    for (int s = 1; s < W; s <<= 1) {
+        const double Ad = __shfl_down(A, s, W), Bd = __shfl_down(B, s, W);
+        if (L + s < W) {
+            B = A * Bd + B;
+            A = A * Ad;
+        }
+    }
+    v = __shfl_down(B, 1, W);
+    if (L == W - 1) v = 0.0;
+#pragma unroll
+    for (int k = ZTH_CMAX - 1; k >= 0; k--) {
+        if (k < C && j0 + k < n) {
+            v = x[k] - q[k] * v;
+            x[k] = v;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < ZTH_CMAX; k++) {
+        const int j = j0 + k;
+        if (k < C && j < n) data[off + (long)j * zs] = x[k];
+    }
+}
+
 // FULL: nz == 16 * J (no padding rows, no per-row bounds checks).  S: element type in
 // memory (FP32 data solved in FP64 when R = double, S = float).  FIX: solve and write back
 // only the near-singular columns (|eig+2| < tau, not pinned) that the FP32 solve left
@@ -320,6 +441,18 @@ __global__ void __launch_bounds__(16 * CPB) k_zsolve(ZArgs a0)
     constexpr bool CP_LDS = sizeof(R) * J > 256;
     ZArgs a = a0;
     int bx = blockIdx.x, by = blockIdx.y;
+    constexpr bool TH = sizeof(R) == 8 && sizeof(S) == 8 && CPB == 16 && J > 8;
+    if constexpr (TH) {
+        // the last blocks (batched) / rows of blocks take the Thomas columns, one each by a wave:
+        // a launch of their own behind this one cost 5 us and a gap, more than their sweeps beside it
+        // (the last, so that the others decide by what they load anyway: a look at nth first, and a
+        // division, cost every block some 1.5 us, 15 % at 512^3)
+        if (a0.items ? bx >= a0.nitems : by >= a0.SY) {
+            const int i = a0.items ? bx - a0.nitems : (by - a0.SY) * gridDim.x + bx;
+            if (i < a0.nth && threadIdx.x < 64) zthomas_column<(J + 3) / 4>(a0, a0.th[i], a0.th_tab);
+            return;
+        }
+    }
     if (CPB * sizeof(S) < 128 && !a0.items) {
         // rows shorter than a 128-byte line (8 FP64 columns): the two blocks sharing a line
         // run on one XCD, so the line is fetched into one L2
@@ -328,7 +461,7 @@ __global__ void __launch_bounds__(16 * CPB) k_zsolve(ZArgs a0)
         by = lin / gridDim.x;
     }
     if (a0.items) {
-        const ZItem it = a0.items[blockIdx.x];
+        const ZItem it = a0.items[bx];
         const ZSolve sv = a0.solves[it.solve];
         a.data = reinterpret_cast<S *>(a0.data) + sv.offset;
         a.SX = sv.SX;
@@ -446,7 +579,16 @@ __global__ void __launch_bounds__(16 * CPB) k_zsolve(ZArgs a0)
 #pragma unroll
         for (int j = 0; j < J; j++) tile[(t + 16 * j) * (CPB + 1) + c] = zero ? (R)0 : d[j];
     }
+    if constexpr (TH) {
+        // (which columns are left out goes through the tile rows' padding: the factors read again
+        // by the storing threads took 25 us at 512^3)
+        if (t == 0) tile[c * (CPB + 1) + CPB] = near ? (R)1 : (R)0;
+    }
     __syncthreads();
+    if constexpr (TH) {
+        // the Thomas columns are another block's to write
+        if (tile[(tid % CPB) * (CPB + 1) + CPB] != (R)0) return;
+    }
     ztile_store<R, J, FULL, OFF32, CPB, decltype(lrow), S>(tile, a, n, lrow, bx, by);
     (void)valid;
     (void)data;

@@ -29,11 +29,23 @@ static hipError_t launch_pcr_c(const ZArgs &a, hipStream_t s)
     if (a.items) {
         // batched: one block per item, column lengths vary inside the launch (every solve's
         // 16 * SX * SY * sizeof(R) is checked below 4 GiB by the caller)
-        grid = dim3((unsigned)a.nitems);
+        grid = dim3((unsigned)(a.nitems + a.nth));
         full = false;
     } else if (16.0 * a.SX * a.SY * sizeof(R) >= 4294967296.0) {
         // staged tiles address rows from a uniform base; lane offsets span 16 rows
         return hipErrorInvalidValue;
+    }
+    if (a.nth && J <= 8) {
+        // their blocks would cost the launches of small grids, where there are hardly such columns, 0.4 us
+        ZArgs b = a;
+        b.nth = 0;
+        const hipError_t e = launch_pcr_c<R, J, CPB>(b, s);
+        b.items = nullptr;
+        return e != hipSuccess ? e : launch_zthomas_f64(b, a.th, a.th_tab, a.nth, s);
+    }
+    if (a.nth) {
+        if (sizeof(R) != 8 || CPB != 16 || !a.th || !a.th_tab) return hipErrorInvalidValue;
+        if (!a.items) grid.y += (a.nth + grid.x - 1) / grid.x;
     }
     constexpr size_t lds = ztile_bytes_cyclic<R, J, CPB>();
 #define PP_ZL(F, O)                                                                                            \
@@ -58,8 +70,9 @@ static hipError_t launch_pcr_c(const ZArgs &a, hipStream_t s)
 bool zsolve_supported_f64(int nz) { return nz >= 4 && nz <= 16 * 32; }
 
 #define PPJ32(R)                                                                                        \
-    PPJ(R, 1) PPJ(R, 2) PPJ(R, 3) PPJ(R, 4) PPJ(R, 5) PPJ(R, 6) PPJ(R, 7) PPJ(R, 8) PPJ(R, 9) PPJ(R, 10) \
-    PPJ(R, 11) PPJ(R, 12) PPJ(R, 13) PPJ(R, 14) PPJ(R, 15) PPJ(R, 16) PPJ(R, 17) PPJ(R, 18)            \
+    PPJ(R, 1) PPJ(R, 2) PPJ(R, 3) PPJ(R, 4) PPJ(R, 5) PPJ(R, 6) PPJ(R, 7) PPJ(R, 8) PPJ9_32(R)
+#define PPJ9_32(R)                                                                                     \
+    PPJ(R, 9) PPJ(R, 10) PPJ(R, 11) PPJ(R, 12) PPJ(R, 13) PPJ(R, 14) PPJ(R, 15) PPJ(R, 16) PPJ(R, 17) PPJ(R, 18)            \
     PPJ(R, 19) PPJ(R, 20) PPJ(R, 21) PPJ(R, 22) PPJ(R, 23) PPJ(R, 24) PPJ(R, 25) PPJ(R, 26)            \
     PPJ(R, 27) PPJ(R, 28) PPJ(R, 29) PPJ(R, 30) PPJ(R, 31) PPJ(R, 32)
 #define PPJ(R, v) \
@@ -68,7 +81,8 @@ bool zsolve_supported_f64(int nz) { return nz >= 4 && nz <= 16 * 32; }
 hipError_t launch_zsolve_pcr_f64(int nz, const ZArgs &a, hipStream_t s)
 {
     switch ((nz + 15) / 16) {
-        PPJ32(double)
+        // (columns of up to 64 rows: launch_ztwist)
+        PPJ(double, 5) PPJ(double, 6) PPJ(double, 7) PPJ(double, 8) PPJ9_32(double)
     default: return launch_zsolve_long_f64(nz, a, s);
     }
 }
@@ -131,114 +145,12 @@ hipError_t launch_zsolve_pcr_f32(int nz, const ZArgs &a, hipStream_t s)
 
 namespace pp {
 
-// The reference's Thomas sweep (thomasLowMem, src/triDiag.cpp:1693-1822, not the pinned
-// branch) on one listed FP64 column per block.  Its factors depend only on the column's
-// eigenvalue and end rows, so the host computes them in the reference's order (bet_0 = b0,
-// tmp_j = 1 / bet_{j-1}, bet_j = eig - tmp_j, the last row bn - tmp) and hands over
-// tab = {1 / bet_j, tmp_j} per column.  The two sweeps are then linear recurrences in the
-// column's values -- forward x_j = (x_j - x_{j-1}) / bet_j, backward x_j -= tmp_{j+1} x_{j+1}
-// -- which one wave runs as a scan: each lane composes the affine maps of its contiguous chunk
-// of rows (C = ceil(nz / 64) <= 16), a Kogge-Stone scan across the 64 lanes gives each lane the
-// value entering its chunk, and the lane sweeps its rows (about 40 dependent steps per sweep
-// instead of nz).  Against the serial sweep this reassociation moves a column by a few 1e-14
-// of its largest value; the PCR steps it replaces lose ~3e-12 on such columns.  The PCR
-// kernel left these columns untouched (|eig + 2| below its tau).
 constexpr int ZTH_CMAX = 16;  // rows per lane: nz <= 64 * 16
 
+// the Thomas columns by themselves: behind the z solvers that have no blocks for them (k_zsolve has)
 __global__ void __launch_bounds__(64) k_zthomas64(ZArgs a0, const ZThomasItem *items, const double *tab)
 {
-    constexpr int W = 64;
-    const ZThomasItem it = items[blockIdx.x];
-    ZArgs a = a0;
-    if (it.solve >= 0) {
-        // batched: the member's field (its z tiles), sizes
-        const ZSolve sv = a0.solves[it.solve];
-        a.data = reinterpret_cast<double *>(a0.data) + sv.offset;
-        a.SX = sv.SX;
-        a.SY = sv.SY;
-        a.nz = sv.nz;
-    }
-    const int n = a.nz;
-    // element j of the column: in place (stride SX*SY) or in its z tile (stride W)
-    long zs = (long)a.SX * a.SY;
-    long off = (long)it.sy * a.SX + it.sx;
-    if (a.tiled) {
-        const int Wt = a.tile_w;
-        const int rows = a.tile_rows ? a.tile_rows : (n + 15) / 16 * 16;
-        off = (((long)(it.sx / Wt) * a.SY + it.sy) * rows) * Wt + it.sx % Wt;
-        zs = Wt;
-    }
-    double *data = reinterpret_cast<double *>(a.data);
-    const double *ib = tab + it.toff, *tp = ib + n;
-    const int L = threadIdx.x, C = (n + W - 1) / W, j0 = L * C;
-    double x[ZTH_CMAX], g[ZTH_CMAX], q[ZTH_CMAX];
-#pragma unroll
-    for (int k = 0; k < ZTH_CMAX; k++) {
-        const int j = j0 + k;
-        const bool in = k < C && j < n;
-        x[k] = in ? data[off + (long)j * zs] : 0.0;
-        g[k] = in ? ib[j] : 0.0;
-        q[k] = (in && j + 1 < n) ? tp[j + 1] : 0.0;
-    }
-    // forward: x_j = -g_j x_{j-1} + x_j g_j, composed over the chunk, scanned in lane order
-    double A = 1.0, B = 0.0;
-#pragma unroll
-    for (int k = 0; k < ZTH_CMAX; k++) {
-        if (k < C && j0 + k < n) {
-            const double m = -g[k];
-            B = m * B + x[k] * g[k];
-            A = m * A;
-        }
-    }
-    for (int s = 1; s < W; s <<= 1) {
-        const double Au = __shfl_up(A, s, W), Bu = __shfl_up(B, s, W);
-        if (L >= s) {
-            B = A * Bu + B;
-            A = A * Au;
-        }
-    }
-    double v = __shfl_up(B, 1, W);
-    if (L == 0) v = 0.0;
-#pragma unroll
-    for (int k = 0; k < ZTH_CMAX; k++) {
-        if (k < C && j0 + k < n) {
-            v = (x[k] - v) * g[k];
-            x[k] = v;
-        }
-    }
-    // backward: x_j = -tmp_{j+1} x_{j+1} + x_j, composed over the chunk from its last row,
-    // scanned in reverse lane order
-    A = 1.0;
-    B = 0.0;
-#pragma unroll
-    for (int k = ZTH_CMAX - 1; k >= 0; k--) {
-        if (k < C && j0 + k < n) {
-            const double m = -q[k];
-            B = m * B + x[k];
-            A = m * A;
-        }
-    }
-    for (int s = 1; s < W; s <<= 1) {
-        const double Ad = __shfl_down(A, s, W), Bd = __shfl_down(B, s, W);
-        if (L + s < W) {
-            B = A * Bd + B;
-            A = A * Ad;
-        }
-    }
-    v = __shfl_down(B, 1, W);
-    if (L == W - 1) v = 0.0;
-#pragma unroll
-    for (int k = ZTH_CMAX - 1; k >= 0; k--) {
-        if (k < C && j0 + k < n) {
-            v = x[k] - q[k] * v;
-            x[k] = v;
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < ZTH_CMAX; k++) {
-        const int j = j0 + k;
-        if (k < C && j < n) data[off + (long)j * zs] = x[k];
-    }
+    zthomas_column<ZTH_CMAX>(a0, items[blockIdx.x], tab);
 }
 
 hipError_t launch_zthomas_f64(const ZArgs &a, const ZThomasItem *items, const double *tab, int nitems, hipStream_t s)
