@@ -901,16 +901,26 @@ constexpr int line_threads(int M, int AX)
     X(4) X(6) X(8) X(10) X(12) X(14) X(16) X(20) X(24) X(28) X(32) X(40) X(48) X(56) X(64) X(80) X(96) X(112) \
         X(128) X(160) X(192) X(224) X(256) X(320) X(384) X(448) X(512)
 
-// Alternative launch shape of the FP64 transforms (chosen per stage by the autotuner): twice
+// Second launch shape of the FP64 transforms: twice
 // the threads per line, half the elements per thread -- fewer registers and more waves in
 // flight for one more radix pass (e.g. M = 256: 4 x 4 x 4 x 4 instead of 8 x 8 x 4); offered
-// where the plan grows by at most one pass, 0 elsewhere
+// where the plan grows by at most one pass, 0 elsewhere.  The one that is not the default
+// (line_wide) is the alternative, chosen per stage by the autotuner
 constexpr int line_threads_alt(int M)
 {
     const int T = line_threads(M, 0);
     if (T == 0 || M / T < 8 || !plan_ok(M, M / (2 * T))) return 0;
     return make_plan(M, M / (2 * T)).n <= make_plan(M, M / T).n + 1 ? 2 * T : 0;
 }
+
+// FP64 lines whose default is that second shape: up to 80 points, where the first has 1 to 4
+// threads a line and 8 KB or more of code run once, and 128-point rows along x.  Both, us, forward / inverse:
+//   y, 512 columns x 512 planes   16 points 22.2 / 22.8 : 16.5 / 16.4   24  33.2 / 33.7 : 21.8 / 23.1
+//                                 48 points 43.7 / 61.3 : 36.8 / 39.1   80  88.0 / 131 : 74.7 / 67.1
+//   x, 32 x 64 rows               48 points 11.1 / 11.1 : 9.0 / 9.1     64   8.6 /  9.0 :  7.2 /  7.4
+//   x, 128 points                 128 x 64 rows 10.2 / 12.7 : 9.2 / 11.1, 512 x 512 rows 104 / 102 : 107 / 87
+// At 256 and 512 points the shapes are within 5 % of each other; y lines of 128 points within 4 %.
+constexpr bool line_wide(int M, int AX) { return line_threads_alt(M) > 0 && (M <= 40 || (M == 64 && AX == 0)); }
 
 template <typename R, int M, int AX, int T = line_threads(M, AX)>
 constexpr int line_lines()
@@ -1029,7 +1039,7 @@ hipError_t launch_line_kind(int form, int N, int AX, int FWD, const LineArgs &a,
 {
     switch (form) {
     case FORM_F64:
-        if (a.variant) {
+        if ((a.variant != 0) != line_wide(N / 2, AX)) {
             if (AX == 0) return FWD ? launch_line_sz<double, double, double, 0, 1, KIND, 1>(N, a, s)
                                     : launch_line_sz<double, double, double, 0, 0, KIND, 1>(N, a, s);
             return FWD ? launch_line_sz<double, double, double, 1, 1, KIND, 1>(N, a, s)
@@ -1091,24 +1101,24 @@ inline bool line_tiled32_f32_variant(int N)
     }
 }
 
+template <int M>
+constexpr int alt_lines_x()
+{
+    if constexpr (line_threads_alt(M) > 0) return line_lines<double, M, 0, line_threads_alt(M)>();
+    else return 0;
+}
+
 // lines (x) or columns (y) per block of the launch for line length N, precision R
 template <typename R>
 inline int line_block_lines(int N, int AX)
 {
     switch (N / 2) {
 #define PPM(m) \
-    case m: return AX == 0 ? line_lines<R, m, 0>() : line_lines<R, m, 1>();
+    case m: return AX == 1 ? line_lines<R, m, 1>() : sizeof(R) == 8 && line_wide(m, 0) ? alt_lines_x<m>() : line_lines<R, m, 0>();
         PP_FFT_LENGTHS(PPM)
 #undef PPM
     default: return 0;
     }
-}
-
-template <int M>
-constexpr int alt_lines_x()
-{
-    if constexpr (line_threads_alt(M) > 0) return line_lines<double, M, 0, line_threads_alt(M)>();
-    else return 0;
 }
 
 // lines (x) or columns (y) per block of the alternative FP64 shape (y keeps the default's)
@@ -1117,7 +1127,7 @@ inline int line_block_lines_alt(int N, int AX)
     if (AX == 1) return line_block_lines<double>(N, 1);
     switch (N / 2) {
 #define PPM(m) \
-    case m: return alt_lines_x<m>();
+    case m: return line_wide(m, 0) ? line_lines<double, m, 0>() : alt_lines_x<m>();
         PP_FFT_LENGTHS(PPM)
 #undef PPM
     default: return 0;
