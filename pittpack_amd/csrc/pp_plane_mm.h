@@ -36,14 +36,19 @@ inline int plane_waves(int nx, int ny, int kx, int ky)
 
 // Planes these kernels take (FP64 form), all members of a batch by the same rule as a single solve.
 // Measured against the line kernels, a solve / a batch of hundreds of members (us):
-//   folded kinds up to 32 points   24x20x18 15.8 : 24.7 / 301 : 305    32x32x32 18.5 : 25.6 / 304 : 320
-//   without a compiled plan        33x33x16 21.6 : 24.6                63x63x63 26.8 : 29.4 / 454 : 686
-//   not: periodic, compiled        32x32x16 22.9 : 27.1 / 388 : 290    (17 outputs pad to 32)
-//   not: compiled past 32          48x48x16 25.2 : 37.3 / 525 : 481    64x64x64 29.9 : 33.4 / 501 : 465
-//   not: planes of < 96 points     8x8x32 20 : 22 / 358 : 238          10x12x16 - / 230 : 266
+//   DD, NN up to 32 points         20x20x16 14.4 : 22.9, 24x20x18 - / 185 : 198, 32x32x16 14.6 : 17.2 / 232 : 214
+//   ND, DN up to 28 points         28x28x16 16.2 : 24.7, but 32x32x16 16.2 : 15.6, 32x16x100 - / 304 : 262
+//   without a compiled plan        33x33x16 21.6 : 24.6, 63x63x63 26.8 : 29.4 / 366 : 596
+//   not: periodic, compiled        32x32x16 22.9 : 27.1 / 388 : 290 then, the lines since 192 (17 outputs pad to 32)
+//   not: compiled past 32          48x48x48 - / 525 : 481 then, the lines since 320; 64x64x64 - / 501 : 465
+//   not: planes of < 96 points     8x8x32 20 : 22 / 358 : 238, but 10x12x16 - / 189 : 229
 // A batch fills the chip, so there the products' padding counts; a single solve does not.
 constexpr int kPlaneMax = 64;
-inline bool plane_axis(int n, int kind) { return n <= kPlaneMax && (!line_compiled(n) || (n <= 32 && kind != KIND_PP)); }
+inline bool plane_axis(int n, int kind)
+{
+    const int fam = mm_family(kind);
+    return n <= kPlaneMax && (!line_compiled(n) || n <= (fam == 0 ? 32 : fam == 1 ? 28 : 0));
+}
 inline bool mm_plane(int nx, int ny, int kx, int ky)
 {
     return plane_axis(nx, kx) && plane_axis(ny, ky) && nx * ny >= 96 && plane_jobs(nx, ny, kx, ky) <= kPlaneWaves;
