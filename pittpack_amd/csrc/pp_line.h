@@ -920,6 +920,8 @@ constexpr int line_threads_alt(int M)
 //   x, 32 x 64 rows               48 points 11.1 / 11.1 : 9.0 / 9.1     64   8.6 /  9.0 :  7.2 /  7.4
 //   x, 128 points                 128 x 64 rows 10.2 / 12.7 : 9.2 / 11.1, 512 x 512 rows 104 / 102 : 107 / 87
 // At 256 and 512 points the shapes are within 5 % of each other; y lines of 128 points within 4 %.
+// The FP32 lines of the mixed form take it at the same lengths (a whole mixed solve of 80x80x80 204 : 167,
+// 48x512x512 740 : 658, 128x128x128 149 : 145).
 constexpr bool line_wide(int M, int AX) { return line_threads_alt(M) > 0 && (M <= 40 || (M == 64 && AX == 0)); }
 
 template <typename R, int M, int AX, int T = line_threads(M, AX)>
@@ -980,12 +982,14 @@ hipError_t launch_line_blocks(const LineArgs &a, hipStream_t s)
 template <typename TIn, typename TOut, typename R, int M, int AX, int FWD, int KIND, int V = 0>
 hipError_t launch_line_cfg(const LineArgs &a, hipStream_t s)
 {
-    constexpr int T = V ? line_threads_alt(M) : line_threads(M, AX);
+    // FP32 lines take the shape that is FP64's default, with the first one's lines per block
+    constexpr bool W32 = sizeof(R) == 4 && line_wide(M, AX);
+    constexpr int T = V || W32 ? line_threads_alt(M) : line_threads(M, AX);
     if constexpr (T == 0) {
         return hipErrorInvalidValue;
     } else {
         // y keeps the default's columns per block in either shape (the z-tile width)
-        constexpr int LINES = (V && AX == 1) ? line_lines<R, M, AX>() : line_lines<R, M, AX, T>();
+        constexpr int LINES = (V && AX == 1) || W32 ? line_lines<R, M, AX>() : line_lines<R, M, AX, T>();
         // the 16-column FP64 blocks of 1024-point y lines (one block per CU) pay off where they
         // write or read whole z-tile rows (two 8-column blocks per CU, each writing half of
         // every tile row, and the same block loading a second plane's columns while it

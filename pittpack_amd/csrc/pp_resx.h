@@ -329,7 +329,8 @@ __global__ void __launch_bounds__(T *LINES, (resx_waves<M, T, LINES, BATCH>())) 
 template <int M, int KIND, int SRC>
 hipError_t launch_resx_cfg(const LineArgs &a, const ResArgs &r, const ResArgs *rsolves, hipStream_t s)
 {
-    constexpr int T = line_threads(M, 0);
+    // the unfused transform's shape
+    constexpr int T = line_wide(M, 0) ? line_threads_alt(M) : line_threads(M, 0);
     if constexpr (T == 0) {
         return hipErrorInvalidValue;
     } else {
