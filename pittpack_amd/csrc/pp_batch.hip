@@ -120,6 +120,9 @@ void BatchCore::plan_lanes(std::initializer_list<std::vector<HostClass> *> stage
     }
 }
 
+// periodic z lines without a compiled plan as dense products, as the single-solve handle decides
+static bool zlines_dense(const SolveSetup &g) { return mm_serves(g.nz, KIND_PP, 1, (long)g.nx * g.ny); }
+
 TableCache::~TableCache()
 {
     for (auto &kv : t_)
@@ -156,9 +159,9 @@ int TableCache::get_mm(int N, int kind, const double *&mm, const double *&mmi)
     return PP_SUCCESS;
 }
 
-int TableCache::get(int N, int kind, int axis, AxisDev &out)
+int TableCache::get(int N, int kind, bool dense, AxisDev &out)
 {
-    if (kind >= 0 && mm_serves(N, kind, axis)) {
+    if (dense) {
         out = AxisDev{};
         return get_mm(N, kind, out.mm, out.mmi);
     }
@@ -228,13 +231,16 @@ long long BatchCore::points() const
 template <typename R>
 int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
 {
-    std::map<std::pair<int, int>, std::vector<LineItem>> cls;
+    std::map<std::array<int, 3>, std::vector<LineItem>> cls;  // {length, kind, dense}
+    auto is_dense = [&](const SolveSetup &g) {
+        return mm_serves(axis == 0 ? g.nx : g.ny, g.kind[axis], axis, (long)(axis == 0 ? g.ny : g.nx) * g.nz);
+    };
     // dense-product classes: launch shape from the class's units of 16 lines / columns
     std::map<std::pair<int, int>, long> units;
     for (const BatchMember &m : mem) {
         if (m.plane) continue;
         const int N = axis == 0 ? m.g.nx : m.g.ny;
-        if (mm_serves(N, m.g.kind[axis], axis))
+        if (is_dense(m.g))
             units[{N, m.g.kind[axis]}] += axis == 0 ? ((long)m.g.ny * m.g.nz + 15) / 16 : (long)((m.g.nx + 15) / 16) * m.g.nz;
     }
     std::map<std::pair<int, int>, MmPlan> plans;
@@ -243,12 +249,12 @@ int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
         if (mem[m].plane) continue;
         const SolveSetup &g = mem[m].g;
         const int N = axis == 0 ? g.nx : g.ny;
-        const auto pl = plans.find({N, g.kind[axis]});
-        const int group = pl == plans.end() ? 1 : pl->second.units;
-        const int lines = line_lines_any<R>(N, g.kind[axis], axis) * (axis == 0 ? group : 1);
+        const bool dense = is_dense(g);
+        const int group = dense ? plans.at({N, g.kind[axis]}).units : 1;
+        const int lines = line_lines_any<R>(N, dense, axis) * (axis == 0 ? group : 1);
         const int planes = axis == 1 ? group : 1;  // y: consecutive planes per block
         if (lines <= 0) return PP_UNSUPPORTED_SIZE;
-        auto &items = cls[{N, g.kind[axis]}];
+        auto &items = cls[{N, g.kind[axis], dense}];
         if (axis == 0) {
             const long nl = (long)g.ny * g.nz;
             for (long bx = 0; bx < (nl + lines - 1) / lines; bx++) items.push_back({m, (int)bx, 0});
@@ -261,13 +267,12 @@ int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
     out.clear();
     for (auto &kv : cls) {
         HostClass c;
-        c.key = kv.first.first;
-        c.kind = kv.first.second;
-        c.axis = axis;
+        c.key = kv.first[0];
+        c.kind = kv.first[1];
+        c.dense = kv.first[2] != 0;
         c.nitems = (int)kv.second.size();
         c.li = std::move(kv.second);
-        const auto pl = plans.find(kv.first);
-        if (pl != plans.end()) c.mm = pl->second;
+        if (c.dense) c.mm = plans.at({c.key, c.kind});
         if (sizeof(R) == 8 && axis == 0 && line_has_variant(c.key)) {
             // x blocks of the alternative shape hold a different number of lines
             const int la = line_block_lines_alt(c.key, 0);
@@ -541,7 +546,7 @@ int BatchCore::plan()
                 HostClass h;
                 h.key = c.key;
                 h.kind = c.kind;
-                h.axis = c.axis;
+                h.dense = c.dense;
                 h.mm = c.mm;
                 h.fused = f != 0;
                 for (const LineItem &it : c.li)
@@ -661,19 +666,20 @@ int BatchCore::bind(char *base, TableCache *tc)
     for (auto *v : {&lx_, &ly_})
         for (HostClass &h : *v) {
             AxisDev t;
-            if ((rc = tc->get(h.key, h.kind, h.axis, t))) return rc;
-            tabs_[{h.key, h.kind, h.axis}] = t;
+            if ((rc = tc->get(h.key, h.kind, h.dense, t))) return rc;
+            tabs_[{h.key, h.kind, h.dense}] = t;
         }
     // periodic z: line tables of length nz
     for (HostClass &h : lzp_) {
         AxisDev t;
-        if ((rc = tc->get(h.key, -1, 1, t))) return rc;
-        tabs_[{h.key, -1, 1}] = t;
+        if ((rc = tc->get(h.key, -1, false, t))) return rc;
+        tabs_[{h.key, -1, 0}] = t;
     }
     for (int m : zpl_) {
         AxisDev t;
-        if ((rc = tc->get(mem[m].g.nz, KIND_PP, 1, t))) return rc;
-        tabs_[{mem[m].g.nz, KIND_PP, 1}] = t;
+        const bool dense = zlines_dense(mem[m].g);
+        if ((rc = tc->get(mem[m].g.nz, KIND_PP, dense, t))) return rc;
+        tabs_[{mem[m].g.nz, KIND_PP, dense}] = t;
     }
     if (precision == 1) {
         d_sums_ = (double *)(base + o_sums_);
@@ -802,7 +808,7 @@ int BatchCore::launch_class(hipStream_t s, const HostClass &c, int form, int axi
     {
         const int v = (form == FORM_F64 && line_has_variant(c.key)) ? (force_var >= 0 ? force_var : c.var[fwd ? 0 : 1]) : 0;
         const bool alt_items = v && axis == 0;
-        const AxisDev &t = tabs_.at({c.key, c.kind, c.axis});
+        const AxisDev &t = tabs_.at({c.key, c.kind, c.dense});
         LineArgs a{};
         a.variant = v;
         a.mm = t.mm;
@@ -944,8 +950,8 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
         ZPerArgs zp{};
         zp.data = pdata;
         zp.nz = c.key;
-        zp.tw = tabs_.at({c.key, -1, 1}).tw;
-        zp.A = tabs_.at({c.key, -1, 1}).A;
+        zp.tw = tabs_.at({c.key, -1, 0}).tw;
+        zp.A = tabs_.at({c.key, -1, 0}).A;
         zp.c2 = d_zc2_ + zc2_off_.at(c.key);
         zp.pinned_zero = f32 ? 1 : 0;
         zp.items = (const ZItem *)c.d_items;
@@ -955,7 +961,7 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
     }
     for (int m : zpl_) {
         const SolveSetup &g = mem[m].g;
-        const AxisDev &t = tabs_.at({g.nz, KIND_PP, 1});
+        const AxisDev &t = tabs_.at({g.nz, KIND_PP, zlines_dense(g)});
         const long off = mem[m].offset;
         void *data = f32 ? (void *)(d_w + off) : (void *)(d_sol + off);
         ZPerArgs zp{};
@@ -1134,7 +1140,7 @@ int BatchCore::run_mixed(hipStream_t s, Marks *mk)
         rc = run_stage(s, lxc_.size(), [&]() -> int {
             for (const HostClass &c : lxc_) {
                 if (c.fused) {
-                    const AxisDev &t = tabs_.at({c.key, c.kind, c.axis});
+                    const AxisDev &t = tabs_.at({c.key, c.kind, c.dense});
                     LineArgs a{};
                     a.in = d_w;
                     a.out = d_w;

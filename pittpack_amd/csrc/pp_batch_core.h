@@ -32,8 +32,8 @@ struct AxisDev {
 class TableCache {
   public:
     ~TableCache();
-    // tables of lines of length N along x (axis 0) or across it; kind -1: a compiled plan's
-    int get(int N, int kind, int axis, AxisDev &out);
+    // tables of lines of length N (dense: as products of `kind`)
+    int get(int N, int kind, bool dense, AxisDev &out);
     // dense-product matrices of (N, kind)
     int get_mm(int N, int kind, const double *&mm, const double *&mmi);
 
@@ -125,7 +125,8 @@ class BatchCore {
 
   private:
     struct HostClass {
-        int key = 0, kind = 0, axis = 0, nitems = 0;
+        int key = 0, kind = 0, nitems = 0;
+        bool dense = false;  // line classes: dense products (mm), not a plan or convolution
         MmPlan mm{};  // dense-product line classes: the launch shape
         std::vector<LineItem> li;
         std::vector<ZItem> zi;
@@ -207,7 +208,7 @@ class BatchCore {
     // region layout (byte offsets)
     size_t o_zth_ = 0, o_zth_tab_ = 0, o_u0_ = 0, o_cacc_ = 0, o_zc2_ = 0, o_smt_ = 0, o_rhs_ = 0, o_sol_ = 0, o_tiles_ = 0, o_w_ = 0, o_lam_ = 0, o_dtab_ = 0, o_ls_ = 0, o_zs_ = 0, o_sums_ = 0, o_plane_ = 0,
            o_upart_ = 0, o_fix_ = 0, o_m00_ = 0, o_res_ = 0, o_ritems_ = 0, o_rpitems_ = 0;
-    std::map<std::array<int, 3>, AxisDev> tabs_;  // {length, kind, axis}; kind -1: periodic z
+    std::map<std::array<int, 3>, AxisDev> tabs_;  // {length, kind, dense}; kind -1: periodic z
     // device pointers of the tables
     double *d_lam_ = nullptr, *d_dtab_ = nullptr, *d_sums_ = nullptr, *d_plane_ = nullptr, *d_upart_ = nullptr;
     LineSolve *d_ls_ = nullptr;

@@ -509,12 +509,19 @@ hipError_t launch_mm_tables(double *out, const double *oct, int N, int kind, hip
 //   y, folded kinds:   331: 152 / 436   602: 268 / 517   750: 260 / 440  1000: 318 / 361
 //   x, quarter-wave:   331: 227 / 262   402: 335 / 223
 //   y, quarter-wave:   331: 227 / 437   509: 282 / 315   602: 514 / 513
+// (x: 440 to 512 folded and 280 up quarter-wave are no faster, and the matrix cores' power slows the rest
+// of a solve by 3 %).  A long line's products are a chain of loads from L2 whatever the number of lines,
+// which the convolution's few passes beat while lines are few -- 1024 / 4096 lines, x then y (us):
+//   101: 8.5 9.1, 7.8 9.1 / 9.0 11.6, 10.9 12.1    201: 12.0 13.8, 10.8 13.0 / 9.2 17.7, 12.0 21.4
+//   401: 25 30, 22 25 / 14 34, 15 45               601: 45 50, 39 45 / 22 58, 27 87
 constexpr int kMmMaxN = 1024;
-inline bool mm_serves(int n, int kind, int axis)
+inline bool mm_serves(int n, int kind, int axis, long lines)
 {
     if (line_compiled(n) || n < 2) return false;
-    if (mm_family(kind) == 1) return n <= (axis == 0 ? 340 : 512);
-    return n <= (axis == 0 ? 620 : kMmMaxN);
+    const bool quarter = mm_family(kind) == 1;
+    if (lines < (n <= (axis == 1 && !quarter ? 208 : 112) ? 0 : n <= 256 ? 2048 : 3072)) return false;
+    if (quarter) return n <= (axis == 0 ? 280 : 512);
+    return axis == 0 ? n <= 440 || (n > 512 && n <= 620) : n <= kMmMaxN;
 }
 
 // Shape of a launch over `nunits` units of 16 lines / columns.  Two units per wave halve the
@@ -578,9 +585,9 @@ hipError_t launch_line_mm_cfg(const LineArgs &a, hipStream_t s)
 // lines (x) or columns (y) per block of whichever launch serves length N (dense x launches take
 // whole multiples of it, mm_plan)
 template <typename R>
-inline int line_lines_any(int N, int kind, int AX)
+inline int line_lines_any(int N, bool dense, int AX)
 {
-    if (mm_serves(N, kind, AX)) return 16;
+    if (dense) return 16;
     return line_compiled(N) ? line_block_lines<R>(N, AX) : bs_block_lines<R>(N, AX);
 }
 

@@ -60,10 +60,15 @@ bool same_key(const Resident &r, int nx, int ny, int nz, const char *bc, const d
            std::memcmp(r.bc, bc, 6) == 0 && std::memcmp(r.X, X, sizeof(r.X)) == 0;
 }
 
-// lines of axis a (0 x, 1 y) whose matrices the handle would have
+// lines of axis a (0 x, 1 y; 2 periodic z) that are dense products, or whose matrices the handle would have
+bool mm_dense(const SolveSetup &g, int a)
+{
+    if (a == 2) return mm_serves(g.nz, KIND_PP, 1, (long)g.nx * g.ny);
+    return mm_serves(a == 0 ? g.nx : g.ny, g.kind[a], a, (long)(a == 0 ? g.ny : g.nx) * g.nz);
+}
 bool mm_lines(const SolveSetup &g, int a)
 {
-    return mm_serves(a == 0 ? g.nx : g.ny, g.kind[a], a) || mm_plane(g.nx, g.ny, g.kind[0], g.kind[1]);
+    return mm_dense(g, a) || mm_plane(g.nx, g.ny, g.kind[0], g.kind[1]);
 }
 
 // lay the tables of `g` out in g_host (offsets into r); false if they exceed kScratchDoubles.
@@ -82,7 +87,7 @@ bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
     for (int a = 0; a < 2; a++) {
         if (dense && mm_lines(g, a)) {
             r.oct[a] = take(mm_octant_size(n[a]));
-            if (mm_serves(n[a], g.kind[a], a)) continue;
+            if (mm_dense(g, a)) continue;
         }
         const AxisTableSizes z = axis_table_sizes(n[a]);
         for (int i = 0; i < 5; i++) r.tab[a][i] = take(z.n[i]);
@@ -97,7 +102,7 @@ bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
         if (zc) {
             r.ztw = take(zs.n[0]);
             r.zA = take(zs.n[1]);
-        } else if (dense && mm_serves(g.nz, KIND_PP, 1)) {
+        } else if (dense && mm_dense(g, 2)) {
             r.oct[2] = take(mm_octant_size(g.nz));
         } else {
             for (int i = 0; i < 5; i++) r.ztab[i] = take(zs.n[i]);
@@ -109,13 +114,13 @@ bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
     if (dense) {
         for (int a = 0; a < 2; a++)
             if (mm_lines(g, a)) r.mm[a] = take(mm_tables_size(n[a], g.kind[a]));
-        if (g.zper && !zc && mm_serves(g.nz, KIND_PP, 1)) r.mm[2] = take(mm_tables_size(g.nz, KIND_PP));
+        if (g.zper && !zc && mm_dense(g, 2)) r.mm[2] = take(mm_tables_size(g.nz, KIND_PP));
     }
     if (o > kScratchDoubles) return false;
     std::memset(g_host, 0, r.used * sizeof(double));
     for (int a = 0; a < 2; a++) {
         if (r.mm[a]) fill_mm_octant(n[a], g_host + r.oct[a]);
-        if (!r.mm[a] || !mm_serves(n[a], g.kind[a], a))
+        if (!r.mm[a] || !mm_dense(g, a))
             fill_axis_tables(n[a], g_host + r.tab[a][0], g_host + r.tab[a][1], g_host + r.tab[a][2],
                              g_host + r.tab[a][3], g_host + r.tab[a][4]);
     }
