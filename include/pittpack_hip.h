@@ -53,7 +53,8 @@ enum {
     /* value k > 0: record per-stage HIP events for the last k solves (pp_get_stage_times);
      * 0 switches timing off */
     PP_OPT_TIMING = 2,
-    /* z solver: 0 = PCR across 16 lanes then Thomas per lane (cyclic rows);
+    /* z solver: 0 = PCR across 16 lanes then Thomas per lane (cyclic rows), short columns by
+     * sweeps from both ends;
      *           1 = partitioned Thomas, contiguous rows per lane, cross-lane scans;
      *           2 = multigrid V-cycles (the reference's MultiGrid alternative) to a
      *               max-norm residual of PP_OPT_MG_TOL * max|rhs| (default 1e-16), or until

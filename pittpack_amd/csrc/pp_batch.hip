@@ -1477,7 +1477,10 @@ int pp_batch_solve(pp_batch b)
         // replay the graph from now on
         hipGraph_t g = nullptr;
         BatchLanes lanes;  // become branches of the graph
-        if (b->core.points() >= BatchLanes::kMinPoints && lanes.create() == PP_SUCCESS) b->core.lanes = &lanes;
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;  // a caller's capture: nothing is created in it
+        if (b->core.points() >= BatchLanes::kMinPoints && hipStreamIsCapturing(b->stream, &cs) == hipSuccess &&
+            cs == hipStreamCaptureStatusNone && lanes.create() == PP_SUCCESS)
+            b->core.lanes = &lanes;
         const hipError_t eb = hipStreamBeginCapture(b->stream, hipStreamCaptureModeRelaxed);
         const int rc = eb == hipSuccess ? b->core.run(b->stream, nullptr) : PP_HIP_ERROR;
         const hipError_t ec = eb == hipSuccess ? hipStreamEndCapture(b->stream, &g) : eb;

@@ -191,7 +191,7 @@ class BatchCore {
     // FP64 members with 513..1024-row columns: the long-column kernel, one launch each
     std::vector<int> zlong_;
     // FP64: nearly singular columns of the PCR classes' members, solved by the reference's
-    // Thomas sweeps after the z classes, and their factor tables
+    // Thomas sweeps in blocks of their z class' launch, and their factor tables
     std::vector<ZThomasItem> zth_;
     std::vector<double> zth_tab_;
     std::vector<int4> fix_;

@@ -54,7 +54,7 @@ struct pp_solver {
     int mg_cycles = 200;                        // multigrid z solver: V-cycle limit
     double mg_tol = 1e-16;                      //   and relative max-norm residual tolerance
     // FP64 form: columns with |eig+2| below zthomas_tau (not pinned) are solved by the
-    // reference's Thomas sweeps after the PCR kernel (0: off); their list, built with the tables
+    // reference's Thomas sweeps beside the PCR blocks (0: off); their list, built with the tables
     double zthomas_tau = 1e-3;
     pp::ZThomasItem *d_zthomas = nullptr;
     double *d_zthomas_tab = nullptr;  // their Thomas factors (zthomas_factors), 2 nz per column

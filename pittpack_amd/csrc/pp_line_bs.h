@@ -1,6 +1,7 @@
 // pp_line_bs.h -- line transforms of any length N (2 <= N <= 1024) for CDNA4 (gfx950):
 // lengths the compiled Stockham plans of pp_line.h do not cover (odd N, N/2 with a prime
-// factor above 7, N/2 not in the compiled list).
+// factor above 7, N/2 not in the compiled list), where pp_line_mm.h's dense products are not
+// faster (mm_serves: long lines, or few of them).
 //
 // The reference gets every length from FFTW / cuFFT plans of any n (src/poissonCPU.cpp:56,87,
 // 162,211, src/poissonGPU.cpp:13,37) and SignalProc handles odd sizes
