@@ -514,12 +514,14 @@ hipError_t launch_mm_tables(double *out, const double *oct, int N, int kind, hip
 // which the convolution's few passes beat while lines are few -- 1024 / 4096 lines, x then y (us):
 //   101: 8.5 9.1, 7.8 9.1 / 9.0 11.6, 10.9 12.1    201: 12.0 13.8, 10.8 13.0 / 9.2 17.7, 12.0 21.4
 //   401: 25 30, 22 25 / 14 34, 15 45               601: 45 50, 39 45 / 22 58, 27 87
+//   x, quarter-wave (twice the products)  67: 9.7 10.2 / 9.0 11.1    27, 1280 lines: a solve 33.1 / 32.2
 constexpr int kMmMaxN = 1024;
 inline bool mm_serves(int n, int kind, int axis, long lines)
 {
     if (line_compiled(n) || n < 2) return false;
     const bool quarter = mm_family(kind) == 1;
-    if (lines < (n <= (axis == 1 && !quarter ? 208 : 112) ? 0 : n <= 256 ? 2048 : 3072)) return false;
+    const int any = axis == 1 ? (quarter ? 112 : 208) : quarter ? 0 : 112;  // up to here any number of lines
+    if (n > any && lines < (n <= 256 ? 2048 : 3072)) return false;
     if (quarter) return n <= (axis == 0 ? 280 : 512);
     return axis == 0 ? n <= 440 || (n > 512 && n <= 620) : n <= kMmMaxN;
 }
