@@ -165,14 +165,17 @@ int TableCache::get(int N, int kind, bool dense, AxisDev &out)
         out = AxisDev{};
         return get_mm(N, kind, out.mm, out.mmi);
     }
-    auto it = t_.find(N);
+    // (kind -1: periodic z, whose tables are a compiled line's)
+    const bool zper = kind < 0 && !line_compiled(N);
+    auto it = t_.find(zper ? -N : N);
     if (it != t_.end()) {
         out = it->second;
         return PP_SUCCESS;
     }
-    const AxisTables &t = axis_tables_cached(N);
+    const AxisTables t = zper ? zper_tables(N) : axis_tables_cached(N);
     AxisDev d;
     auto up = [](double **dst, const std::vector<double> &v) -> int {
+        if (v.empty()) return PP_SUCCESS;
         if (hipMalloc((void **)dst, v.size() * sizeof(double)) != hipSuccess) return PP_ALLOCATION_FAIL;
         if (hipMemcpy(*dst, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
             return PP_HIP_ERROR;
@@ -182,7 +185,7 @@ int TableCache::get(int N, int kind, bool dense, AxisDev &out)
     if ((rc = up(&d.tw, t.tw)) || (rc = up(&d.A, t.A)) || (rc = up(&d.B, t.B)) || (rc = up(&d.C, t.C)) ||
         (rc = up(&d.D, t.D)))
         return rc;
-    t_[N] = d;
+    t_[zper ? -N : N] = d;
     out = d;
     return PP_SUCCESS;
 }

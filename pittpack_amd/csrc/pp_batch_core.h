@@ -42,7 +42,7 @@ class TableCache {
         double *base = nullptr;  // octant table, then the matrices
         const double *mm = nullptr, *mmi = nullptr;
     };
-    std::map<int, AxisDev> t_;
+    std::map<int, AxisDev> t_;  // by length; -length: periodic z only
     std::map<std::pair<int, int>, Matrices> m_;  // {length, symmetry family}
 };
 

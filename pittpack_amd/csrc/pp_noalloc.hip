@@ -96,15 +96,14 @@ bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
     r.lamy = take((size_t)g.ny);
     r.dtab = take(dirichlet_table_size(g));
     const bool zc = g.zper && zperiodic_supported(g.nz);
-    AxisTableSizes zs{};
     if (g.zper) {
-        zs = axis_table_sizes(g.nz);
         if (zc) {
-            r.ztw = take(zs.n[0]);
-            r.zA = take(zs.n[1]);
+            r.ztw = take((size_t)g.nz);
+            r.zA = take((size_t)g.nz + 2);
         } else if (dense && mm_dense(g, 2)) {
             r.oct[2] = take(mm_octant_size(g.nz));
         } else {
+            const AxisTableSizes zs = axis_table_sizes(g.nz);
             for (int i = 0; i < 5; i++) r.ztab[i] = take(zs.n[i]);
         }
         r.zc2 = take((size_t)g.nz);
@@ -130,9 +129,7 @@ bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
     r.zsing_x = r.zsing_y = -1;
     if (g.zper) {
         if (zc) {
-            // only tw and A of the line tables are read
-            static double unused[3][1024 + 2];
-            fill_axis_tables(g.nz, g_host + r.ztw, g_host + r.zA, unused[0], unused[1], unused[2]);
+            fill_zper_tables(g.nz, g_host + r.ztw, g_host + r.zA);
         } else if (r.mm[2]) {
             fill_mm_octant(g.nz, g_host + r.oct[2]);
         } else {

@@ -224,6 +224,36 @@ inline const AxisTables &axis_tables_cached(int N)
     return *p;
 }
 
+// tw and A of the one-pass periodic z solve (pp_zperiodic.hip), nz = 2 M: a compiled line's tables of
+// length nz, also for the lengths no line transform is compiled for; nz and nz + 2 doubles
+inline void fill_zper_tables(int nz, double *tw, double *A)
+{
+    const int M = nz / 2;
+    for (int k = 0; k <= M; k++) {
+        const double a = -2.0 * kPi * (double)k / (double)nz;
+        A[2 * k] = std::cos(a);
+        A[2 * k + 1] = std::sin(a);
+        if (k == M) break;
+        const double w = -2.0 * kPi * (double)k / (double)M;
+        tw[2 * k] = std::cos(w);
+        tw[2 * k + 1] = std::sin(w);
+    }
+}
+inline AxisTables zper_tables(int nz)
+{
+    AxisTables t;
+    if (line_compiled(nz)) {
+        const AxisTables &line = axis_tables_cached(nz);
+        t.tw = line.tw;
+        t.A = line.A;
+        return t;
+    }
+    t.tw.resize(nz);
+    t.A.resize(nz + 2);
+    fill_zper_tables(nz, t.tw.data(), t.A.data());
+    return t;
+}
+
 // octant table of the dense-product transforms (pp_line_mm.h): {cos, sin}(2 pi q / (8 N)),
 // q = 0 .. N
 inline void fill_mm_octant(int N, double *oct)

@@ -330,7 +330,7 @@ int build_tables(pp_solver *h)
     h->zsing_x = h->zsing_y = -1;
     if (h->g.zper) {
         if (zperiodic_supported(h->g.nz)) {
-            const AxisTables &zt = axis_tables_cached(h->g.nz);
+            const AxisTables zt = zper_tables(h->g.nz);
             if ((rc = upload((void **)&h->d_ztw, zt.tw)) || (rc = upload((void **)&h->d_zA, zt.A))) return rc;
         } else {
             // real z-line transforms of length nz (R2HC / HC2R)

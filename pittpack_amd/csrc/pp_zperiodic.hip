@@ -14,7 +14,7 @@
 // solves that column from FP64 plane sums instead (k_mode00, pp_mixed.hip) and has it
 // written as zeros here.
 //
-// Lengths without a compiled plan take three passes instead of one: real z-line
+// Lengths without a plan (PP_ZPER_LENGTHS) take three passes instead of one: real z-line
 // transforms of any length (the line kernels) around a division kernel (k_zper_divide).
 //
 // Storage is FP64 (FP64 form) or FP32 (the mixed form's work field); the arithmetic of the
@@ -194,20 +194,27 @@ __global__ void k_smt_v1_batch(double *data, const SmtItem *items)
     smt_v1_body(data + it.offset, it.stride, it.nz, it.diag);
 }
 
+// The half lengths M = nz / 2: the line transforms' and, whole in one thread's registers, 5 and 7
+// (columns of 10 and 14 points, us a whole solve, one pass : z-line transforms: 512x512x10 77.7 : 148,
+// 512x512x14 83.7 : 139, 64x64x10 21.1 : 27.7; 200 members of 24x24x10 in a batch, whose z-line transforms are
+// three launches of each member's own, 50.9 : 1687)
+#define PP_ZPER_LENGTHS(X) X(5) X(7) PP_FFT_LENGTHS(X)
+constexpr int zper_threads(int M) { return M == 5 || M == 7 ? 1 : line_threads(M, 1); }
+
 // columns per block: 16 (128-byte FP64 rows) while the slices fit 80 KB, 8 for longer lines, as
 // the y transforms on the field in place
 template <int M>
 constexpr int zper_lines_m()
 {
-    constexpr int L = line_lines<double, M, 1>();
-    return line_threads(M, 1) >= 64 && L > 8 ? 8 : L;
+    constexpr int L = line_lines<double, M, 1, zper_threads(M)>();
+    return zper_threads(M) >= 64 && L > 8 ? 8 : L;
 }
 
 // grid: column blocks x SY (one solve), or nitems blocks (batched, a.items set)
 template <typename S, int M>
 static hipError_t launch_zper_m(const ZPerArgs &a, int nitems, hipStream_t s)
 {
-    constexpr int T = line_threads(M, 1);
+    constexpr int T = zper_threads(M);
     constexpr int LINES = zper_lines_m<M>();
     const size_t lds = (size_t)LINES * line_slots<M>() * sizeof(cpx<double>);
     auto kern = k_zper<S, M, T, LINES>;
@@ -221,14 +228,14 @@ static hipError_t launch_zper_m(const ZPerArgs &a, int nitems, hipStream_t s)
     return hipGetLastError();
 }
 
-bool zperiodic_supported(int nz) { return nz >= 8 && line_compiled(nz); }
+bool zperiodic_supported(int nz) { return nz >= 8 && nz % 2 == 0 && zper_threads(nz / 2) > 0; }
 
 int zper_lines(int nz)
 {
-    switch (nz / 2) {
+    switch (zperiodic_supported(nz) ? nz / 2 : 0) {
 #define PPM(m) \
     case m: return zper_lines_m<m>();
-        PP_FFT_LENGTHS(PPM)
+        PP_ZPER_LENGTHS(PPM)
 #undef PPM
     default: return 0;
     }
@@ -272,10 +279,10 @@ hipError_t launch_zper_divide_f32(const ZPerArgs &a, hipStream_t s) { return lau
 template <typename S>
 static hipError_t launch_zperiodic_s(const ZPerArgs &a, int nitems, hipStream_t s)
 {
-    switch (line_compiled(a.nz) ? a.nz / 2 : 0) {
+    switch (zperiodic_supported(a.nz) ? a.nz / 2 : 0) {
 #define PPM(m) \
     case m: return launch_zper_m<S, m>(a, nitems, s);
-        PP_FFT_LENGTHS(PPM)
+        PP_ZPER_LENGTHS(PPM)
 #undef PPM
     default: return hipErrorInvalidValue;
     }
