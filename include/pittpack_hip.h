@@ -330,7 +330,10 @@ int pp_batch_synchronize(pp_batch b);
  * requests of any supported size, boundary condition and precision are admitted by HBM
  * footprint into a device pool of hbm_bytes, grouped into batches (one per precision,
  * at most PP_OPT_BATCH_MEMBERS requests) and launched on up to `streams` HIP streams, so
- * batches admitted while others run overlap on the device.  Twiddle tables stay resident.
+ * batches admitted while others run overlap on the device.  Twiddle tables stay resident beside
+ * the pool (below 0.5 MB a line length); the matrices of dense-product lines of more than 64
+ * points (some 8 n^2 bytes) lie in the pool and count in the footprint.  A request that fits the
+ * pool only without them runs those lines as convolutions.
  * A request's result does not depend on the batch it ran in.
  * ------------------------------------------------------------------------------------- */
 typedef struct pp_server_s *pp_server;

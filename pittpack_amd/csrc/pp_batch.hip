@@ -120,8 +120,30 @@ void BatchCore::plan_lanes(std::initializer_list<std::vector<HostClass> *> stage
     }
 }
 
-// periodic z lines without a compiled plan as dense products, as the single-solve handle decides
-static bool zlines_dense(const SolveSetup &g) { return mm_serves(g.nz, KIND_PP, 1, (long)g.nx * g.ny); }
+// (as the single-solve handle decides, unless the member keeps to short matrices)
+bool BatchCore::dense(const BatchMember &m, int a)
+{
+    const SolveSetup &g = m.g;
+    const int n = a == 0 ? g.nx : a == 1 ? g.ny : g.nz;
+    if (!m.dense && n > kMmResident) return false;
+    if (a == 2) return mm_serves(n, KIND_PP, 1, (long)g.nx * g.ny);
+    return mm_serves(n, g.kind[a], a, (long)(a == 0 ? g.ny : g.nx) * g.nz);
+}
+
+std::set<std::pair<int, int>> BatchCore::matrices() const
+{
+    static const int of_family[3] = {KIND_NN, KIND_ND, KIND_PP};
+    std::set<std::pair<int, int>> r;
+    auto put = [&](int n, int kind) {
+        if (n > kMmResident) r.insert({n, of_family[mm_family(kind)]});
+    };
+    for (const auto *v : {&lx_, &ly_})
+        for (const HostClass &c : *v)
+            if (c.dense) put(c.key, c.kind);
+    for (int m : zpl_)
+        if (dense(mem[m], 2)) put(mem[m].g.nz, KIND_PP);
+    return r;
+}
 
 TableCache::~TableCache()
 {
@@ -129,30 +151,52 @@ TableCache::~TableCache()
         for (double *p : {kv.second.tw, kv.second.A, kv.second.B, kv.second.C, kv.second.D})
             if (p) (void)hipFree(p);
     for (auto &kv : m_)
-        if (kv.second.base) (void)hipFree(kv.second.base);
+        if (kv.second.own) (void)hipFree(kv.second.own);
+}
+
+size_t TableCache::mm_bytes(int N, int kind)
+{
+    const size_t oct = (mm_octant_size(N) + 31) / 32 * 32;
+    return ((oct + mm_tables_size(N, kind)) * sizeof(double) + 255) / 256 * 256;
+}
+
+// octant table, then the matrices; finished before the first batch that reads them, on whichever
+// stream that runs
+int TableCache::write_mm(int N, int kind, double *base, Matrices &e)
+{
+    std::vector<double> oct(mm_octant_size(N));
+    fill_mm_octant(N, oct.data());
+    const size_t o = (oct.size() + 31) / 32 * 32;
+    if (hipMemcpy(base, oct.data(), oct.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
+        launch_mm_tables(base + o, base, N, kind, nullptr) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess)
+        return PP_HIP_ERROR;
+    e.mm = base + o;
+    e.mmi = e.mm + mm_inverse_offset(N, kind);
+    return PP_SUCCESS;
+}
+
+int TableCache::place_mm(int N, int kind, char *at)
+{
+    Matrices e;
+    const int rc = write_mm(N, kind, (double *)at, e);
+    if (!rc) m_[{N, mm_family(kind)}] = e;
+    return rc;
 }
 
 int TableCache::get_mm(int N, int kind, const double *&mm, const double *&mmi)
 {
     Matrices &e = m_[{N, mm_family(kind)}];
-    if (!e.base) {
-        std::vector<double> oct(mm_octant_size(N));
-        fill_mm_octant(N, oct.data());
-        const size_t o = (oct.size() + 31) / 32 * 32;
-        if (hipMalloc((void **)&e.base, (o + mm_tables_size(N, kind)) * sizeof(double)) != hipSuccess) {
-            e.base = nullptr;
+    if (!e.mm) {
+        if (hipMalloc((void **)&e.own, mm_bytes(N, kind)) != hipSuccess) {
+            (void)hipGetLastError();
+            e.own = nullptr;
             return PP_ALLOCATION_FAIL;
         }
-        // finished before the first batch that reads them, on whichever stream that runs
-        if (hipMemcpy(e.base, oct.data(), oct.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
-            launch_mm_tables(e.base + o, e.base, N, kind, nullptr) != hipSuccess ||
-            hipStreamSynchronize(nullptr) != hipSuccess) {
-            (void)hipFree(e.base);
-            e.base = nullptr;
-            return PP_HIP_ERROR;
+        if (const int rc = write_mm(N, kind, e.own, e)) {
+            (void)hipFree(e.own);
+            e.own = nullptr;
+            return rc;
         }
-        e.mm = e.base + o;
-        e.mmi = e.mm + mm_inverse_offset(N, kind);
     }
     mm = e.mm;
     mmi = e.mmi;
@@ -235,15 +279,12 @@ template <typename R>
 int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
 {
     std::map<std::array<int, 3>, std::vector<LineItem>> cls;  // {length, kind, dense}
-    auto is_dense = [&](const SolveSetup &g) {
-        return mm_serves(axis == 0 ? g.nx : g.ny, g.kind[axis], axis, (long)(axis == 0 ? g.ny : g.nx) * g.nz);
-    };
     // dense-product classes: launch shape from the class's units of 16 lines / columns
     std::map<std::pair<int, int>, long> units;
     for (const BatchMember &m : mem) {
         if (m.plane) continue;
         const int N = axis == 0 ? m.g.nx : m.g.ny;
-        if (is_dense(m.g))
+        if (dense(m, axis))
             units[{N, m.g.kind[axis]}] += axis == 0 ? ((long)m.g.ny * m.g.nz + 15) / 16 : (long)((m.g.nx + 15) / 16) * m.g.nz;
     }
     std::map<std::pair<int, int>, MmPlan> plans;
@@ -252,12 +293,12 @@ int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
         if (mem[m].plane) continue;
         const SolveSetup &g = mem[m].g;
         const int N = axis == 0 ? g.nx : g.ny;
-        const bool dense = is_dense(g);
-        const int group = dense ? plans.at({N, g.kind[axis]}).units : 1;
-        const int lines = line_lines_any<R>(N, dense, axis) * (axis == 0 ? group : 1);
+        const bool mm = dense(mem[m], axis);
+        const int group = mm ? plans.at({N, g.kind[axis]}).units : 1;
+        const int lines = line_lines_any<R>(N, mm, axis) * (axis == 0 ? group : 1);
         const int planes = axis == 1 ? group : 1;  // y: consecutive planes per block
         if (lines <= 0) return PP_UNSUPPORTED_SIZE;
-        auto &items = cls[{N, g.kind[axis], dense}];
+        auto &items = cls[{N, g.kind[axis], mm}];
         if (axis == 0) {
             const long nl = (long)g.ny * g.nz;
             for (long bx = 0; bx < (nl + lines - 1) / lines; bx++) items.push_back({m, (int)bx, 0});
@@ -680,9 +721,9 @@ int BatchCore::bind(char *base, TableCache *tc)
     }
     for (int m : zpl_) {
         AxisDev t;
-        const bool dense = zlines_dense(mem[m].g);
-        if ((rc = tc->get(mem[m].g.nz, KIND_PP, dense, t))) return rc;
-        tabs_[{mem[m].g.nz, KIND_PP, dense}] = t;
+        const bool mm = dense(mem[m], 2);
+        if ((rc = tc->get(mem[m].g.nz, KIND_PP, mm, t))) return rc;
+        tabs_[{mem[m].g.nz, KIND_PP, mm}] = t;
     }
     if (precision == 1) {
         d_sums_ = (double *)(base + o_sums_);
@@ -964,7 +1005,7 @@ int BatchCore::run_z_stage(hipStream_t s, bool f32)
     }
     for (int m : zpl_) {
         const SolveSetup &g = mem[m].g;
-        const AxisDev &t = tabs_.at({g.nz, KIND_PP, zlines_dense(g)});
+        const AxisDev &t = tabs_.at({g.nz, KIND_PP, dense(mem[m], 2)});
         const long off = mem[m].offset;
         void *data = f32 ? (void *)(d_w + off) : (void *)(d_sol + off);
         ZPerArgs zp{};

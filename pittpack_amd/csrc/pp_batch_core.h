@@ -10,6 +10,7 @@
 
 #include <array>
 #include <map>
+#include <set>
 #include <vector>
 
 #include "pp_launch.h"
@@ -34,14 +35,19 @@ class TableCache {
     ~TableCache();
     // tables of lines of length N (dense: as products of `kind`)
     int get(int N, int kind, bool dense, AxisDev &out);
-    // dense-product matrices of (N, kind)
+    // dense-product matrices of (N, kind): where the caller has placed them, else allocated
     int get_mm(int N, int kind, const double *&mm, const double *&mmi);
+    // ... in the caller's memory (mm_bytes, 256-byte aligned) until drop_mm; kinds of one family share them
+    static size_t mm_bytes(int N, int kind);
+    int place_mm(int N, int kind, char *at);
+    void drop_mm(int N, int kind) { m_.erase({N, mm_family(kind)}); }
 
   private:
     struct Matrices {
-        double *base = nullptr;  // octant table, then the matrices
+        double *own = nullptr;  // its allocation (null: placed by the caller)
         const double *mm = nullptr, *mmi = nullptr;
     };
+    int write_mm(int N, int kind, double *base, Matrices &e);
     std::map<int, AxisDev> t_;  // by length; -length: periodic z only
     std::map<std::pair<int, int>, Matrices> m_;  // {length, symmetry family}
 };
@@ -71,6 +77,11 @@ struct BatchLanes {
     hipError_t merge(hipStream_t s);
 };
 
+// Matrices of lines of up to this many points count as tables (35 KB at most, some 2 MB if every length
+// and family of them is met); longer ones take some 8 N^2 bytes (the real DFT's 4 N^2), 4.8 GB all
+// together, which a server places in its pool (pp_server.hip)
+constexpr int kMmResident = 64;
+
 struct BatchMember {
     SolveSetup g;
     long offset = 0;  // element offset of the member's field in the rhs / solution / work arenas
@@ -78,6 +89,7 @@ struct BatchMember {
     long dtab_off = 0;
     bool pinned = false;  // mixed form: pinned (0,0) column solved in FP64 from plane sums
     long sums_off = 0, plane_off = 0, upart_off = 0;
+    bool dense = true;   // may multiply with matrices of more than kMmResident points
     bool plane = false;  // FP64: both transforms of a plane in one launch (pp_plane_mm.h)
     long toff = 0;  // FP64: offset of the member's z tiles in the tile arena (-1: none)
 };
@@ -103,6 +115,9 @@ class BatchCore {
     int bind(char *base, TableCache *tc);
     // asynchronous uploads of the planned tables (host copies stay alive in this object)
     int upload(hipStream_t s);
+    // planned: the matrices of more than kMmResident points its lines multiply with, {length, kind} (one
+    // kind of each family)
+    std::set<std::pair<int, int>> matrices() const;
     // the solve of every member (right-hand sides kept, solutions in the solution arena)
     int run(hipStream_t s, Marks *mk);
     BatchLanes *lanes = nullptr;  // a captured run's stages, class by class over these (null: in series)
@@ -143,6 +158,8 @@ class BatchCore {
         int lane = 0;        // stream of the class within its stage (0: the batch's own)
         bool fused = false;  // correction x classes: members whose residual runs in k_resx
     };
+    // are the member's lines along axis a (0 x, 1 y; 2 periodic z without a plan) dense products?
+    static bool dense(const BatchMember &m, int a);
     hipStream_t lane(hipStream_t s, int k) const { return forked_ && k > 0 ? lanes->side[k - 1] : s; }
     void plan_lanes(std::initializer_list<std::vector<HostClass> *> stage);
     int launch_class(hipStream_t s, const HostClass &c, int form, int axis, int fwd, const void *in, void *out,

@@ -14,7 +14,9 @@
 // finished batches by polling their events.  A request that does not fit may be overtaken
 // by later, smaller ones only a bounded number of times (PP_OPT_MAX_OVERTAKE); after that
 // nothing behind it is admitted until it runs, so a large request cannot starve under a
-// stream of small ones.  Twiddle tables stay resident for the server's lifetime;
+// stream of small ones.  Twiddle tables stay resident for the server's lifetime; the matrices of
+// long dense-product lines (8 N^2 bytes) lie in the pool, are counted with the requests that
+// multiply with them, stay for the next ones and give way where a batch needs the room;
 // per-request eigenvalue and boundary tables are planned on the host and uploaded with the
 // batch.  Solutions go device -> pinned staging on the batch's stream; the waiting caller
 // copies them into its own buffer, so the scheduler never blocks on a host copy.  A member's
@@ -30,6 +32,7 @@
 #include <map>
 #include <mutex>
 #include <new>
+#include <set>
 #include <thread>
 #include <vector>
 
@@ -106,6 +109,15 @@ class RangePool {
     size_t cap_ = 0, used_ = 0;
 };
 
+using MmKey = std::pair<int, int>;  // {length, kind}, one kind of each family (BatchCore::matrices)
+
+// matrices in the pool
+struct Mats {
+    size_t off = 0;
+    int users = 0;       // batches in flight that read them
+    long long last = 0;  // launch number of the latest one
+};
+
 struct Request {
     long long ticket = 0;
     int nx = 0, ny = 0, nz = 0;
@@ -115,7 +127,9 @@ struct Request {
     const double *rhs = nullptr;  // host right-hand side (null: counter generator with `seed`)
     unsigned long long seed = 0;
     bool want = false;            // copy the solution back to the host
-    size_t need = 0;              // device footprint: the region of this request planned alone
+    size_t need = 0;              // the region of this request planned alone, and
+    std::set<MmKey> mats;         //   the matrices beside it: its device footprint
+    bool dense = true;            // false: the pool has no room for both, so its long lines are convolutions
     int overtaken = 0;            // batches admitted past this request while it did not fit
     long long batch_seq = -1;     // launch number of the batch that ran it
     double t_submit = 0, t_launch = 0, t_done = 0;
@@ -132,6 +146,7 @@ struct InFlight {
     int slot = -1;
     hipEvent_t done = nullptr;
     std::vector<Request *> reqs;
+    std::set<MmKey> mats;
 };
 
 }  // namespace
@@ -141,6 +156,7 @@ struct pp_server_s {
     char *stage = nullptr;     // pinned host staging for solutions
     RangePool dpool, spool;
     TableCache tables;
+    std::map<MmKey, Mats> mats;  // (the scheduler's)
     std::vector<hipStream_t> streams;
     std::vector<bool> slot_busy;
     std::vector<hipEvent_t> events;
@@ -164,19 +180,103 @@ struct pp_server_s {
 
 namespace {
 
+size_t mats_bytes(const std::set<MmKey> &keys)
+{
+    size_t b = 0;
+    for (const MmKey &k : keys) b += TableCache::mm_bytes(k.first, k.second);
+    return b;
+}
+
 // device footprint of one request: its region planned as a batch of one (the scheduler's
 // batches use the same refinement setting; a batch's region never exceeds the sum of its
-// members' regions).  Returns a PittPack code for a request that cannot be planned.
-int request_bytes(const Request *r, int refine, size_t &bytes)
+// members' regions) and its matrices.  A request whose region fits `cap` but not with its matrices
+// keeps to short ones: by its shape and the pool alone, so its result does not depend on the load.
+// Returns a PittPack code for a request that cannot be planned.
+int request_bytes(Request *r, int refine, size_t cap)
 {
-    BatchCore c;
-    c.precision = r->precision;
-    c.refine = refine;
-    int id = -1;
-    int rc = c.add(r->nx, r->ny, r->nz, r->bc, r->X, &id);
-    if (!rc) rc = c.plan();
-    bytes = rc ? 0 : c.region_bytes;
-    return rc;
+    r->need = 0;
+    for (bool dense : {true, false}) {
+        BatchCore c;
+        c.precision = r->precision;
+        c.refine = refine;
+        int id = -1;
+        int rc = c.add(r->nx, r->ny, r->nz, r->bc, r->X, &id);
+        if (rc) return rc;
+        c.mem[id].dense = r->dense = dense;
+        if ((rc = c.plan())) return rc;
+        r->need = c.region_bytes;
+        r->mats = c.matrices();
+        if (r->mats.empty() || r->need + mats_bytes(r->mats) <= cap) break;
+    }
+    return PP_SUCCESS;
+}
+
+// (pool and matrices: the scheduler thread, holding the lock that callers read the pool under)
+void drop_mats(pp_server_s *s, std::map<MmKey, Mats>::iterator it)
+{
+    s->tables.drop_mm(it->first.first, it->first.second);
+    s->dpool.release(it->second.off);
+    s->mats.erase(it);
+}
+
+// room in the pool, from unused matrices if need be, the longest unused first
+bool pool_alloc(pp_server_s *s, size_t bytes, size_t &off)
+{
+    while (!s->dpool.alloc(bytes, off)) {
+        auto old = s->mats.end();
+        for (auto it = s->mats.begin(); it != s->mats.end(); ++it)
+            if (it->second.users == 0 && (old == s->mats.end() || it->second.last < old->second.last)) old = it;
+        if (old == s->mats.end()) return false;
+        drop_mats(s, old);
+    }
+    return true;
+}
+
+void unpin(pp_server_s *s, const std::set<MmKey> &keys)
+{
+    for (const MmKey &k : keys) {
+        auto it = s->mats.find(k);
+        if (it != s->mats.end()) it->second.users--;
+    }
+}
+
+// a batch's region (bytes at off) and matrices (pinned; `fresh`: those yet to be written).  Where
+// matrices left in the pool are in the way, a second attempt starts without them
+bool place(pp_server_s *s, size_t bytes, const std::set<MmKey> &keys, size_t &off, std::set<MmKey> &fresh)
+{
+    for (int attempt = 0; attempt < 2; attempt++) {
+        fresh.clear();
+        std::set<MmKey> held;
+        for (const MmKey &k : keys) {
+            auto it = s->mats.find(k);
+            if (it == s->mats.end()) continue;
+            it->second.users++;
+            held.insert(k);
+        }
+        const bool region = pool_alloc(s, bytes, off);
+        bool ok = region;
+        for (auto k = keys.begin(); ok && k != keys.end(); ++k) {
+            if (held.count(*k)) continue;
+            Mats m;
+            if (!(ok = pool_alloc(s, TableCache::mm_bytes(k->first, k->second), m.off))) break;
+            m.users = 1;
+            s->mats[*k] = m;
+            fresh.insert(*k);
+        }
+        if (ok) {
+            for (const MmKey &k : keys) s->mats[k].last = s->batches;
+            return true;
+        }
+        for (const MmKey &k : fresh) drop_mats(s, s->mats.find(k));
+        if (region) s->dpool.release(off);
+        unpin(s, held);
+        for (auto it = s->mats.begin(); it != s->mats.end();) {
+            auto next = std::next(it);
+            if (it->second.users == 0) drop_mats(s, it);
+            it = next;
+        }
+    }
+    return false;
 }
 
 void fail_request(pp_server_s *s, Request *r, int rc)
@@ -209,6 +309,7 @@ bool retire(pp_server_s *s)
                 s->points_done += r->points();
             }
             s->dpool.release(f->off);
+            unpin(s, f->mats);
             s->slot_busy[f->slot] = false;
             s->last_done = t;
         }
@@ -236,6 +337,8 @@ bool launch(pp_server_s *s, std::vector<Request *> &group, int slot)
             std::lock_guard<std::mutex> lk(s->mu);
             fail_request(s, r, rc);
         } else {
+            f->core.mem[id].dense = r->dense;
+            f->mats.insert(r->mats.begin(), r->mats.end());
             ok.push_back(r);
         }
     }
@@ -246,9 +349,10 @@ bool launch(pp_server_s *s, std::vector<Request *> &group, int slot)
     int rc = f->core.plan();
     size_t off = 0;
     bool fits;
+    std::set<MmKey> fresh;
     {
         std::lock_guard<std::mutex> lk(s->mu);
-        fits = !rc && s->dpool.alloc(f->core.region_bytes, off);
+        fits = !rc && place(s, f->core.region_bytes, f->mats, off, fresh);
     }
     if (rc || !fits) {
         delete f;
@@ -264,7 +368,9 @@ bool launch(pp_server_s *s, std::vector<Request *> &group, int slot)
     f->done = s->events[slot];
     f->reqs = ok;
     hipStream_t st = s->streams[slot];
-    rc = f->core.bind(s->dev + off, &s->tables);
+    for (auto k = fresh.begin(); !rc && k != fresh.end(); ++k)
+        rc = s->tables.place_mm(k->first, k->second, s->dev + s->mats.at(*k).off);
+    if (!rc) rc = f->core.bind(s->dev + off, &s->tables);
     if (!rc) rc = f->core.upload(st);
     {
         // callers read a request's status under the lock
@@ -299,6 +405,8 @@ bool launch(pp_server_s *s, std::vector<Request *> &group, int slot)
         std::lock_guard<std::mutex> lk(s->mu);
         for (Request *r : ok) fail_request(s, r, rc);
         s->dpool.release(off);
+        unpin(s, f->mats);
+        for (const MmKey &k : fresh) drop_mats(s, s->mats.find(k));  // perhaps not written
         delete f;
         return true;
     }
@@ -328,7 +436,14 @@ void worker_loop(pp_server_s *s)
                 s->cv_work.wait(lk, [&] { return s->stop || !s->queue.empty(); });
                 if (s->stop && s->queue.empty()) return;
             }
+            // (unused matrices give way; a request's count unless a batch in flight, or a request
+            // admitted before it, holds them)
             size_t budget = s->dpool.cap() - s->dpool.used();
+            std::set<MmKey> pinned;
+            for (const auto &kv : s->mats) {
+                if (kv.second.users > 0) pinned.insert(kv.first);
+                else budget += TableCache::mm_bytes(kv.first.first, kv.first.second);
+            }
             // requests left behind this round because they did not fit; once one of them has
             // been overtaken max_overtake times, nothing behind it is admitted
             std::vector<Request *> skipped;
@@ -348,7 +463,11 @@ void worker_loop(pp_server_s *s)
                         ++it;
                         continue;
                     }
-                    bool fits = r->need <= budget;
+                    std::set<MmKey> more;
+                    for (const MmKey &k : r->mats)
+                        if (!pinned.count(k)) more.insert(k);
+                    const size_t need = r->need + mats_bytes(more);
+                    bool fits = need <= budget;
                     // solution staging (pinned host) for callers that want the result
                     if (fits && r->want && !r->staged) {
                         if (s->spool.alloc((size_t)r->points() * sizeof(double), r->stage_off)) r->staged = true;
@@ -363,7 +482,8 @@ void worker_loop(pp_server_s *s)
                         ++it;
                         continue;
                     }
-                    budget -= r->need;
+                    budget -= need;
+                    pinned.insert(more.begin(), more.end());
                     groups[p].push_back(r);
                     it = s->queue.erase(it);
                 }
@@ -500,7 +620,7 @@ int pp_server_submit(pp_server s, int nx, int ny, int nz, const char *bc, const 
     }
     // plan the request alone: unsupported sizes or boundary conditions are returned here, and
     // what can never be admitted is rejected
-    const int prc = request_bytes(r, refine, r->need);
+    const int prc = request_bytes(r, refine, s->dpool.cap());
     if (prc) {
         delete r;
         return prc;
@@ -541,9 +661,8 @@ int pp_server_footprint(pp_server s, int nx, int ny, int nz, const char *bc, con
         std::lock_guard<std::mutex> lk(s->mu);
         refine = s->refine;
     }
-    size_t b = 0;
-    const int rc = request_bytes(&r, refine, b);
-    *bytes = (long long)b;
+    const int rc = request_bytes(&r, refine, s->dpool.cap());
+    *bytes = rc ? 0 : (long long)(r.need + mats_bytes(r.mats));
     return rc;
 }
 
