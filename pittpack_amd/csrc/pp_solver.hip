@@ -567,9 +567,14 @@ int run_fp64_stages(pp_solver *h, const double *rhs, double *field)
     hipStream_t s = h->stream;
     bool zt = use_ztiles(h);
     int rc;
+    // periodic z needs no second field: in place where there is no room for one, and in a capture that
+    // begins before there is one (it takes no allocation)
+    if (zt && h->g.zper && !h->d_zt) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) zt = false;
+    }
     if (zt && (rc = ensure_ztiles(h))) {
         if (!h->g.zper || rc != PP_ALLOCATION_FAIL) return rc;
-        // periodic z needs no second field: in place where there is no room for one
         (void)hipGetLastError();
         h->no_zt = true;
         zt = false;
