@@ -24,6 +24,7 @@ struct HostRing {
     static constexpr int kSlots = 2;
     static constexpr size_t kChunk = (size_t)1 << 20;
     char *buf = nullptr;
+    int device = -1;  // of its events
     hipEvent_t ev[kCopyThreads * kSlots] = {};
     std::mutex in_use;
 };
@@ -31,7 +32,8 @@ void free_ring(HostRing &r);
 
 // dst (host) <- src (device, 16-byte aligned) on `s`, finished and the stream drained on return.
 // Copies under kRingMin (2 MB: 0.11 against 0.12 ms, 4 MB: 0.19 against 0.24), registered host memory, the
-// per-thread stream (another one on each helper), a ring that another thread is using, and any failure to get the ring are the runtime's.
+// per-thread stream (another one on each helper), a ring that another thread is using, a stream, source or
+// ring of another device than the caller's current one, and whatever fails on the way are the runtime's.
 constexpr size_t kRingMin = (size_t)4 << 20;
 hipError_t copy_to_host(HostRing &r, double *dst, const double *src, size_t count, hipStream_t s);
 

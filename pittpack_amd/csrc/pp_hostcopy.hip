@@ -18,9 +18,9 @@ __global__ void __launch_bounds__(256) k_to_host(double *__restrict__ out, const
     if (n % 2 && blockIdx.x == 0 && threadIdx.x == 0) out[n - 1] = in[n - 1];
 }
 
-bool ring_ready(HostRing &r)
+bool ring_ready(HostRing &r, int device)
 {
-    if (r.buf) return true;
+    if (r.buf) return r.device == device;
     const int n = kCopyThreads * HostRing::kSlots;
     if (hipHostMalloc((void **)&r.buf, n * HostRing::kChunk, hipHostMallocDefault) != hipSuccess) {
         r.buf = nullptr;
@@ -34,7 +34,21 @@ bool ring_ready(HostRing &r)
             free_ring(r);
             return false;
         }
+    r.device = device;
     return true;
+}
+
+// kernels and events of one device serve its own streams alone: the current device, if the stream and the
+// source are its own too, else -1
+int one_device(const double *src, hipStream_t s)
+{
+    int device = 0;
+    hipDevice_t of_stream = 0;
+    hipPointerAttribute_t a{};
+    bool ok = hipGetDevice(&device) == hipSuccess && hipPointerGetAttributes(&a, src) == hipSuccess && a.device == device;
+    if (ok && s) ok = hipStreamGetDevice(s, &of_stream) == hipSuccess && of_stream == device;
+    if (!ok) (void)hipGetLastError();
+    return ok ? device : -1;
 }
 
 // memory the device reaches by itself
@@ -103,13 +117,15 @@ void free_ring(HostRing &r)
 hipError_t copy_to_host(HostRing &r, double *dst, const double *src, size_t count, hipStream_t s)
 {
     const size_t bytes = count * sizeof(double);
-    int device = 0;
-    std::unique_lock<std::mutex> lk(r.in_use, std::try_to_lock);
-    if (!lk.owns_lock() || bytes < kRingMin || s == hipStreamPerThread || registered(dst) || hipGetDevice(&device) != hipSuccess ||
-        !ring_ready(r)) {
+    auto plain = [&] {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
         return e != hipSuccess ? e : hipStreamSynchronize(s);
-    }
+    };
+    int device = -1;
+    std::unique_lock<std::mutex> lk(r.in_use, std::try_to_lock);
+    if (!lk.owns_lock() || bytes < kRingMin || s == hipStreamPerThread || registered(dst) ||
+        (device = one_device(src, s)) < 0 || !ring_ready(r, device))
+        return plain();
     hipError_t err[kCopyThreads];
     on_threads(kCopyThreads, [&](int w) {
         err[w] = hipSetDevice(device);
@@ -119,7 +135,9 @@ hipError_t copy_to_host(HostRing &r, double *dst, const double *src, size_t coun
     hipError_t e = hipStreamSynchronize(s);
     for (hipError_t w : err)
         if (w != hipSuccess) e = w;
-    return e;
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    return plain();
 }
 
 void copy_by_threads(void *dst, const void *src, size_t bytes)
