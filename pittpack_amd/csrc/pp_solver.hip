@@ -770,14 +770,14 @@ int autotune(pp_solver *h)
     // line shapes: every combination of the stages' two shapes (at most 16), timed round-robin
     // over three rounds (best whole-solve time each, so drift spreads over all of them and
     // the effect of a stage's output order on the next stage counts); the default
-    // combination is kept unless another is more than 0.5% faster
+    // combination is kept unless another is more than 0.5% faster.  Small planes run none of them
     const int len[4] = {h->g.nx, h->g.ny, h->g.ny, h->g.nx};
     int stages[4], nv = 0;
     for (int i = 0; i < 4; i++)
-        if (line_has_variant(len[i])) stages[nv++] = i;
+        if (line_has_variant(len[i]) && !use_plane(h)) stages[nv++] = i;
     const int ncomb = 1 << nv;
     std::vector<double> tc((size_t)ncomb, 1e30);
-    for (int round = 0; round < 3 && !rc; round++) {
+    for (int round = 0; round < 3 && nv && !rc; round++) {
         for (int comb = 0; comb < ncomb && !rc; comb++) {
             for (int i = 0; i < 4; i++) h->line_var[i] = 0;
             for (int k = 0; k < nv; k++) h->line_var[stages[k]] = (comb >> k) & 1;
