@@ -207,7 +207,9 @@ int pp_solve_device_oop(pp_handle h, const double *d_rhs, double *d_u);
  * PP_OPT_ZERO_MODE rule (0 or 1) are arguments; d_rhs is kept, the solution goes to d_u (may
  * equal d_rhs), asynchronous on `stream` (hipStream_t as void*, null = default stream).  It
  * calls no allocator: its tables live in a fixed 2 MiB device array per GPU, held until the
- * process ends, and the z solve runs on d_u in place (no z-tile buffer).  Limits: the
+ * process ends, and the z solve runs on d_u in place (no z-tile buffer).  An axis whose
+ * dense-product matrices do not fit beside the other tables (some 8 n^2 bytes: long lines
+ * without a compiled plan) runs as a convolution, which differs in rounding.  Limits: the
  * handle's sizes (lines 2..1024, z columns 4..1024, periodic z 2..1024); larger grids get
  * PP_UNSUPPORTED_SIZE.  A call with new sizes, boundary conditions, box or zero-mode rule
  * rebuilds the tables on the host, copies them in and synchronises `stream` (PP_CALL_ORDER

@@ -20,33 +20,25 @@
 #include "pittpack_hip.h"
 #include "pp_handle.h"
 #include "pp_launch.h"
-#include "pp_plane_mm.h"
+#include "pp_noalloc.h"
 #include "pp_setup.h"
 
 namespace {
 
 using namespace pp;
 
-constexpr size_t kScratchDoubles = 256 * 1024;  // 2 MiB per GPU
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) double scratch[kScratchDoubles];
 
-// the tables of the last call per device (host side) and where they sit in scratch
-struct Resident {
+// the tables of the last call per device (host side)
+struct Resident : NoallocTables {
     bool valid = false;
     int nx = 0, ny = 0, nz = 0, zero_mode = 0;
     char bc[6] = {};
     double X[6] = {};
-    size_t tab[2][5] = {};  // offsets (doubles) of tw, A, B, C, D per axis
-    size_t ztab[5] = {};    // periodic z without a compiled plan: real z-line tables
-    size_t lamx = 0, lamy = 0, dtab = 0, ztw = 0, zA = 0, zc2 = 0;
-    // dense-product lines (x, y, periodic z): where their matrices are written (0: none) and
-    // their octant tables
-    size_t mm[3] = {}, oct[3] = {};
     int zsing_x = -1, zsing_y = -1;
     double zsing_eig = -2.0;
-    size_t used = 0;  // doubles of scratch in use
 };
 
 std::mutex g_mu;
@@ -60,66 +52,18 @@ bool same_key(const Resident &r, int nx, int ny, int nz, const char *bc, const d
            std::memcmp(r.bc, bc, 6) == 0 && std::memcmp(r.X, X, sizeof(r.X)) == 0;
 }
 
-// lines of axis a (0 x, 1 y; 2 periodic z) that are dense products, or whose matrices the handle would have
-bool mm_dense(const SolveSetup &g, int a)
+// lay the tables of `g` out (pp_noalloc.h) and fill the part that is copied in g_host; false if they
+// exceed the array
+bool build_host_tables(const SolveSetup &g, Resident &r)
 {
-    if (a == 2) return mm_serves(g.nz, KIND_PP, 1, (long)g.nx * g.ny);
-    return mm_serves(a == 0 ? g.nx : g.ny, g.kind[a], a, (long)(a == 0 ? g.ny : g.nx) * g.nz);
-}
-bool mm_lines(const SolveSetup &g, int a)
-{
-    return mm_dense(g, a) || mm_plane(g.nx, g.ny, g.kind[0], g.kind[1]);
-}
-
-// lay the tables of `g` out in g_host (offsets into r); false if they exceed kScratchDoubles.
-// dense: lines without a compiled plan take the dense products (their octant table here, room
-// for their matrices behind the copied part), else the chirp convolution
-bool build_host_tables(const SolveSetup &g, Resident &r, bool dense)
-{
-    size_t o = 0;
     r = Resident{};
-    auto take = [&](size_t n) {
-        const size_t at = o;
-        o += (n + 31) / 32 * 32;  // 256-byte aligned sub-arrays
-        return at;
-    };
-    const int n[2] = {g.nx, g.ny};
-    for (int a = 0; a < 2; a++) {
-        if (dense && mm_lines(g, a)) {
-            r.oct[a] = take(mm_octant_size(n[a]));
-            if (mm_dense(g, a)) continue;
-        }
-        const AxisTableSizes z = axis_table_sizes(n[a]);
-        for (int i = 0; i < 5; i++) r.tab[a][i] = take(z.n[i]);
-    }
-    r.lamx = take((size_t)g.nx);
-    r.lamy = take((size_t)g.ny);
-    r.dtab = take(dirichlet_table_size(g));
+    if (!noalloc_layout(g, zperiodic_supported(g.nz), r)) return false;
     const bool zc = g.zper && zperiodic_supported(g.nz);
-    if (g.zper) {
-        if (zc) {
-            r.ztw = take((size_t)g.nz);
-            r.zA = take((size_t)g.nz + 2);
-        } else if (dense && mm_dense(g, 2)) {
-            r.oct[2] = take(mm_octant_size(g.nz));
-        } else {
-            const AxisTableSizes zs = axis_table_sizes(g.nz);
-            for (int i = 0; i < 5; i++) r.ztab[i] = take(zs.n[i]);
-        }
-        r.zc2 = take((size_t)g.nz);
-    }
-    r.used = o;
-    // the matrices are written on the device, behind the part that is copied
-    if (dense) {
-        for (int a = 0; a < 2; a++)
-            if (mm_lines(g, a)) r.mm[a] = take(mm_tables_size(n[a], g.kind[a]));
-        if (g.zper && !zc && mm_dense(g, 2)) r.mm[2] = take(mm_tables_size(g.nz, KIND_PP));
-    }
-    if (o > kScratchDoubles) return false;
+    const int n[2] = {g.nx, g.ny};
     std::memset(g_host, 0, r.used * sizeof(double));
     for (int a = 0; a < 2; a++) {
         if (r.mm[a]) fill_mm_octant(n[a], g_host + r.oct[a]);
-        if (!r.mm[a] || !mm_dense(g, a))
+        if (!r.mm[a] || !noalloc_dense(g, a))
             fill_axis_tables(n[a], g_host + r.tab[a][0], g_host + r.tab[a][1], g_host + r.tab[a][2],
                              g_host + r.tab[a][3], g_host + r.tab[a][4]);
     }
@@ -206,8 +150,7 @@ extern "C" int pp_solve_device_oop_noalloc(int nx, int ny, int nz, const char *b
             if (cs != hipStreamCaptureStatusNone) return PP_CALL_ORDER;
             g_res[dev].valid = false;
             Resident nr;
-            // matrices that do not fit the array: the chirp convolution, whose tables do
-            if (!build_host_tables(g, nr, true) && !build_host_tables(g, nr, false)) return PP_UNSUPPORTED_SIZE;
+            if (!build_host_tables(g, nr)) return PP_UNSUPPORTED_SIZE;
             if (hipMemcpyAsync(base, g_host, nr.used * sizeof(double), hipMemcpyHostToDevice, s) != hipSuccess)
                 return PP_HIP_ERROR;
             const int len[3] = {nx, ny, nz}, kind[3] = {g.kind[0], g.kind[1], KIND_PP};

@@ -1,0 +1,55 @@
+"""Host rules that choose a transform's kernel, compiled for the host alone (tests/dispatch_rules.cpp): the
+table layout of the no-allocation entry point."""
+import ctypes
+import os
+import random
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    from pittpack_amd import build
+
+    so = str(tmp_path_factory.mktemp("rules") / "librules.so")
+    subprocess.run([build.hipcc(), "-x", "hip", "--offload-arch=gfx950", "--offload-host-only", "-O1", "-std=c++17", "-fPIC",
+                    "-shared", "-I" + build.SRC, "-I" + os.path.join(ROOT, "include"),
+                    os.path.join(HERE, "dispatch_rules.cpp"), "-o", so], check=True, capture_output=True)
+    L = ctypes.CDLL(so)
+    L.rule_dense.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long]
+    return L
+
+
+def layout(rules, nx, ny, nz, bc, one_pass):
+    starts, ends = (ctypes.c_long * 32)(), (ctypes.c_long * 32)()
+    count, room = ctypes.c_int(0), ctypes.c_long(0)
+    bits = rules.rule_noalloc(nx, ny, nz, bc.encode(), int(one_pass), starts, ends, ctypes.byref(count), ctypes.byref(room))
+    return bits, sorted(zip(starts[: count.value], ends[: count.value])), room.value
+
+
+def test_noalloc_axes_keep_the_matrices_that_fit(rules):
+    """one axis whose matrices do not fit does not cost the others theirs"""
+    for shape, bc, axes in (((101, 509, 97), "DDNNDD", 1), ((509, 101, 97), "NNDDDD", 2), ((101, 97, 331), "NNNNPP", 3 | 4),
+                            ((331, 331, 331), "PPPPPP", 1 | 2 | 4), ((439, 1021, 9), "NNNNDD", 1), ((24, 20, 18), "NNDDDD", 3),
+                            ((64, 64, 701), "NNNNPP", 4), ((64, 64, 767), "NNNNPP", 0)):
+        bits = layout(rules, *shape, bc, False)[0]
+        assert bits & 8 and bits & 7 == axes, (shape, bc, bits & 7)
+
+
+def test_noalloc_layouts_fit_and_do_not_overlap(rules):
+    rng = random.Random(7)
+    kinds = ["PP", "NN", "DD", "ND", "DN"]
+    sizes = [2, 3, 4, 17, 33, 63, 64, 65, 101, 331, 439, 509, 620, 701, 1021, 1023, 1024]
+    for _ in range(4000):
+        n = [rng.choice(sizes) if rng.random() < 0.6 else rng.randint(2, 1024) for _ in range(3)]
+        bc = "".join(rng.choice(kinds) for _ in range(3))
+        for one_pass in (False, True) if bc.endswith("PP") else (False,):
+            bits, spans, room = layout(rules, *n, bc, one_pass)
+            assert bits & 8, (n, bc)
+            assert spans[0][0] >= 0 and spans[-1][1] <= room, (n, bc)
+            assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:])), (n, bc, spans)
+            assert all(a % 32 == 0 for a, _ in spans)
