@@ -257,7 +257,7 @@ int BatchCore::add(int nx, int ny, int nz, const char *bc, const double *X, int 
     const int rc = setup_boundary(m.g, bc);
     if (rc) return rc;
     if (precision == 0 && !zper) {
-        const int ly = line_lines_any<double>(ny, m.g.kind[1], 1);
+        const int ly = line_lines_any<double>(ny, line_route(ny, m.g.kind[1], 1, (long)nx * nz), 1);
         if (ly <= 0 || zsolve_cpb<double>() % ly != 0) return PP_UNSUPPORTED_SIZE;
     }
     for (int i = 0; i < 6; i++) m.g.X[i] = X[i];
@@ -295,7 +295,7 @@ int BatchCore::plan_lines(int axis, std::vector<HostClass> &out)
         const int N = axis == 0 ? g.nx : g.ny;
         const bool mm = dense(mem[m], axis);
         const int group = mm ? plans.at({N, g.kind[axis]}).units : 1;
-        const int lines = line_lines_any<R>(N, mm, axis) * (axis == 0 ? group : 1);
+        const int lines = line_lines_any<R>(N, mm ? LineRoute::DENSE : LineRoute::PLAN, axis) * (axis == 0 ? group : 1);
         const int planes = axis == 1 ? group : 1;  // y: consecutive planes per block
         if (lines <= 0) return PP_UNSUPPORTED_SIZE;
         auto &items = cls[{N, g.kind[axis], mm}];

@@ -584,12 +584,19 @@ hipError_t launch_line_mm_cfg(const LineArgs &a, hipStream_t s)
     return launch_line_mm_pw<TIn, TOut, AX, FWD, KIND, 1>(a, p, grid, s);
 }
 
-// lines (x) or columns (y) per block of whichever launch serves length N (dense x launches take
+// what serves a line: a compiled plan or the chirp convolution, or the dense products
+enum class LineRoute { PLAN, DENSE };
+inline LineRoute line_route(int n, int kind, int axis, long lines)
+{
+    return mm_serves(n, kind, axis, lines) ? LineRoute::DENSE : LineRoute::PLAN;
+}
+
+// lines (x) or columns (y) per block of the launch that serves length N (dense x launches take
 // whole multiples of it, mm_plan)
 template <typename R>
-inline int line_lines_any(int N, bool dense, int AX)
+inline int line_lines_any(int N, LineRoute route, int AX)
 {
-    if (dense) return 16;
+    if (route == LineRoute::DENSE) return 16;
     return line_compiled(N) ? line_block_lines<R>(N, AX) : bs_block_lines<R>(N, AX);
 }
 

@@ -432,7 +432,7 @@ bool use_ztiles(pp_solver *h)
     } else if (h->zsolver != 0 || (!zsolve_supported_f64(h->g.nz) && !zsolve_long_supported_f64(h->g.nz))) {
         return false;
     }
-    const int ly = line_lines_any<double>(h->g.ny, h->g.kind[1], 1);
+    const int ly = line_lines_any<double>(h->g.ny, line_route(h->g.ny, h->g.kind[1], 1, (long)h->g.nx * h->g.nz), 1);
     return ly > 0 && zsolve_cpb<double>() % ly == 0;
 }
 

@@ -1,5 +1,5 @@
 """Host rules that choose a transform's kernel, compiled for the host alone (tests/dispatch_rules.cpp): the
-table layout of the no-allocation entry point."""
+table layout of the no-allocation entry point, and the y blocks that z tiles rest on."""
 import ctypes
 import os
 import random
@@ -21,6 +21,7 @@ def rules(tmp_path_factory):
                     os.path.join(HERE, "dispatch_rules.cpp"), "-o", so], check=True, capture_output=True)
     L = ctypes.CDLL(so)
     L.rule_dense.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long]
+    L.rule_y_block.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_long]
     return L
 
 
@@ -53,3 +54,12 @@ def test_noalloc_layouts_fit_and_do_not_overlap(rules):
             assert spans[0][0] >= 0 and spans[-1][1] <= room, (n, bc)
             assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:])), (n, bc, spans)
             assert all(a % 32 == 0 for a, _ in spans)
+
+
+def test_y_blocks_divide_a_z_tile(rules):
+    """every FP64 y launch's columns fill a 16-column z tile in whole blocks"""
+    for n in range(2, 1025):
+        for kind in range(5):
+            for lines in (16, 100000):
+                cols = rules.rule_y_block(n, kind, lines)
+                assert cols > 0 and 16 % cols == 0, (n, kind, lines, cols)
