@@ -1,11 +1,14 @@
 """Host rules that choose a transform's kernel, compiled for the host alone (tests/dispatch_rules.cpp): the
-table layout of the no-allocation entry point, and the y blocks that z tiles rest on."""
+table layout of the no-allocation entry point, the y blocks that z tiles rest on, and
+the routes that the tests of short dense lines mean to take."""
 import ctypes
 import os
 import random
 import subprocess
 
 import pytest
+
+import dense_line_shapes
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -63,3 +66,18 @@ def test_y_blocks_divide_a_z_tile(rules):
             for lines in (16, 100000):
                 cols = rules.rule_y_block(n, kind, lines)
                 assert cols > 0 and 16 % cols == 0, (n, kind, lines, cols)
+
+
+@pytest.mark.parametrize("kind", dense_line_shapes.KINDS)
+def test_short_dense_line_shapes_take_their_route(rules, kind):
+    number = {k: i for i, k in enumerate(dense_line_shapes.KINDS)}
+    lanes = set()
+    for n in dense_line_shapes.LENGTHS:
+        for (nz, ny, nx), bc, axis, dense in dense_line_shapes.shapes(kind, n):
+            kx, ky = number[bc[:2]], number[bc[2:4]]
+            lines = (nx if axis else ny) * nz
+            got = not rules.rule_plane(nx, ny, kx, ky) and bool(rules.rule_dense(n, (kx, ky)[axis], axis, lines))
+            assert got == dense, (n, (nz, ny, nx), bc, axis)
+            if axis == 0 and dense:
+                lanes.add(rules.rule_stage_lanes(n, kx))
+    assert lanes == {8, 16, 32, 64}
