@@ -126,8 +126,8 @@ bool BatchCore::dense(const BatchMember &m, int a)
     const SolveSetup &g = m.g;
     const int n = a == 0 ? g.nx : a == 1 ? g.ny : g.nz;
     if (!m.dense && n > kMmResident) return false;
-    if (a == 2) return mm_serves(n, KIND_PP, 1, (long)g.nx * g.ny);
-    return mm_serves(n, g.kind[a], a, (long)(a == 0 ? g.ny : g.nx) * g.nz);
+    if (a == 2) return mm_serves(n, KIND_PP, 1, g.nx * g.ny, (long)g.nx * g.ny);
+    return mm_serves(n, g.kind[a], a, g.nx, (long)(a == 0 ? g.ny : g.nx) * g.nz);
 }
 
 std::set<std::pair<int, int>> BatchCore::matrices() const
@@ -257,7 +257,7 @@ int BatchCore::add(int nx, int ny, int nz, const char *bc, const double *X, int 
     const int rc = setup_boundary(m.g, bc);
     if (rc) return rc;
     if (precision == 0 && !zper) {
-        const int ly = line_lines_any<double>(ny, line_route(ny, m.g.kind[1], 1, (long)nx * nz), 1);
+        const int ly = line_lines_any<double>(ny, line_route(ny, m.g.kind[1], 1, nx, (long)nx * nz), 1);
         if (ly <= 0 || zsolve_cpb<double>() % ly != 0) return PP_UNSUPPORTED_SIZE;
     }
     for (int i = 0; i < 6; i++) m.g.X[i] = X[i];

@@ -515,15 +515,31 @@ hipError_t launch_mm_tables(double *out, const double *oct, int N, int kind, hip
 //   101: 8.5 9.1, 7.8 9.1 / 9.0 11.6, 10.9 12.1    201: 12.0 13.8, 10.8 13.0 / 9.2 17.7, 12.0 21.4
 //   401: 25 30, 22 25 / 14 34, 15 45               601: 45 50, 39 45 / 22 58, 27 87
 //   x, quarter-wave (twice the products)  67: 9.7 10.2 / 9.0 11.1    27, 1280 lines: a solve 33.1 / 32.2
+// Columns fill units of 16, the convolution's blocks (8 columns from 129 points on, 4 from 257) less: `wide`
+// is how much more the products pad.  y, a whole solve, dense / chirp, cols x planes:
+//   folded        12x320  401: 0.86  509: 0.96  767: 1.00 1021: 1.43    40x128 1021: 1.18  767: 0.83
+//                 4x960   201: 0.89  254: 0.92  331: 1.14  509: 1.52    8x512   613: 0.85  767: 1.03
+//   quarter-wave  12x320  254: 0.87  331: 1.03  509: 1.44               40x128  331: 0.89  401: 1.07
+//                 4x960   130: 0.87  201: 1.15  331: 1.60               8x512   201: 1.00  254: 1.11
+// lie on either side of n * wide = 1100 (1234 from 513 to 800 points, whose chirps are long) and 400.
 constexpr int kMmMaxN = 1024;
-inline bool mm_serves(int n, int kind, int axis, long lines)
+inline bool mm_columns(int n, bool quarter, int cols)
+{
+    const int block = bs_block_lines<double>(n, 1);
+    const long dense = (cols + 15) / 16 * 16, chirp = (cols + block - 1) / block * block;
+    if (16 * dense <= 17 * chirp) return n <= (quarter ? 512 : kMmMaxN);
+    return n * dense <= (quarter ? 400 : n > 512 && n <= 800 ? 1234 : 1100) * chirp;
+}
+
+// cols: y, the columns of a plane
+inline bool mm_serves(int n, int kind, int axis, int cols, long lines)
 {
     if (line_compiled(n) || n < 2) return false;
     const bool quarter = mm_family(kind) == 1;
     const int any = axis == 1 ? (quarter ? 112 : 208) : quarter ? 0 : 112;  // up to here any number of lines
     if (n > any && lines < (n <= 256 ? 2048 : 3072)) return false;
-    if (quarter) return n <= (axis == 0 ? 280 : 512);
-    return axis == 0 ? n <= 440 || (n > 512 && n <= 620) : n <= kMmMaxN;
+    if (axis == 1) return mm_columns(n, quarter, cols);
+    return quarter ? n <= 280 : n <= 440 || (n > 512 && n <= 620);
 }
 
 // Shape of a launch over `nunits` units of 16 lines / columns.  Two units per wave halve the
@@ -586,9 +602,9 @@ hipError_t launch_line_mm_cfg(const LineArgs &a, hipStream_t s)
 
 // what serves a line: a compiled plan or the chirp convolution, or the dense products
 enum class LineRoute { PLAN, DENSE };
-inline LineRoute line_route(int n, int kind, int axis, long lines)
+inline LineRoute line_route(int n, int kind, int axis, int cols, long lines)
 {
-    return mm_serves(n, kind, axis, lines) ? LineRoute::DENSE : LineRoute::PLAN;
+    return mm_serves(n, kind, axis, cols, lines) ? LineRoute::DENSE : LineRoute::PLAN;
 }
 
 // lines (x) or columns (y) per block of the launch that serves length N (dense x launches take

@@ -27,8 +27,8 @@ struct NoallocTables {
 // lines of axis a (0 x, 1 y; 2 periodic z) that are dense products, or whose matrices the handle would have
 inline bool noalloc_dense(const SolveSetup &g, int a)
 {
-    if (a == 2) return mm_serves(g.nz, KIND_PP, 1, (long)g.nx * g.ny);
-    return mm_serves(a == 0 ? g.nx : g.ny, g.kind[a], a, (long)(a == 0 ? g.ny : g.nx) * g.nz);
+    if (a == 2) return mm_serves(g.nz, KIND_PP, 1, g.nx * g.ny, (long)g.nx * g.ny);
+    return mm_serves(a == 0 ? g.nx : g.ny, g.kind[a], a, g.nx, (long)(a == 0 ? g.ny : g.nx) * g.nz);
 }
 inline bool noalloc_matrices(const SolveSetup &g, int a, bool one_pass)
 {

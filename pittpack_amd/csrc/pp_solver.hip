@@ -76,7 +76,7 @@ hipError_t launch_line(int form, int kind, int N, int AX, int FWD, const LineArg
 {
     // (a batch's line classes bring matrices only to be used; a handle's may be a plane's)
     const long lines = AX == 0 ? a0.nlines : (long)a0.ncols * a0.nplanes;
-    if (a0.mm && (a0.items || mm_serves(N, kind, AX, lines))) {
+    if (a0.mm && (a0.items || mm_serves(N, kind, AX, a0.ncols, lines))) {
         LineArgs a = a0;
         a.n = N;
         switch (kind) {
@@ -318,7 +318,7 @@ int build_tables(pp_solver *h)
     int rc;
     const bool plane = mm_plane(n[0], n[1], h->g.kind[0], h->g.kind[1]);
     for (int a = 0; a < 2; a++) {
-        const bool mm = mm_serves(n[a], h->g.kind[a], a, (long)n[1 - a] * h->g.nz);
+        const bool mm = mm_serves(n[a], h->g.kind[a], a, n[0], (long)n[1 - a] * h->g.nz);
         if ((rc = upload_axis(h, n[a], h->g.kind[a], mm || plane, !mm, h->tab64[a]))) return rc;
     }
     const std::vector<double> lx = eig_factors(h->g, 0), ly = eig_factors(h->g, 1);
@@ -334,7 +334,7 @@ int build_tables(pp_solver *h)
             if ((rc = upload((void **)&h->d_ztw, zt.tw)) || (rc = upload((void **)&h->d_zA, zt.A))) return rc;
         } else {
             // real z-line transforms of length nz (R2HC / HC2R)
-            const bool mm = mm_serves(h->g.nz, KIND_PP, 1, (long)n[0] * n[1]);
+            const bool mm = mm_serves(h->g.nz, KIND_PP, 1, n[0] * n[1], (long)n[0] * n[1]);
             if ((rc = upload_axis(h, h->g.nz, KIND_PP, mm, !mm, h->tabz))) return rc;
         }
         if ((rc = upload((void **)&h->d_zc2, zper_cos2(h->g.nz)))) return rc;
@@ -432,7 +432,7 @@ bool use_ztiles(pp_solver *h)
     } else if (h->zsolver != 0 || (!zsolve_supported_f64(h->g.nz) && !zsolve_long_supported_f64(h->g.nz))) {
         return false;
     }
-    const int ly = line_lines_any<double>(h->g.ny, line_route(h->g.ny, h->g.kind[1], 1, (long)h->g.nx * h->g.nz), 1);
+    const int ly = line_lines_any<double>(h->g.ny, line_route(h->g.ny, h->g.kind[1], 1, h->g.nx, (long)h->g.nx * h->g.nz), 1);
     return ly > 0 && zsolve_cpb<double>() % ly == 0;
 }
 

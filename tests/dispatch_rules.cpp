@@ -11,10 +11,13 @@ static_assert(!std::is_invocable_v<decltype(line_lines_any<double>), int, int, i
 extern "C" {
 
 // 1 dense products, 0 a compiled plan or the chirp convolution
-int rule_dense(int n, int kind, int axis, long lines) { return mm_serves(n, kind, axis, lines); }
+int rule_dense(int n, int kind, int axis, int cols, long lines) { return mm_serves(n, kind, axis, cols, lines); }
 int rule_plane(int nx, int ny, int kx, int ky) { return mm_plane(nx, ny, kx, ky); }
 // columns of an FP64 y block of the launch that serves the line
-int rule_y_block(int n, int kind, long lines) { return line_lines_any<double>(n, line_route(n, kind, 1, lines), 1); }
+int rule_y_block(int n, int kind, int cols, long lines)
+{
+    return line_lines_any<double>(n, line_route(n, kind, 1, cols, lines), 1);
+}
 // lanes a line's staging takes in an x launch
 int rule_stage_lanes(int n, int kind)
 {

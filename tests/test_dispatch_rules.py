@@ -1,6 +1,7 @@
 """Host rules that choose a transform's kernel, compiled for the host alone (tests/dispatch_rules.cpp): the
-table layout of the no-allocation entry point, the y blocks that z tiles rest on, and
-the routes that the tests of short dense lines mean to take."""
+table layout of the no-allocation entry point, the y blocks that z tiles rest on,
+the routes that the tests of short dense lines mean to take, and on which side of the rules the grids lie whose
+two routes have been measured."""
 import ctypes
 import os
 import random
@@ -23,8 +24,8 @@ def rules(tmp_path_factory):
                     "-shared", "-I" + build.SRC, "-I" + os.path.join(ROOT, "include"),
                     os.path.join(HERE, "dispatch_rules.cpp"), "-o", so], check=True, capture_output=True)
     L = ctypes.CDLL(so)
-    L.rule_dense.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long]
-    L.rule_y_block.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_long]
+    L.rule_dense.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long]
+    L.rule_y_block.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long]
     return L
 
 
@@ -63,9 +64,9 @@ def test_y_blocks_divide_a_z_tile(rules):
     """every FP64 y launch's columns fill a 16-column z tile in whole blocks"""
     for n in range(2, 1025):
         for kind in range(5):
-            for lines in (16, 100000):
-                cols = rules.rule_y_block(n, kind, lines)
-                assert cols > 0 and 16 % cols == 0, (n, kind, lines, cols)
+            for nx, lines in ((4, 16), (500, 100000)):
+                cols = rules.rule_y_block(n, kind, nx, lines)
+                assert cols > 0 and 16 % cols == 0, (n, kind, nx, lines, cols)
 
 
 @pytest.mark.parametrize("kind", dense_line_shapes.KINDS)
@@ -76,8 +77,27 @@ def test_short_dense_line_shapes_take_their_route(rules, kind):
         for (nz, ny, nx), bc, axis, dense in dense_line_shapes.shapes(kind, n):
             kx, ky = number[bc[:2]], number[bc[2:4]]
             lines = (nx if axis else ny) * nz
-            got = not rules.rule_plane(nx, ny, kx, ky) and bool(rules.rule_dense(n, (kx, ky)[axis], axis, lines))
+            got = not rules.rule_plane(nx, ny, kx, ky) and bool(rules.rule_dense(n, (kx, ky)[axis], axis, nx, lines))
             assert got == dense, (n, (nz, ny, nx), bc, axis)
             if axis == 0 and dense:
                 lanes.add(rules.rule_stage_lanes(n, kx))
     assert lanes == {8, 16, 32, 64}
+
+
+DD, NN, PP, ND, DN = range(5)
+# (n, kind, axis, other two extents) -> time of a solve with dense lines / with convolutions, on an MI355X
+MEASURED = [
+    # y lines in few columns, which the products pad to 16
+    ((331, NN, 1, 4, 960), 1.14), ((509, NN, 1, 4, 960), 1.52), ((1021, PP, 1, 4, 960), 2.32), ((254, NN, 1, 4, 960), 0.92),
+    ((1021, NN, 1, 12, 320), 1.43), ((401, NN, 1, 12, 320), 0.86), ((1021, PP, 1, 40, 128), 1.18), ((767, PP, 1, 40, 128), 0.83),
+    ((767, NN, 1, 8, 512), 1.03), ((613, NN, 1, 8, 512), 0.85), ((767, NN, 1, 4, 960), 1.69), ((1021, NN, 1, 128, 128), 0.90),
+    ((201, ND, 1, 4, 960), 1.15), ((331, DN, 1, 4, 960), 1.60), ((130, ND, 1, 4, 960), 0.87), ((94, ND, 1, 4, 960), 0.63),
+    ((127, ND, 1, 4, 960), 0.70), ((331, ND, 1, 12, 320), 1.03), ((509, ND, 1, 12, 320), 1.44), ((254, DN, 1, 12, 320), 0.87),
+    ((401, ND, 1, 40, 128), 1.07), ((331, ND, 1, 40, 128), 0.89), ((254, ND, 1, 8, 512), 1.11), ((509, ND, 1, 128, 128), 0.86),
+]
+
+
+def test_the_faster_route(rules):
+    for (n, kind, axis, a, b), ratio in MEASURED:
+        cols, lines = (a, a * b) if axis else (n, a * b)
+        assert bool(rules.rule_dense(n, kind, axis, cols, lines)) == (ratio < 1), (n, kind, axis, a, b, ratio)
