@@ -543,7 +543,10 @@ inline bool mm_serves(int n, int kind, int axis, int cols, long lines)
 }
 
 // Shape of a launch over `nunits` units of 16 lines / columns.  Two units per wave halve the
-// matrix traffic from L2; one where two do not fit LDS or leave CUs without a block.  More
+// matrix traffic from L2; one where two do not fit LDS or leave CUs without waves: a pair of units of short
+// lines is a wave or two (1024 units, a whole solve, us, two / one a wave / convolution: x 19 points 36.4 /
+// 33.1 / 36.0, quarter-wave 39.5 / 34.3 / 36.0, 94 points 55.5 / 51.2 / 71.8; 201 and 331 points 3 and 6 %
+// slower with one).  More
 // units per block while the block stays small (8 waves, 64 KB: two or more blocks per CU, so
 // one block's loads overlap another's products) and three blocks per CU remain.
 struct MmPlan {
@@ -554,15 +557,18 @@ inline MmPlan mm_plan(int N, int kind, int axis, long nunits)
     const int fam = mm_family(kind), KT = mm_rows16(N, fam) / 16;
     const long ub = (long)(mm_unit(N, fam, axis) + (axis == 0 ? mm_xextra : 0)) * 8;
     MmPlan p;
-    p.pw = 2 * ub <= 158 * 1024 && nunits >= 2 * 512 ? 2 : 1;
+    p.pw = 2 * ub <= 158 * 1024 && nunits >= (N <= 64 ? 4096 : N <= 128 ? 2048 : 1024) ? 2 : 1;
     int g = 1;
     while ((g + 1) * KT <= 8 && (g + 1) * p.pw * ub <= 64 * 1024 && nunits >= 768L * (g + 1) * p.pw) g++;
     p.units = g * p.pw;
     const int jobs = g * KT, most = p.units * ub > 80 * 1024 ? 16 : 8;
     const int rounds = (jobs + most - 1) / most;
     p.waves = (jobs + rounds - 1) / rounds;
-    // small lines: enough threads to stage the units
-    while (p.waves < 4 && p.waves * 64 < 32 * p.units) p.waves++;
+    // short lines: enough threads to stage the units, more while units are few (256 units of quarter-wave x
+    // lines of 19 points, a whole solve: 23.8 us with one wave a block, 21.8 with two, the convolution 22.8;
+    // from 4096 units more threads are more waves than the loads need: y lines of 17 points 0.84 -> 0.90 of it)
+    const int per = nunits <= 1024 ? 128 : 32;
+    while (p.waves < 4 && p.waves * 64 < per * p.units) p.waves++;
     return p;
 }
 

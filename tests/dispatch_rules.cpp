@@ -25,6 +25,13 @@ int rule_stage_lanes(int n, int kind)
     return d <= 8 ? 8 : d <= 16 ? 16 : d <= 32 ? 32 : 64;
 }
 
+// waves that a dense launch over `units` units of 16 lines / columns brings to the chip
+long rule_dense_waves(int n, int kind, int axis, long units)
+{
+    const MmPlan p = mm_plan(n, kind, axis, units);
+    return (units + p.units - 1) / p.units * p.waves;
+}
+
 // the layout of the no-allocation entry point: 0 where it does not fit, else a bit for each axis with its
 // matrices; ends[i] of starts[i] .. ends[i]: its sub-arrays (*count of them), in doubles
 int rule_noalloc(int nx, int ny, int nz, const char *bc, int one_pass, long *starts, long *ends, int *count, long *room)

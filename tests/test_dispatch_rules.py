@@ -25,6 +25,8 @@ def rules(tmp_path_factory):
                     os.path.join(HERE, "dispatch_rules.cpp"), "-o", so], check=True, capture_output=True)
     L = ctypes.CDLL(so)
     L.rule_dense.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long]
+    L.rule_dense_waves.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long]
+    L.rule_dense_waves.restype = ctypes.c_long
     L.rule_y_block.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long]
     return L
 
@@ -101,3 +103,13 @@ def test_the_faster_route(rules):
     for (n, kind, axis, a, b), ratio in MEASURED:
         cols, lines = (a, a * b) if axis else (n, a * b)
         assert bool(rules.rule_dense(n, kind, axis, cols, lines)) == (ratio < 1), (n, kind, axis, a, b, ratio)
+
+
+def test_short_dense_lines_bring_waves(rules):
+    """short lines in a thousand units or fewer: at least a wave a unit (with half of that, 1024 units were
+    slower than the convolution)"""
+    for n in list(range(2, 65)) + [65, 94, 127]:
+        for kind in range(5):
+            for axis in (0, 1):
+                for units in (64, 256, 512, 1024):
+                    assert rules.rule_dense_waves(n, kind, axis, units) >= units, (n, kind, axis, units)
