@@ -522,6 +522,10 @@ hipError_t launch_mm_tables(double *out, const double *oct, int N, int kind, hip
 //   quarter-wave  12x320  254: 0.87  331: 1.03  509: 1.44               40x128  331: 0.89  401: 1.07
 //                 4x960   130: 0.87  201: 1.15  331: 1.60               8x512   201: 1.00  254: 1.11
 // lie on either side of n * wide = 1100 (1234 from 513 to 800 points, whose chirps are long) and 400.
+// Lines of a few points fill little of a tile of 16 outputs, so many of them are the convolution's, one
+// thread's each, and 2 points always.  A whole solve, dense / chirp, 4096, 16384, 65536 and 262144 lines:
+//   x   2 points 1.04 1.06 1.04 1.12    5 0.99 1.02 1.01 1.02    13 0.91 0.95 0.91 0.80
+//   y   2 points 1.02 1.01 1.03 1.55    5 0.98 0.97 1.02 1.30    13 0.98 0.95 1.03 1.21    17 0.99 0.92 0.89 0.93
 constexpr int kMmMaxN = 1024;
 inline bool mm_columns(int n, bool quarter, int cols)
 {
@@ -534,7 +538,8 @@ inline bool mm_columns(int n, bool quarter, int cols)
 // cols: y, the columns of a plane
 inline bool mm_serves(int n, int kind, int axis, int cols, long lines)
 {
-    if (line_compiled(n) || n < 2) return false;
+    if (line_compiled(n) || n < 3) return false;
+    if (n < (axis == 1 ? 16 : 8) && lines > (n == 3 ? 4096 : 16384)) return false;
     const bool quarter = mm_family(kind) == 1;
     const int any = axis == 1 ? (quarter ? 112 : 208) : quarter ? 0 : 112;  // up to here any number of lines
     if (n > any && lines < (n <= 256 ? 2048 : 3072)) return false;

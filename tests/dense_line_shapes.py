@@ -20,4 +20,5 @@ def shapes(kind, n):
         out += [((16, n, 128), "NN" + kind + "DN", 1, True), ((23, n, 89), "DD" + kind + "DD", 1, False)]
     else:
         out += [((5, n, 70), "NN" + kind + "DN", 1, True), ((4, n, 67), "DD" + kind + "DD", 1, True)]
-    return out
+    # (two points are the convolution's)
+    return [(s, bc, axis, dense and n > 2) for s, bc, axis, dense in out]
