@@ -515,6 +515,10 @@ hipError_t launch_mm_tables(double *out, const double *oct, int N, int kind, hip
 //   101: 8.5 9.1, 7.8 9.1 / 9.0 11.6, 10.9 12.1    201: 12.0 13.8, 10.8 13.0 / 9.2 17.7, 12.0 21.4
 //   401: 25 30, 22 25 / 14 34, 15 45               601: 45 50, 39 45 / 22 58, 27 87
 //   x, quarter-wave (twice the products)  67: 9.7 10.2 / 9.0 11.1    27, 1280 lines: a solve 33.1 / 32.2
+// Quarter-wave lines along x just short of 256 points have the chirp of 512 at its best: a whole solve, dense /
+// chirp, 2112, 3072, 4096, 16384 and 65536 lines
+//   138: 0.97 0.98 0.86 0.76 0.79    170: 1.02 1.05 0.94 0.88 0.93    201: 1.10 1.09 0.96 0.94 1.00
+//   222: 1.12 1.13 1.01 0.96 1.03    243: 1.15 1.16 1.03 1.00 1.02    271: 1.00 1.02 0.90 0.74 0.78
 // Columns fill units of 16, the convolution's blocks (8 columns from 129 points on, 4 from 257) less: `wide`
 // is how much more the products pad.  y, a whole solve, dense / chirp, cols x planes:
 //   folded        12x320  401: 0.86  509: 0.96  767: 1.00 1021: 1.43    40x128 1021: 1.18  767: 0.83
@@ -542,9 +546,10 @@ inline bool mm_serves(int n, int kind, int axis, int cols, long lines)
     if (n < (axis == 1 ? 16 : 8) && lines > (n == 3 ? 4096 : 16384)) return false;
     const bool quarter = mm_family(kind) == 1;
     const int any = axis == 1 ? (quarter ? 112 : 208) : quarter ? 0 : 112;  // up to here any number of lines
-    if (n > any && lines < (n <= 256 ? 2048 : 3072)) return false;
+    if (n > any && lines < (axis == 0 && quarter && n > 150 ? 4096 : n <= 256 ? 2048 : 3072)) return false;
     if (axis == 1) return mm_columns(n, quarter, cols);
-    return quarter ? n <= 280 : n <= 440 || (n > 512 && n <= 620);
+    if (quarter) return n <= 232 || (n > 256 && n <= 280);
+    return n <= 440 || (n > 512 && n <= 620);
 }
 
 // Shape of a launch over `nunits` units of 16 lines / columns.  Two units per wave halve the
