@@ -552,11 +552,14 @@ inline bool mm_serves(int n, int kind, int axis, int cols, long lines)
     return n <= 440 || (n > 512 && n <= 620);
 }
 
-// Shape of a launch over `nunits` units of 16 lines / columns.  Two units per wave halve the
-// matrix traffic from L2; one where two do not fit LDS or leave CUs without waves: a pair of units of short
-// lines is a wave or two (1024 units, a whole solve, us, two / one a wave / convolution: x 19 points 36.4 /
-// 33.1 / 36.0, quarter-wave 39.5 / 34.3 / 36.0, 94 points 55.5 / 51.2 / 71.8; 201 and 331 points 3 and 6 %
-// slower with one).  More
+// Shape of a launch over `nunits` units of 16 lines / columns.  One unit a wave: two halve the matrix traffic
+// from L2, but half as many blocks end in emptier last rounds, and short lines are left with too few waves.  A
+// whole solve, two / one a wave, over the convolution's time, 1056, 2046 and 4092 units (ND: quarter-wave):
+//   x   19 0.96/0.91 0.94/0.89 0.88/0.84   185 ND 1.12/0.93 0.94/0.89 0.97/0.87   331 0.82/0.76 0.66/0.68 0.69/0.72
+//   y   67 0.61/0.59 0.50/0.54 0.51/0.47   201 ND 0.82/0.72 0.76/0.69 0.70/0.66   439 0.72/0.63 0.65/0.60 0.55/0.56
+// Two are faster at 4096 units and more of folded lines of 113 to 256 points (x 254 points 0.81/0.85, y 127 points
+// at 16384 0.54/0.58, but 67 points 0.62/0.63, 300 points 0.69/0.62), and where their block has a CU of its own,
+// with up to 16 waves, as long as its rounds over the CUs are as full (x 331 points, 1536 units 0.68/0.72).  More
 // units per block while the block stays small (8 waves, 64 KB: two or more blocks per CU, so
 // one block's loads overlap another's products) and three blocks per CU remain.
 struct MmPlan {
@@ -567,7 +570,9 @@ inline MmPlan mm_plan(int N, int kind, int axis, long nunits)
     const int fam = mm_family(kind), KT = mm_rows16(N, fam) / 16;
     const long ub = (long)(mm_unit(N, fam, axis) + (axis == 0 ? mm_xextra : 0)) * 8;
     MmPlan p;
-    p.pw = 2 * ub <= 158 * 1024 && nunits >= (N <= 64 ? 4096 : N <= 128 ? 2048 : 1024) ? 2 : 1;
+    const bool whole = nunits >= 1024 && (nunits + 511) / 512 * 2 <= (nunits + 255) / 256;  // two cost no round more
+    const bool pair = N > 256 ? 2 * ub > 80 * 1024 && 2 * ub <= 158 * 1024 && whole : N > 112 && nunits >= 4096;
+    p.pw = fam != 1 && pair ? 2 : 1;
     int g = 1;
     while ((g + 1) * KT <= 8 && (g + 1) * p.pw * ub <= 64 * 1024 && nunits >= 768L * (g + 1) * p.pw) g++;
     p.units = g * p.pw;

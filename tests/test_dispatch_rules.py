@@ -114,10 +114,10 @@ def test_the_faster_route(rules):
 
 
 def test_short_dense_lines_bring_waves(rules):
-    """short lines in a thousand units or fewer: at least a wave a unit (with half of that, 1024 units were
+    """at least a wave a unit (with half of that, 1024 units of short lines and 1056 of quarter-wave ones were
     slower than the convolution)"""
-    for n in list(range(2, 65)) + [65, 94, 127]:
+    for n in list(range(2, 65)) + [65, 94, 127, 170, 201]:
         for kind in range(5):
             for axis in (0, 1):
-                for units in (64, 256, 512, 1024):
+                for units in (64, 256, 512, 1024, 1056):
                     assert rules.rule_dense_waves(n, kind, axis, units) >= units, (n, kind, axis, units)
