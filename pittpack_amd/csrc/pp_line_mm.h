@@ -36,6 +36,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <type_traits>
 
 #include "pp_line.h"
@@ -519,24 +520,36 @@ hipError_t launch_mm_tables(double *out, const double *oct, int N, int kind, hip
 // chirp, 2112, 3072, 4096, 16384 and 65536 lines
 //   138: 0.97 0.98 0.86 0.76 0.79    170: 1.02 1.05 0.94 0.88 0.93    201: 1.10 1.09 0.96 0.94 1.00
 //   222: 1.12 1.13 1.01 0.96 1.03    243: 1.15 1.16 1.03 1.00 1.02    271: 1.00 1.02 0.90 0.74 0.78
-// Columns fill units of 16, the convolution's blocks (8 columns from 129 points on, 4 from 257) less: `wide`
-// is how much more the products pad.  y, a whole solve, dense / chirp, cols x planes:
+// Columns fill units of 16, the convolution's blocks (8 columns from 129 points on, 4 from 257) less, and the
+// units of long lines go over the CUs in rounds of 256: mm_stretch is how much longer the products take for both.
+// y, a whole solve, dense / chirp, cols x planes:
 //   folded        12x320  401: 0.86  509: 0.96  767: 1.00 1021: 1.43    40x128 1021: 1.18  767: 0.83
 //                 4x960   201: 0.89  254: 0.92  331: 1.14  509: 1.52    8x512   613: 0.85  767: 1.03
 //   quarter-wave  12x320  254: 0.87  331: 1.03  509: 1.44               40x128  331: 0.89  401: 1.07
 //                 4x960   130: 0.87  201: 1.15  331: 1.60               8x512   201: 1.00  254: 1.11
-// lie on either side of n * wide = 1100 (1234 from 513 to 800 points, whose chirps are long) and 400.
+// and whole units, 256, 264, 384 and 512 of them (rounds 1.00, 1.94, 1.33 and 1.00 times as long as they are full):
+//   y folded  767: 0.63 0.89 0.73 0.64    1021: 0.90 1.30 1.05 0.90    quarter-wave 331: 0.78 0.88 0.79 0.67
+//   x folded  371: 0.88 1.07 0.93 0.80     613: 0.91 1.24 0.99 0.84    quarter-wave 509: 0.95 1.22 1.08 0.94 (y)
+//   x quarter-wave  185: 0.96 1.10 1.02 0.90    213: 0.98 1.13 1.04 0.94    280: 0.92 1.03 0.89 0.77
 // Lines of a few points fill little of a tile of 16 outputs, so many of them are the convolution's, one
 // thread's each, and 2 points always.  A whole solve, dense / chirp, 4096, 16384, 65536 and 262144 lines:
 //   x   2 points 1.04 1.06 1.04 1.12    5 0.99 1.02 1.01 1.02    13 0.91 0.95 0.91 0.80
 //   y   2 points 1.02 1.01 1.03 1.55    5 0.98 0.97 1.02 1.30    13 0.98 0.95 1.03 1.21    17 0.99 0.92 0.89 0.93
 constexpr int kMmMaxN = 1024;
-inline bool mm_columns(int n, bool quarter, int cols)
+inline double mm_stretch(int axis, int cols, long lines, int block)
+{
+    if (axis == 0) return (double)((lines + 4095) / 4096) * 4096 / lines;
+    const long units = (long)((cols + 15) / 16) * (lines / cols);
+    return (double)((units + 255) / 256) * 4096 / ((double)((cols + block - 1) / block * block) * (lines / cols));
+}
+inline bool mm_columns(int n, bool quarter, int cols, long lines)
 {
     const int block = bs_block_lines<double>(n, 1);
     const long dense = (cols + 15) / 16 * 16, chirp = (cols + block - 1) / block * block;
-    if (16 * dense <= 17 * chirp) return n <= (quarter ? 512 : kMmMaxN);
-    return n * dense <= (quarter ? 400 : n > 512 && n <= 800 ? 1234 : 1100) * chirp;
+    if (n <= 256) return n * dense <= (quarter ? 400 : 1100) * chirp;  // (rounds tell less of them)
+    const double s = mm_stretch(1, cols, lines, block);
+    if (quarter) return n <= 512 && n * std::sqrt((double)n) * s <= 11900;
+    return n <= 512 ? n * s <= 1100 : (double)n * n * s <= 1.17e6;
 }
 
 // cols: y, the columns of a plane
@@ -547,9 +560,11 @@ inline bool mm_serves(int n, int kind, int axis, int cols, long lines)
     const bool quarter = mm_family(kind) == 1;
     const int any = axis == 1 ? (quarter ? 112 : 208) : quarter ? 0 : 112;  // up to here any number of lines
     if (n > any && lines < (axis == 0 && quarter && n > 150 ? 4096 : n <= 256 ? 2048 : 3072)) return false;
-    if (axis == 1) return mm_columns(n, quarter, cols);
-    if (quarter) return n <= 232 || (n > 256 && n <= 280);
-    return n <= 440 || (n > 512 && n <= 620);
+    if (axis == 1) return mm_columns(n, quarter, cols, lines);
+    if (n <= (quarter ? 150 : 256)) return true;
+    const double s = n * mm_stretch(0, 0, lines, 1);
+    if (quarter) return n <= 232 ? s <= 255 : n > 256 && n <= 280 && s <= 500;
+    return n <= 440 ? s <= 560 : n > 512 && n <= 620 && s <= 842;
 }
 
 // Shape of a launch over `nunits` units of 16 lines / columns.  One unit a wave: two halve the matrix traffic

@@ -41,7 +41,7 @@ def layout(rules, nx, ny, nz, bc, one_pass):
 def test_noalloc_axes_keep_the_matrices_that_fit(rules):
     """one axis whose matrices do not fit does not cost the others theirs"""
     for shape, bc, axes in (((101, 509, 97), "DDNNDD", 1), ((509, 101, 97), "NNDDDD", 2), ((101, 97, 331), "NNNNPP", 3 | 4),
-                            ((331, 331, 331), "PPPPPP", 1 | 2 | 4), ((439, 1021, 9), "NNNNDD", 1), ((24, 20, 18), "NNDDDD", 3),
+                            ((331, 331, 331), "PPPPPP", 1 | 2 | 4), ((401, 1021, 8), "NNNNDD", 1), ((24, 20, 18), "NNDDDD", 3),
                             ((64, 64, 701), "NNNNPP", 4), ((64, 64, 767), "NNNNPP", 0)):
         bits = layout(rules, *shape, bc, False)[0]
         assert bits & 8 and bits & 7 == axes, (shape, bc, bits & 7)
@@ -100,6 +100,14 @@ MEASURED = [
     ((201, ND, 0, 96, 22), 1.10), ((254, ND, 0, 96, 24), 1.16), ((255, DN, 0, 128, 32), 1.05), ((254, ND, 0, 512, 128), 1.05),
     ((185, DN, 0, 96, 32), 1.07), ((279, ND, 0, 96, 32), 1.05), ((201, ND, 0, 128, 64), 0.93), ((222, ND, 0, 128, 128), 0.96),
     ((138, ND, 0, 96, 22), 0.97), ((271, ND, 0, 128, 64), 0.75), ((254, NN, 0, 96, 32), 0.98),
+    # units in rounds of 256
+    ((767, NN, 1, 96, 44), 0.89), ((1021, NN, 1, 96, 44), 1.30), ((1021, PP, 1, 96, 64), 1.05), ((1021, NN, 1, 96, 42), 0.90),
+    ((897, NN, 1, 96, 53), 1.10), ((897, NN, 1, 96, 74), 0.87), ((613, NN, 1, 96, 44), 0.75), ((509, NN, 1, 96, 44), 0.84),
+    ((331, ND, 1, 96, 44), 0.88), ((401, DN, 1, 96, 44), 1.06), ((509, ND, 1, 96, 64), 1.08), ((509, ND, 1, 96, 85), 0.94),
+    ((371, NN, 0, 96, 44), 1.07), ((371, NN, 0, 96, 64), 0.93), ((439, PP, 0, 96, 48), 1.14), ((439, NN, 0, 96, 74), 0.92),
+    ((613, NN, 0, 96, 44), 1.24), ((613, DD, 0, 96, 85), 0.84), ((523, NN, 0, 96, 44), 1.08), ((331, NN, 0, 96, 53), 0.93),
+    ((185, ND, 0, 96, 44), 1.10), ((185, ND, 0, 96, 85), 0.90), ((213, DN, 0, 96, 88), 1.05), ((280, ND, 0, 96, 44), 1.03),
+    ((280, ND, 0, 96, 64), 0.89), ((155, ND, 0, 96, 64), 0.91),
     # very short lines
     ((2, NN, 0, 128, 32), 1.04), ((2, PP, 1, 512, 512), 1.55), ((3, ND, 1, 512, 512), 1.31), ((4, NN, 0, 512, 512), 1.07),
     ((5, NN, 1, 128, 128), 0.97), ((7, NN, 1, 512, 512), 1.22), ((13, ND, 1, 512, 512), 1.15), ((15, PP, 1, 512, 128), 1.06),
