@@ -924,6 +924,13 @@ constexpr int line_threads_alt(int M)
 // 48x512x512 740 : 658, 128x128x128 149 : 145).
 constexpr bool line_wide(int M, int AX) { return line_threads_alt(M) > 0 && (M <= 40 || (M == 64 && AX == 0)); }
 
+// ... but the corrections' x forward, fused with the residual (pp_resx.h) or not, with the same rounding in both,
+// keeps the first shape at 64 and 128 points: four elements a thread leave the fused kernel's residual quads
+// waiting for each other behind a block twice the size (us, first and second step, eight / four elements: 128
+// points 22 27 / 25 28, in a batch 59 66 / 63 103; 64 points 25 31 / 27 32, in a batch 59 72 / 64 110; by itself
+// the transform is within 3 % of the other shape's time, in a batch 3 to 10 % faster)
+constexpr bool line_wide_correction(int M) { return line_wide(M, 0) && M != 32 && M != 64; }
+
 template <typename R, int M, int AX, int T = line_threads(M, AX)>
 constexpr int line_lines()
 {
@@ -983,7 +990,7 @@ template <typename TIn, typename TOut, typename R, int M, int AX, int FWD, int K
 hipError_t launch_line_cfg(const LineArgs &a, hipStream_t s)
 {
     // FP32 lines take the shape that is FP64's default, with the first one's lines per block
-    constexpr bool W32 = sizeof(R) == 4 && line_wide(M, AX);
+    constexpr bool W32 = sizeof(R) == 4 && (AX == 0 && FWD && sizeof(TIn) == 4 ? line_wide_correction(M) : line_wide(M, AX));
     constexpr int T = V || W32 ? line_threads_alt(M) : line_threads(M, AX);
     if constexpr (T == 0) {
         return hipErrorInvalidValue;

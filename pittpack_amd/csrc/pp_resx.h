@@ -326,11 +326,13 @@ __global__ void __launch_bounds__(T *LINES, (resx_waves<M, T, LINES, BATCH>())) 
     line_body<float, float, float, M, T, LINES, 0, 1, KIND>(a, ad, t, L, xin, lds, (long)bx * LINES);
 }
 
+// threads a line: the unfused transform's (line_wide_correction)
+constexpr int resx_threads(int M) { return line_wide_correction(M) ? line_threads_alt(M) : line_threads(M, 0); }
+
 template <int M, int KIND, int SRC>
 hipError_t launch_resx_cfg(const LineArgs &a, const ResArgs &r, const ResArgs *rsolves, hipStream_t s)
 {
-    // the unfused transform's shape
-    constexpr int T = line_wide(M, 0) ? line_threads_alt(M) : line_threads(M, 0);
+    constexpr int T = resx_threads(M);
     if constexpr (T == 0) {
         return hipErrorInvalidValue;
     } else {

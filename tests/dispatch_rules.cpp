@@ -2,6 +2,7 @@
 #include <type_traits>
 
 #include "pp_noalloc.h"
+#include "pp_resx.h"
 
 using namespace pp;
 
@@ -31,6 +32,9 @@ long rule_dense_waves(int n, int kind, int axis, long units)
     const MmPlan p = mm_plan(n, kind, axis, units);
     return (units + p.units - 1) / p.units * p.waves;
 }
+
+// elements a thread holds of a line of n points in the fused correction step
+int rule_resx_elements(int n) { return n / 2 / resx_threads(n / 2); }
 
 // the layout of the no-allocation entry point: 0 where it does not fit, else a bit for each axis with its
 // matrices; ends[i] of starts[i] .. ends[i]: its sub-arrays (*count of them), in doubles

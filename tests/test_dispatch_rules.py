@@ -129,3 +129,9 @@ def test_short_dense_lines_bring_waves(rules):
             for axis in (0, 1):
                 for units in (64, 256, 512, 1024, 1056):
                     assert rules.rule_dense_waves(n, kind, axis, units) >= units, (n, kind, axis, units)
+
+
+def test_fused_correction_shapes(rules):
+    """elements a thread holds of a line in the fused correction step, as measured: eight of 64 and 128 points
+    (four: up to 1.6 times slower), half of what the narrow shape has of 32 and 80"""
+    assert [rules.rule_resx_elements(n) for n in (32, 64, 80, 128, 256, 512)] == [4, 8, 10, 8, 8, 8]
