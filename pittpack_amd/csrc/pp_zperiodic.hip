@@ -25,6 +25,7 @@
 #include "pp_fft.h"
 #include "pp_launch.h"
 #include "pp_line.h"
+#include "pp_zper.h"
 #include "pp_zsing.h"
 #include "pp_zsolve.h"
 
@@ -51,7 +52,7 @@ __global__ void __launch_bounds__(T *LINES, (zper_min_waves<M, T, LINES>())) k_z
 {
     using R = double;
     constexpr int E = M / T;
-    constexpr int LS = line_slots<M>();
+    constexpr int LS = zper_slots<M>();
     extern __shared__ __align__(16) unsigned char smem_zp[];
     cpx<R> *lds = reinterpret_cast<cpx<R> *>(smem_zp);
     const int tid = threadIdx.x;
@@ -194,29 +195,13 @@ __global__ void k_smt_v1_batch(double *data, const SmtItem *items)
     smt_v1_body(data + it.offset, it.stride, it.nz, it.diag);
 }
 
-// The half lengths M = nz / 2: the line transforms' and, whole in one thread's registers, 5 and 7
-// (columns of 10 and 14 points, us a whole solve, one pass : z-line transforms: 512x512x10 77.7 : 148,
-// 512x512x14 83.7 : 139, 64x64x10 21.1 : 27.7; 200 members of 24x24x10 in a batch, whose z-line transforms are
-// three launches of each member's own, 50.9 : 1687)
-#define PP_ZPER_LENGTHS(X) X(5) X(7) PP_FFT_LENGTHS(X)
-constexpr int zper_threads(int M) { return M == 5 || M == 7 ? 1 : line_threads(M, 1); }
-
-// columns per block: 16 (128-byte FP64 rows) while the slices fit 80 KB, 8 for longer lines, as
-// the y transforms on the field in place
-template <int M>
-constexpr int zper_lines_m()
-{
-    constexpr int L = line_lines<double, M, 1, zper_threads(M)>();
-    return zper_threads(M) >= 64 && L > 8 ? 8 : L;
-}
-
 // grid: column blocks x SY (one solve), or nitems blocks (batched, a.items set)
 template <typename S, int M>
 static hipError_t launch_zper_m(const ZPerArgs &a, int nitems, hipStream_t s)
 {
     constexpr int T = zper_threads(M);
     constexpr int LINES = zper_lines_m<M>();
-    const size_t lds = (size_t)LINES * line_slots<M>() * sizeof(cpx<double>);
+    const size_t lds = (size_t)LINES * zper_slots<M>() * sizeof(cpx<double>);
     auto kern = k_zper<S, M, T, LINES>;
     if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -3,6 +3,7 @@
 
 #include "pp_noalloc.h"
 #include "pp_resx.h"
+#include "pp_zper.h"
 
 using namespace pp;
 
@@ -33,6 +34,16 @@ long rule_dense_waves(int n, int kind, int axis, long units)
     return (units + p.units - 1) / p.units * p.waves;
 }
 
+// threads a block, and LDS slots a column, of the one-pass periodic z solve of nz rows (0: other lengths)
+int rule_zper(int nz, int *slots)
+{
+    switch (nz / 2) {
+#define PPM(m) case m: *slots = zper_slots<m>(); return zper_threads(m) * zper_lines_m<m>();
+        PP_ZPER_LENGTHS(PPM)
+#undef PPM
+    default: return 0;
+    }
+}
 // elements a thread holds of a line of n points in the fused correction step
 int rule_resx_elements(int n) { return n / 2 / resx_threads(n / 2); }
 

@@ -135,3 +135,11 @@ def test_fused_correction_shapes(rules):
     """elements a thread holds of a line in the fused correction step, as measured: eight of 64 and 128 points
     (four: up to 1.6 times slower), half of what the narrow shape has of 32 and 80"""
     assert [rules.rule_resx_elements(n) for n in (32, 64, 80, 128, 256, 512)] == [4, 8, 10, 8, 8, 8]
+
+
+def test_periodic_z_blocks_are_whole_waves(rules):
+    slots = ctypes.c_int(0)
+    served = [nz for nz in range(8, 1025, 2) if rules.rule_zper(nz, ctypes.byref(slots))]
+    assert len(served) == 29 and served[:4] == [8, 10, 12, 14]
+    for nz in served:
+        assert rules.rule_zper(nz, ctypes.byref(slots)) % 64 == 0, nz

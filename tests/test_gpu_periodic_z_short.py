@@ -1,6 +1,7 @@
-"""Periodic z of 10 and 14 points: half a length of 5 or 7, held by one thread, in the one-pass kernel
-(no line transform of those lengths is compiled), where it can go wrong: ragged x extents, with and
-without a singular column, every form, and a batch's members in one launch of their class.
+"""Short periodic z in the one-pass kernel, whose blocks take as many columns as fill a wave, and 10 and 14
+points, half a length of 5 or 7 held by one thread (no line transform of those lengths is compiled), where they
+can go wrong: ragged x extents, with and without a singular column, every form, and a batch's members in one
+launch of their class.
 
 Bar: max-norm difference <= 1e-12 relative to max|u_oracle|, the FP64 bar of every parity test; batch
 members bitwise the single solves."""
@@ -14,8 +15,8 @@ from pittpack_amd import rng as prng
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nz", [8, 10, 12, 14])
-@pytest.mark.parametrize("nx", [16, 23, 70])
+@pytest.mark.parametrize("nz", [8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 56, 80])
+@pytest.mark.parametrize("nx", [16, 23, 70, 130])
 def test_short_periodic_z(nx, nz):
     box = [0, 1, 0, 1, 0, nz / 16.0]
     for bc in ("PPPPPP", "DDNNPP", "NDDNPP"):
@@ -29,7 +30,7 @@ def test_short_periodic_z(nx, nz):
 
 
 @pytest.mark.parametrize("precision", [0, 1])
-@pytest.mark.parametrize("nz", [10, 14])
+@pytest.mark.parametrize("nz", [10, 14, 16, 24, 48])
 def test_short_periodic_z_members_share_a_launch(nz, precision):
     shapes = [(nz, 24, 24), (nz, 18, 23), (nz, 30, 66), (nz, 16, 16)]
     print(f"short periodic z batch nz={nz} precision={precision}", flush=True)
