@@ -23,8 +23,10 @@ constexpr int zper_lines_m()
     return T >= 64 && L > 8 ? 8 : T < 4 ? 64 / T : L;
 }
 
-// LDS slots of a column
+// LDS slots of a column: an odd number, so that the 16 columns of a wave's access start on different banks (z stage,
+// us, with the line transforms' number / odd: 112 elements, whose 120 slots start on two, 512x512x224 582 323 and
+// 20x240x224 32.9 22.4, where full-length lines took 584 and 25.2; 56 elements, 60 slots, 512x512x112 138 109)
 template <int M>
-constexpr int zper_slots() { return line_slots<M>(); }
+constexpr int zper_slots() { return line_slots<M>() | 1; }
 
 }  // namespace pp

@@ -137,9 +137,11 @@ def test_fused_correction_shapes(rules):
     assert [rules.rule_resx_elements(n) for n in (32, 64, 80, 128, 256, 512)] == [4, 8, 10, 8, 8, 8]
 
 
-def test_periodic_z_blocks_are_whole_waves(rules):
+def test_periodic_z_blocks_are_whole_waves_on_all_banks(rules):
     slots = ctypes.c_int(0)
     served = [nz for nz in range(8, 1025, 2) if rules.rule_zper(nz, ctypes.byref(slots))]
     assert len(served) == 29 and served[:4] == [8, 10, 12, 14]
     for nz in served:
         assert rules.rule_zper(nz, ctypes.byref(slots)) % 64 == 0, nz
+        # 16 columns' first elements on the 64 banks, four banks each
+        assert len({4 * slots.value * col % 64 for col in range(16)}) == 16, (nz, slots.value)
