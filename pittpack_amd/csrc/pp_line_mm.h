@@ -526,6 +526,7 @@ hipError_t launch_mm_tables(double *out, const double *oct, int N, int kind, hip
 //   folded        12x320  401: 0.86  509: 0.96  767: 1.00 1021: 1.43    40x128 1021: 1.18  767: 0.83
 //                 4x960   201: 0.89  254: 0.92  331: 1.14  509: 1.52    8x512   613: 0.85  767: 1.03
 //   quarter-wave  12x320  254: 0.87  331: 1.03  509: 1.44               40x128  331: 0.89  401: 1.07
+//                 20x160  250: 1.10                                     20x200  254: 0.87
 //                 4x960   130: 0.87  201: 1.15  331: 1.60               8x512   201: 1.00  254: 1.11
 // and whole units, 256, 264, 384 and 512 of them (rounds 1.00, 1.94, 1.33 and 1.00 times as long as they are full):
 //   y folded  767: 0.63 0.89 0.73 0.64    1021: 0.90 1.30 1.05 0.90    quarter-wave 331: 0.78 0.88 0.79 0.67
@@ -545,8 +546,12 @@ inline double mm_stretch(int axis, int cols, long lines, int block)
 inline bool mm_columns(int n, bool quarter, int cols, long lines)
 {
     const int block = bs_block_lines<double>(n, 1);
-    const long dense = (cols + 15) / 16 * 16, chirp = (cols + block - 1) / block * block;
-    if (n <= 256) return n * dense <= (quarter ? 400 : 1100) * chirp;  // (rounds tell less of them)
+    if (n <= 256) {
+        // (rounds tell less: of shorter lines more than one block runs on a CU; few units leave either idle)
+        const long dense = (cols + 15) / 16 * 16, chirp = (cols + block - 1) / block * block, units = dense / 16 * (lines / cols);
+        const double rounds = units <= 256 ? 1.0 : (double)((units + 255) / 256 * 256) / units;
+        return quarter ? n * dense * (0.4 + 0.6 * rounds) <= 410 * chirp : n * dense <= 1100 * chirp;
+    }
     const double s = mm_stretch(1, cols, lines, block);
     if (quarter) return n <= 512 && n * std::sqrt((double)n) * s <= 11900;
     return n <= 512 ? n * s <= 1100 : (double)n * n * s <= 1.17e6;

@@ -96,6 +96,7 @@ MEASURED = [
     ((201, ND, 1, 4, 960), 1.15), ((331, DN, 1, 4, 960), 1.60), ((130, ND, 1, 4, 960), 0.87), ((94, ND, 1, 4, 960), 0.63),
     ((127, ND, 1, 4, 960), 0.70), ((331, ND, 1, 12, 320), 1.03), ((509, ND, 1, 12, 320), 1.44), ((254, DN, 1, 12, 320), 0.87),
     ((401, ND, 1, 40, 128), 1.07), ((331, ND, 1, 40, 128), 0.89), ((254, ND, 1, 8, 512), 1.11), ((509, ND, 1, 128, 128), 0.86),
+    ((250, ND, 1, 20, 160), 1.10), ((193, ND, 1, 8, 296), 1.03), ((254, ND, 1, 20, 200), 0.87), ((201, ND, 1, 96, 44), 0.85),
     # quarter-wave x lines
     ((201, ND, 0, 96, 22), 1.10), ((254, ND, 0, 96, 24), 1.16), ((255, DN, 0, 128, 32), 1.05), ((254, ND, 0, 512, 128), 1.05),
     ((185, DN, 0, 96, 32), 1.07), ((279, ND, 0, 96, 32), 1.05), ((201, ND, 0, 128, 64), 0.93), ((222, ND, 0, 128, 128), 0.96),
