@@ -195,7 +195,7 @@ def bench_batched(pa, count: int, steps: int, refine: int, sample: int = 8, auto
             B.solve()
         kt = B.kernel_times()
         m, pts = B.count()
-        launches = B.launch_count()
+        classes = B.launch_count()
         key = "fp64" if prec == 0 else "mixed"
         sols = {i: B.get_solution(i) for i in picks}
         errs_o = []
@@ -207,7 +207,7 @@ def bench_batched(pa, count: int, steps: int, refine: int, sample: int = 8, auto
             errs_o.append(float(np.abs(sols[i] - o).max() / np.abs(o).max()))
         if prec == 0:
             ref = sols
-        res = {"ms_per_step": ms, "value": pts / (ms * 1e-3), "launches_per_stage_xyz": launches,
+        res = {"ms_per_step": ms, "value": pts / (ms * 1e-3), "shape_classes_per_stage_xyz": classes,
                "plan_and_upload_s": plan_s, "hip_graph": True, "kernels_ms": kt}
         res["oracle_checked_members"] = len(picks)
         res["rel_max_diff_vs_oracle_max"] = max(errs_o)

@@ -98,8 +98,8 @@ enum {
      * configuration. */
     PP_OPT_AUTOTUNE = 11,
     /* testing: force every FP64 line stage (and the mixed form's FP32 tiled y stages) to the
-     * default (0) or alternative (1) launch shape where it has one; -1 (default) = the
-     * autotuner's choice */
+     * default (0) or alternative (1) launch shape where it has one, and small planes to the line
+     * stages (batches: those not yet finalized); -1 (default) = the autotuner's choice */
     PP_OPT_LINE_VARIANT = 12,
     /* server: how many admitted batches may overtake a queued request that does not fit
      * before nothing behind it is admitted (default 4); bounds the wait of large requests
@@ -125,7 +125,9 @@ enum {
 };
 
 /* PencilDcmp(argc, argv, nx, ny, nz) / make_Poisson (src/pencilDcmp.cpp:232-452,6432-6440).
- * Global grid sizes (one GPU holds the whole grid).  Allocates the device field. */
+ * Global grid sizes (one GPU holds the whole grid).  Allocates the device field.  Tables follow with
+ * the first solve: below 0.5 MB a line length, and where its lines are dense products their matrices,
+ * some 8 n^2 bytes (8 MB at n = 1021; the real DFT half of that). */
 int pp_create(int nx, int ny, int nz, pp_handle *out);
 
 /* ~PencilDcmp (src/pencilDcmp.cpp:528-658) */
@@ -227,8 +229,9 @@ int pp_set_option(pp_handle h, int key, long long value);
 int pp_set_option_double(pp_handle h, int key, double value);
 
 /* Mean durations (ms) of the five stages of the FP64 form over the solves recorded since
- * the last call: x forward, y forward, z solve, y inverse, x inverse.  Requires
- * PP_OPT_TIMING.  Synchronises the handle's stream. */
+ * the last call: x forward, y forward, z solve, y inverse, x inverse.  Small planes (at most
+ * 64 x 64 points) run x and y in one launch: its time counts as the x stage's, the y stage's is
+ * about zero.  Requires PP_OPT_TIMING.  Synchronises the handle's stream. */
 int pp_get_stage_times(pp_handle h, float *ms5);
 
 /* Mean durations (ms) between consecutive kernel launches of the recorded solves (any
@@ -301,8 +304,10 @@ int pp_batch_destroy(pp_batch b);
 int pp_batch_add(pp_batch b, int nx, int ny, int nz, const char *bc, const double *X, int *id);
 int pp_batch_finalize(pp_batch b);
 int pp_batch_count(pp_batch b, int *members, long long *points);
-/* shape classes per stage: x, y, z.  A stage runs as one launch per class; FP64 members with
- * small planes (at most 64 x 64 points) share launches for both x and y, whatever their classes */
+/* shape classes per stage: x, y, z, distinct lengths and kinds of x and y lines and rows of z columns (the
+ * launches of a stage where no class splits: lines of one length as dense products and as convolutions are
+ * two launches, and so are z columns of one length by either z kernel; FP64 members with small planes, at most
+ * 64 x 64 points, share launches for both x and y, whatever their classes) */
 int pp_batch_launch_count(pp_batch b, int *per_stage3);
 /* device pointers of a member's right-hand side and solution (nx*ny*nz doubles each) */
 int pp_batch_field(pp_batch b, int id, double **d_rhs);

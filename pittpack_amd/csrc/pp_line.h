@@ -919,7 +919,8 @@ constexpr int line_threads_alt(int M)
 //                                 48 points 43.7 / 61.3 : 36.8 / 39.1   80  88.0 / 131 : 74.7 / 67.1
 //   x, 32 x 64 rows               48 points 11.1 / 11.1 : 9.0 / 9.1     64   8.6 /  9.0 :  7.2 /  7.4
 //   x, 128 points                 128 x 64 rows 10.2 / 12.7 : 9.2 / 11.1, 512 x 512 rows 104 / 102 : 107 / 87
-// At 256 and 512 points the shapes are within 5 % of each other; y lines of 128 points within 4 %.
+// At 256 and 512 points the shapes are within 5 % of each other; y lines of 128 points within 4 %.  96, 112 and 160
+// points have no second shape (make_plan: their plans would grow by two passes, or have none).
 // The FP32 lines of the mixed form take it at the same lengths (a whole mixed solve of 80x80x80 204 : 167,
 // 48x512x512 740 : 658, 128x128x128 149 : 145).
 constexpr bool line_wide(int M, int AX) { return line_threads_alt(M) > 0 && (M <= 40 || (M == 64 && AX == 0)); }

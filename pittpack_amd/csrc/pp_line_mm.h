@@ -12,7 +12,7 @@
 //   PP inverse       e_n from the real, o_n from the imaginary parts; x_n, x_{N-n} = e_n +- o_n
 //   ND / DN          no such symmetry: the two halves of the outputs, each from the whole line
 //
-// so a line costs N multiply-adds per point (2 N quarter-wave), all of them on the matrix cores
+// so a line costs N / 2 multiply-adds per point (N quarter-wave), all of them on the matrix cores
 // (v_mfma_f64_16x16x4: 68 TFLOP/s measured, about 45 on full-entropy data, whose power lowers the
 // clock), where the chirp convolution (pp_line_bs.h) spends two complex FFTs of 2 to 4 N points
 // on every real line.  The sum runs in two interleaved chains, which keeps its rounding below
@@ -27,8 +27,8 @@
 //
 // A block stages `tiles` units of 16 lines (x) or 16 columns of one plane (y), folded, in LDS
 // (so the fused input scaling, the Dirichlet term and the line sums happen on the way in), then
-// its waves take output row tiles of 16: two accumulator sets (e and o) per unit, PW units per
-// wave, so that one matrix element loaded from L2 feeds PW products.  Results go
+// its waves take output row tiles of 16: two accumulator sets (e and o) per unit, PW units (one, or two,
+// mm_plan) per wave, so that one matrix element loaded from L2 feeds PW products.  Results go
 // from the accumulators straight to global memory: the data is the A operand for x (lanes of a
 // result row are 16 consecutive outputs of one line) and the B operand for y (16 consecutive
 // columns), so stores are whole 128-byte segments without an LDS round trip.  Even and odd
@@ -345,7 +345,7 @@ __global__ void __launch_bounds__(1024) k_line_mm(LineArgs a0, int units)
                             if (f.ja == N - 1) va -= dl[3 * l + 2];
                             if (f.jb == N - 1) vb -= dl[3 * l + 2];
                         }
-                        // the value the transform takes in the input's precision
+                        // the line's sum, of the values that are transformed
                         if (f.ja >= 0) sum[u] += va;
                         if (f.jb >= 0) sum[u] += vb;
                     }
@@ -504,7 +504,7 @@ hipError_t launch_mm_tables(double *out, const double *oct, int N, int kind, hip
 // ---------------------------------------------------------------------------------------
 
 // The lines these kernels serve (given their matrices): those without a compiled plan, up to the
-// length where N multiply-adds per point (2 N quarter-wave) cost more than the chirp convolution.
+// length where N / 2 multiply-adds per point (N quarter-wave) cost more than the chirp convolution.
 // Measured against it on 16M points, us per transform, dense / chirp:
 //   x, folded kinds:   331: 153 / 264   509: 183 / 183   602: 280 / 293   650: 301 / 277
 //   y, folded kinds:   331: 152 / 436   602: 268 / 517   750: 260 / 440  1000: 318 / 361
